@@ -1177,7 +1177,12 @@ int stage_default_variant(const lc_batch_item* it, int count, int prec) {
     if (p > most) { most = p; big = i; }
   }
   const int form = item_form(it[big]);
-  const int v = select_variant(prec, form, it[big].op, item_box(it[big]));
+  int v = select_variant(prec, form, it[big].op, item_box(it[big]));
+  if (form == FORM_DWT || form == FORM_IDWT) {
+    std::vector<Box3> boxes;
+    for (int i = 0; i < count; ++i) boxes.push_back(item_box(it[i]));
+    v = wav_batch_variant(prec, v, boxes.data(), count);
+  }
   if (has_batch_form(form, v)) return v;
   bool fit = true;
   for (int i = 0; i < count; ++i) fit = fit && plane_fits(item_box(it[i]), prec);

@@ -1,306 +1,353 @@
-// lc_body_wavq.hpp -- device body of the plane-at-a-time 3D sym8 wavelet
-// kernel (internal).  Same arithmetic and summation order as sepw3d_body (x
-// pass, then y, then z, each over the window steps in increasing order and
-// within a step value 0 before value 1), so both give identical bits.
+// lc_body_wavq.hpp -- device body of the pair-wise 3D sym8 wavelet kernel
+// (internal).  Same arithmetic and summation order as sepw3d_body (x, then y,
+// then z; within a pass the window steps in increasing order, value 0 before
+// value 1), so both give identical bits.
 //
-// The structure is the magic-filter kernel's (lc_body_sepq.hpp), carried
-// over to the two-value steps of the wavelet: the block works one input
-// z-plane per barrier instead of one z-step (two planes) per two barriers.
+// The two values of a step lie next to each other in LDS, so that every filter
+// read takes a whole step (16 bytes in FP64) at any step offset, and a block
+// works one input z-step (two planes) per pair of barriers:
 //
-//   * x-waves filter the rows of the plane's tile (both x-bands of QX output
-//     steps per task) with 16-byte LDS reads; in LDS every row keeps its two
-//     values per step as two runs (value 0, then value 1), each 16-byte
-//     aligned, and the row stride is an odd number of 16-byte units;
-//   * the x-filtered plane is stored transposed, B[col][row] (col = output
-//     value of the x-bands, band-major), and y-waves filter one column each
-//     for one output step (both y-bands) from the previous plane's B, then
-//     push the two values into a 16-plane ring in registers;
-//   * every second plane (the last value of an input step) the y-waves emit
-//     the output step whose 8-step z window is complete: both z-bands of both
-//     y-bands, four values per lane.
+//   * the tile A[plane][row][step] holds pairs (value 0, value 1 along x);
+//     row 2 s1 + v1 is value v1 of y-step s1;
+//   * x-tasks filter QX output steps of a row (both x-bands) from QX + 7 pair
+//     reads and write them transposed into B[plane][col][s1] as the v1 half of
+//     a pair;
+//   * y-tasks (one column, one output step per lane) read 8 pairs per plane
+//     and push the y-bands into a ring of 8 z-steps in registers; the lane
+//     emits the output z-step whose window is complete (both z-bands).  With
+//     HB = 2 the two y-bands go to two lanes: half the ring per lane and half
+//     the serial work per step, for grids that leave the chip idle.
+//
+// All waves run x-tasks, then y-tasks: one tile and one x-filtered copy in
+// LDS, so that several blocks fit on a CU and fill each other's barriers.
+// Strides of A and B are odd numbers of pairs, and consecutive lanes take
+// consecutive rows (x) or columns (y): no bank conflicts.
+//
+// What bounds it (96^3 pairs and a 128-orbital batch, FP64): bytes.  Without
+// its FMAs the batch takes as long as with them (1.45 ms on fixed 16 x 16
+// tiles, HBM traffic 1.7 times the arrays); the FMAs and LDS reads alone take
+// 0.87 ms.  Hence tiles of any shape, chosen per grid (WavqShape): no lanes
+// on padding and the widest tile the block holds, since a halo read that
+// misses L2 costs as much as an input value.  The form it replaced worked a
+// plane per barrier on 8 x 8 tiles with 8-byte y reads (LDS busy 52% of its
+// cycles, a fifth of that bank conflicts): 1.65 ms for the same batch.
 //
 // ME: the epilogue reads y (F_AY).  Without (ME false) every wave issues the
-// same memory operations in every plane: the outputs are stored after the
-// x/y branch by all waves, as buffer stores that drop the x-waves' and the
-// invalid lanes' values (offset out of range) and the planes that emit
-// nothing (record count 0), so the compiler's wait counts are exact and a
-// plane waits only for the tile loads it uses.
+// same memory operations in every step, the outputs as buffer stores that drop
+// invalid lanes (offset out of range) and the steps that emit nothing (record
+// count 0), so the compiler's wait counts are exact and a step waits only for
+// the tile loads it uses.
 #pragma once
 
-#include "lc_body_sepq.hpp"
+#include <type_traits>
+
 #include "lc_body_wav.hpp"
 
 namespace lc {
 
-// the shapes this kernel takes: whole 16-byte pieces per x-task, whole waves
-// of x- and y-tasks (some shapes exist in one precision only)
-template <typename R, int TX, int TY, int QX>
-constexpr bool wavq_shape_ok() {
-  if (QX <= 0 || QX > TX || TX % QX != 0 || QX % Vec16<R>::N != 0) return false;
-  const int nr = 2 * (TY + 7), ars = 64 / igcd(64, TX / QX);
-  const int ar = (nr + ars - 1) / ars * ars;
-  return (ar * (TX / QX)) % 64 == 0 && (2 * TX * TY) % 64 == 0;
+template <typename R>
+struct Pair2;
+template <> struct Pair2<double> { using T = double2; };
+template <> struct Pair2<float> { using T = float2; };
+
+// A block's tile is tx x ty output steps, chosen per grid: any shape whose
+// y-tasks, x-tasks and tile pairs fit the block's lanes (WavqBlock::fits).
+// The strides and task maps follow from it once per block.
+struct WavqShape {
+  int tx, ty;
+  int txr;     // columns per x-band in B: whole x-tasks
+  int as, bs;  // row stride of A, column stride of B (odd numbers of pairs)
+  int nr;      // tile rows per plane
+  __host__ __device__ WavqShape(int tx_, int ty_, int qx) : tx(tx_), ty(ty_) {
+    txr = (tx + qx - 1) / qx * qx;
+    as = (txr + 7) | 1;
+    bs = (ty + 7) | 1;
+    nr = 2 * (ty + 7);
+  }
+  __host__ __device__ int pa() const { return nr * as; }          // pairs per plane of A
+  __host__ __device__ int pb() const { return 2 * txr * bs; }     // and of B
+  __host__ __device__ int pairs() const { return nr * (tx + 7); } // tile pairs per plane
+  __host__ __device__ int xtasks(int qx) const { return 2 * nr * (txr / qx); }
+};
+// A block for S output steps per plane: its lanes, the tile pairs per lane and
+// plane, the rounds of x-tasks, its LDS bytes (rs = sizeof(R)), and the tiles
+// it takes.
+struct WavqBlock {
+  int S, QX, HB;
+  constexpr int nt() const { return 2 * HB * S; }
+  constexpr int nul() const { return HB == 2 || S >= 512 ? 2 : 3; }
+  constexpr int nxl() const { return QX == 2 && HB == 1 ? 2 : 1; }
+  // four blocks of 256 lanes (FP64) or eight (FP32) fill the 160 KB of a CU
+  constexpr size_t lds(int rs) const { return (size_t)nt() * 20 * rs; }
+  bool fits(const WavqShape& g, int rs) const {
+    return g.tx * g.ty <= S && g.xtasks(QX) <= nxl() * nt() && g.pairs() <= nul() * nt() &&
+           4 * (size_t)rs * (g.pa() + g.pb()) <= lds(rs);
+  }
+};
+
+// The high-pass taps are the low-pass taps reversed with alternating signs, so
+// 16 values serve all 32 coefficients of a pass.  FP64: kept in scalar
+// registers behind an empty asm, the sign an operand modifier (32 separate
+// constants are more scalar registers than a wave has left, and spill to VGPR
+// lanes: 53 spills against none).  FP32: instruction literals (128-orbital
+// batch 0.80 ms, 0.94 with the taps in scalar registers).
+template <typename R>
+struct WavTaps {
+  R v[FLP::N];
+  __device__ __forceinline__ WavTaps() {
+#pragma unroll
+    for (int k = 0; k < FLP::N; ++k) {
+      v[k] = tap<R, FLP>(k);
+      if constexpr (sizeof(R) == 8) asm("" : "+s"(v[k]));
+    }
+  }
+  // index of the tap of this magnitude, and its sign
+  static constexpr int idx(R c) {
+    for (int k = 0; k < FLP::N; ++k)
+      if (tap<R, FLP>(k) == c || tap<R, FLP>(k) == -c) return k;
+    return -1;
+  }
+  template <class C, int CO, int CI, int S>
+  __device__ __forceinline__ R get() const {
+    constexpr R c = C::template c<R>(CO, CI, S);
+    constexpr int k = idx(c);
+    static_assert(k >= 0, "a low-pass tap up to its sign");
+    return tap<R, FLP>(k) == c ? v[k] : -v[k];
+  }
+};
+// f(integral_constant<0>) .. f(integral_constant<N - 1>)
+template <int N, class F>
+__device__ __forceinline__ void static_for(F&& f) {
+  if constexpr (N > 0) {
+    static_for<N - 1>(f);
+    f(std::integral_constant<int, N - 1>{});
+  }
 }
 
-template <typename R, class Op, int TX, int TY, int QX>
-struct WavqGeo {
-  static constexpr int W = Op::W, V = Vec16<R>::N;
-  static constexpr int TWS = TX + W - 1, TH = TY + W - 1;  // input steps per tile row / column
-  static constexpr int RX = (QX + W - 1 + V - 1) / V;       // 16-byte reads per run of an x-task
-  // one run of a row (the values c of its TWS steps), 16-byte aligned and
-  // holding every value a task's last 16-byte piece reads
-  static constexpr int TWSP = V * ((imax(TWS, TX - QX + RX * V) + V - 1) / V);
-  static constexpr int TWP = 2 * TWSP + ((2 * TWSP / V) % 2 ? 0 : V);  // odd number of 16-byte units
-  static constexpr int NR = 2 * TH;                                     // tile rows: (value, step) of y
-  static constexpr int ARS = 64 / igcd(64, TX / QX);
-  static constexpr int AR = (NR + ARS - 1) / ARS * ARS;                 // x-task rows (whole waves)
-  static constexpr int BHT = odd_ceil(AR);                              // column stride of B
-  static constexpr int NXT = AR * (TX / QX);                            // x-tasks per plane
-  static constexpr int NYT = 2 * TX * TY;                               // y-tasks per plane
-  static constexpr int NWX = NXT / 64, NWY = NYT / 64;
-  static constexpr int NT = 64 * (NWX + NWY);
-  static constexpr int NA = NR * 2 * TWS;                               // tile values per plane
-  static constexpr int NAP = (NA + NT - 1) / NT;                        // per lane
-  static constexpr size_t SA = lds_align(sizeof(R) * (AR * TWP + V));  // one half, spare slot
-  static constexpr size_t SB = lds_align(sizeof(R) * 2 * TX * BHT);
-  static constexpr size_t lds_bytes() { return 2 * (SA + SB); }
-  static_assert(W == 8, "sym8 split filters");
-  static_assert(TX % QX == 0 && QX % V == 0, "tile shape");
-  static_assert(NXT % 64 == 0 && NYT % 64 == 0 && NT <= 1024, "whole waves per pass");
-};
-// the prefetch slot of plane s is s % PD: static in the 16-plane unrolled loop
-template <int PD>
-constexpr bool wavq_pd_ok() { return PD >= 1 && (2 * 8) % PD == 0; }
+// one pair of adjacent values at byte offset `boff` (kOffNone reads zeros)
+template <typename R>
+__device__ __forceinline__ typename Pair2<R>::T plane_ld2(__amdgpu_buffer_rsrc_t rs, int boff) {
+  using T = typename Pair2<R>::T;
+  if constexpr (sizeof(R) == 8)
+    return __builtin_bit_cast(T, __builtin_amdgcn_raw_buffer_load_b128(rs, boff, 0, 0));
+  else
+    return __builtin_bit_cast(T, __builtin_amdgcn_raw_buffer_load_b64(rs, boff, 0, 0));
+}
 
-// KB > 0: the x- and y-tasks consume their LDS reads as they arrive, with a
-// scheduling fence every KB 16-byte pieces (x) or KB window steps (y), so that
-// few values are in flight: fewer VGPRs, more waves per SIMD.  The FMAs run
-// in the same order either way.
-template <typename R, class Op, int TX, int TY, int QX, int PD, bool ME = true, bool NTS = false, int KB = 0>
+template <typename R, class Op, int S, int QX, int HB, int PD, bool ME>
 __device__ __forceinline__ void wavq_body(const FusedArgs<R>& p, int bx, int by, int zc, int arr,
                                           unsigned char* lds) {
-  using G = WavqGeo<R, Op, TX, TY, QX>;
-  static_assert(wavq_pd_ok<PD>(), "prefetch depth must divide the 16-plane ring");
-  constexpr int K = WavCoef<Op>::K;
-  constexpr int W = G::W, V = G::V, NT = G::NT, TWS = G::TWS, TWSP = G::TWSP, TWP = G::TWP;
-  constexpr int TH = G::TH, AR = G::AR, BHT = G::BHT, NA = G::NA, NAP = G::NAP, RX = G::RX;
-  constexpr int NP = 2 * W;  // ring planes: the z window of one output step
-  constexpr int HA = G::SA / sizeof(R), HB = G::SB / sizeof(R);
-  constexpr int LO = Op::LO;
-  R* const A = reinterpret_cast<R*>(lds);              // [2][AR][TWP] (+ spare slot)
-  R* const B = reinterpret_cast<R*>(lds + 2 * G::SA);  // [2][2 TX][BHT]: transposed
+  using P2 = typename Pair2<R>::T;
+  using C = WavCoef<Op>;
+  constexpr WavqBlock kB{S, QX, HB};
+  constexpr int K = C::K, W = Op::W, LO = Op::LO, NT = kB.nt(), NUL = kB.nul(), NXL = kB.nxl();
+  static_assert(W == 8 && NT % (64 * HB) == 0, "sym8 split filters, whole waves per band");
+  const WavqShape g(p.tile_x, p.tile_y, QX);
+  const int PA = g.pa(), PB = g.pb(), tws = g.tx + W - 1;
+  P2* const A = reinterpret_cast<P2*>(lds);  // [2][nr][as]
+  P2* const B = A + 2 * PA;                  // [2][2 txr][bs]
 
   const int t = threadIdx.x;
   const R* __restrict__ xa = p.x + arr * p.nti;
   R* __restrict__ ya = p.y + arr * p.nto;
-  const int X0 = p.d0.olo + bx * TX, Y0 = p.d1.olo + by * TY;
+  const int X0 = p.d0.olo + bx * g.tx, Y0 = p.d1.olo + by * g.ty;
   const int zb = p.d2.olo + zc * p.zchunk;
   const int ze = min(zb + p.zchunk, p.d2.olo + p.d2.nout);
   const long rs_in = 2L * p.d0.nx, ps_in = 4L * p.d0.nx * p.d1.nx;
   const long rs_out = 2L * p.d0.ny, ps_out = 4L * p.d0.ny * p.d1.ny;
-  const int sfirst = zb + LO;              // input z-step of plane 0 (planes 2 j + c)
-  const int np = 2 * ((ze - zb) + W - 1);  // input planes of this chunk
+  const int nsteps = (ze - zb) + W - 1;  // input z-steps of this chunk
 
-  // ---- tile values of this lane: element t + j NT of every plane
-  int aoff[NAP], aslot[NAP];
+  // ---- tile pairs of this lane: pair t + j NT of a plane (the same places in
+  // both planes).  Along x the DWT finds its pair adjacent in memory, the
+  // IDWT its two values nx apart (one per band).
+  int aoff[NUL], aslot[NUL];
 #pragma unroll
-  for (int j = 0; j < NAP; ++j) {
-    const int f = t + j * NT;
-    const int rr = f / (2 * TWS), cc = f % (2 * TWS);
-    // memory order along x: the DWT interleaves the pair, the IDWT stores bands
-    const int s0 = K == KDWT ? (cc >> 1) : cc % TWS;
-    const int v0 = K == KDWT ? (cc & 1) : cc / TWS;
-    const int v1 = rr / TH, s1 = rr % TH;
+  for (int j = 0; j < NUL; ++j) {
+    const int u = t + j * NT;
+    const int rr = u / tws, s0 = u - rr * tws;
+    const int s1 = rr >> 1, v1 = rr & 1;
     const int j0 = fsrc(p.d0, X0 + LO + s0), j1 = fsrc(p.d1, Y0 + LO + s1);
-    const bool ok = f < NA && j0 >= 0 && j1 >= 0;
-    aoff[j] = plane_boff<R>(ok ? (int)(in_elem<K>(j0, v0, p.d0.nx) + rs_in * in_elem<K>(j1, v1, p.d1.nx)) : -1);
-    aslot[j] = f < NA ? rr * TWP + v0 * TWSP + s0 : AR * TWP;  // past the tile: the spare slot
+    const bool ok = rr < g.nr && j0 >= 0 && j1 >= 0;
+    aoff[j] = plane_boff<R>(ok ? (int)(in_elem<K>(j0, 0, p.d0.nx) + rs_in * in_elem<K>(j1, v1, p.d1.nx)) : -1);
+    aslot[j] = rr < g.nr ? rr * g.as + s0 : -1;
   }
-  // plane q of the chunk: value q % 2 of input z-step sfirst + q / 2
-  ZCursor zc_ld(p.d2, sfirst);
-  int ld_q = 0;
-  auto load_next = [&](R* dst) {  // the next plane in order (uniform)
-    const int s2 = ld_q < np ? zc_ld.src() : -1;
-    const int c2 = ld_q & 1;
-    const long pl = s2 >= 0 ? in_elem<K>(s2, c2, p.d2.nx) : 0;
-    const __amdgpu_buffer_rsrc_t rs = span_rsrc(xa + ps_in * pl, s2 >= 0 ? ps_in : 0);
+  const int hoff = p.d0.nx * (int)sizeof(R);  // IDWT: L to H
+  ZCursor zcur(p.d2, zb + LO);
+  P2 bufs[PD][2][NUL];
+  auto load_step = [&](P2 (&buf)[2][NUL]) {
+    const int s2 = zcur.src();
+    zcur.next();
 #pragma unroll
-    for (int j = 0; j < NAP; ++j) dst[j] = plane_ld<R>(rs, aoff[j]);
-    if (c2) zc_ld.next();
-    ++ld_q;
+    for (int c = 0; c < 2; ++c) {
+      const long pl = s2 >= 0 ? in_elem<K>(s2, c, p.d2.nx) : 0;
+      const __amdgpu_buffer_rsrc_t rs = span_rsrc(xa + ps_in * pl, s2 >= 0 ? ps_in : 0);
+#pragma unroll
+      for (int j = 0; j < NUL; ++j) {
+        if constexpr (K == KDWT) {
+          buf[c][j] = plane_ld2<R>(rs, aoff[j]);
+        } else {
+          buf[c][j].x = plane_ld<R>(rs, aoff[j]);
+          buf[c][j].y = plane_ld<R>(rs, aoff[j], hoff);
+        }
+      }
+    }
   };
 
-  const int wv = __builtin_amdgcn_readfirstlane(t >> 6), ln = t & 63;
-  const bool xwave = wv < G::NWX;
-  // x-task: row xr of column group xg; consecutive lanes take consecutive rows
-  const int xt = wv * 64 + ln;
-  const int xr = xt % AR, xg = xt / AR;
-  const int xo = xr * TWP + xg * QX;  // run 0 of the task in A (16-byte aligned)
-  const int bo = (xg * QX) * BHT + xr;
-  // y-task: output column (band c0, step i0l) and output step yi along y;
-  // consecutive lanes take consecutive output values in memory
-  const int yt = (wv - G::NWX) * 64 + ln;
-  const int yl = yt % (2 * TX), yi = yt / (2 * TX);
-  const int c0 = K == KIDWT ? (yl & 1) : yl / TX;
-  const int i0l = K == KIDWT ? (yl >> 1) : yl % TX;
-  const int ycol = c0 * TX + i0l;     // column of B
-  const int yo = ycol * BHT + yi;     // run 0 of the task in B
-  const bool out_ok = !xwave && (X0 + i0l < p.d0.olo + p.d0.nout) && (Y0 + yi < p.d1.olo + p.d1.nout);
-  const long oxy = out_elem<K>(X0 + i0l - p.d0.oy, c0, p.d0.ny) + rs_out * out_elem<K>(Y0 + yi - p.d1.oy, 0, p.d1.ny);
+  // ---- y-task: output column yl (memory order along x), output step yi and,
+  // with HB = 2, one y-band
+  constexpr int NB = 2 / HB;
+  const int band = HB == 2 ? __builtin_amdgcn_readfirstlane(t / (NT / 2)) : 0;
+  const int yt = HB == 2 ? t - band * (NT / 2) : t;
+  const bool ylane = yt < 2 * g.tx * g.ty;
+  const int yi = ylane ? yt / (2 * g.tx) : 0, yl = ylane ? yt - yi * 2 * g.tx : 0;
+  const int c0 = K == KIDWT ? (yl & 1) : (yl >= g.tx ? 1 : 0);
+  const int i0l = K == KIDWT ? (yl >> 1) : yl - c0 * g.tx;
+  const P2* const ycol = B + (K == KIDWT ? yl : c0 * g.txr + i0l) * g.bs + yi;
+  const bool out_ok = ylane && (X0 + i0l < p.d0.olo + p.d0.nout) && (Y0 + yi < p.d1.olo + p.d1.nout);
   const long oyb = rs_out * (out_elem<K>(0, 1, p.d1.ny) - out_elem<K>(0, 0, p.d1.ny));  // y-band 1 - y-band 0
+  const long oxy = out_elem<K>(X0 + i0l - p.d0.oy, c0, p.d0.ny) +
+                   rs_out * out_elem<K>(Y0 + yi - p.d1.oy, 0, p.d1.ny) + band * oyb;
   const long ozb = ps_out * (out_elem<K>(0, 1, p.d2.ny) - out_elem<K>(0, 0, p.d2.ny));  // z-band 1 - z-band 0
-  long zo = ps_out * out_elem<K>(zb - p.d2.oy, 0, p.d2.ny);
   const long zstep = ps_out * (out_elem<K>(1, 0, p.d2.ny) - out_elem<K>(0, 0, p.d2.ny));
+  long zo = ps_out * out_elem<K>(zb - p.d2.oy, 0, p.d2.ny);
 
-  R ring[2][NP];  // [y-band][plane mod 16]
+  // ---- x-tasks: consecutive lanes take consecutive rows of both planes
+  // (offsets of the row in A, of the first output value in B)
+  const P2* xsrc[NXL];
+  R* xdst[NXL];
+  bool xlane[NXL];
 #pragma unroll
-  for (int b = 0; b < 2; ++b)
-#pragma unroll
-    for (int k = 0; k < NP; ++k) ring[b][k] = R(0);
-  R buf[PD][NAP];
-#pragma unroll
-  for (int u = 0; u < PD; ++u) load_next(buf[u]);
-#pragma unroll
-  for (int j = 0; j < NAP; ++j) A[aslot[j]] = buf[0][j];
-  load_next(buf[0]);
-  __syncthreads();
+  for (int r = 0; r < NXL; ++r) {
+    const int xt = t + r * NT;
+    const int xg = xt / (2 * g.nr), row = xt - xg * 2 * g.nr, c = row >= g.nr ? 1 : 0;
+    xlane[r] = xt < g.xtasks(QX);
+    xsrc[r] = A + (xlane[r] ? row * g.as + xg * QX : 0);
+    // row 2 s1 + v1 of the plane: half v1 of pair s1
+    xdst[r] = reinterpret_cast<R*>(B + c * PB + (K == KIDWT ? 2 : 1) * xg * QX * g.bs) + (row - c * g.nr);
+  }
+  const int dq = (K == KIDWT ? 4 : 2) * g.bs;               // next step's column
+  const int d1 = (K == KIDWT ? 2 : 2 * g.txr) * g.bs;       // x-band 1 - x-band 0
 
-  const int nsteps = np + 1;
-  for (int sb = 0;; sb += NP) {
+  const WavTaps<R> taps;
+  R ring[NB][W][2];  // [y-band][z-step mod 8][plane]
 #pragma unroll
-    for (int u = 0; u < NP; ++u) {
+  for (int b = 0; b < NB; ++b)
+#pragma unroll
+    for (int k = 0; k < W; ++k) ring[b][k][0] = ring[b][k][1] = R(0);
+#pragma unroll
+  for (int k = 0; k < PD; ++k) load_step(bufs[k]);
+
+  for (int sb = 0;; sb += W) {
+#pragma unroll
+    for (int u = 0; u < W; ++u) {
       const int s = sb + u;
-      // ---- tile of plane s + 1, then the load of plane s + 1 + PD
-      {
-        R* a1 = A + ((u + 1) & 1) * HA;
-        R* bq = buf[(u + 1) % PD];
+      // ---- tile of step s, then the loads of step s + PD
+      P2 (&buf)[2][NUL] = bufs[u % PD];
 #pragma unroll
-        for (int j = 0; j < NAP; ++j) a1[aslot[j]] = bq[j];
-        load_next(bq);
-      }
-      R outv[2][2];  // ME false: [y-band][z-band] of the step this plane completes
+      for (int c = 0; c < 2; ++c)
 #pragma unroll
-      for (int b = 0; b < 2; ++b) outv[b][0] = outv[b][1] = R(0);
-      if (xwave) {
-        // ---- x-task on plane s: two runs of 16-byte reads along the row
-        const R* row = A + (u & 1) * HA + xo;
-        R* bd = B + (u & 1) * HB + bo;
-        if constexpr (KB == 0) {
-          R v[2][RX * V];
+        for (int j = 0; j < NUL; ++j)
+          if (aslot[j] >= 0) A[c * PA + aslot[j]] = buf[c][j];
+      load_step(buf);
+      __syncthreads();
 #pragma unroll
-          for (int c = 0; c < 2; ++c)
-#pragma unroll
-            for (int m = 0; m < RX; ++m) lds_read16(row + c * TWSP + m * V, &v[c][m * V]);
-#pragma unroll
-          for (int q = 0; q < QX; ++q) {
-            R o0, o1;
-            wav_step<R, Op>([&](int ss, int c) { return v[c][q + ss]; }, o0, o1);
-            bd[q * BHT] = o0;
-            bd[(TX + q) * BHT] = o1;
-          }
-        } else {
-          // piece m of both runs feeds every output whose window holds it;
-          // each accumulator still takes its terms step by step, value 0
-          // before value 1 (the order of wav_step)
-          using C = WavCoef<Op>;
+      for (int r = 0; r < NXL; ++r) {
+        if (xlane[r]) {
           R t0[QX], t1[QX];
 #pragma unroll
           for (int q = 0; q < QX; ++q) t0[q] = t1[q] = R(0);
-#pragma unroll
-          for (int m = 0; m < RX; ++m) {
-            if (m > 0 && m % KB == 0) __builtin_amdgcn_sched_barrier(0);
-            R v0[V], v1[V];
-            lds_read16(row + m * V, v0);
-            lds_read16(row + TWSP + m * V, v1);
-#pragma unroll
-            for (int e = 0; e < V; ++e) {
-              const int k = m * V + e;
-#pragma unroll
-              for (int q = 0; q < QX; ++q) {
-                const int ss = k - q;
-                if (ss >= 0 && ss < W) {
-                  t0[q] = fmar(v0[e], C::template c<R>(0, 0, ss), t0[q]);
-                  t1[q] = fmar(v0[e], C::template c<R>(1, 0, ss), t1[q]);
-                  t0[q] = fmar(v1[e], C::template c<R>(0, 1, ss), t0[q]);
-                  t1[q] = fmar(v1[e], C::template c<R>(1, 1, ss), t1[q]);
-                }
+          static_for<QX + W - 1>([&](auto kk) {
+            constexpr int k = decltype(kk)::value;
+            const P2 v = xsrc[r][k];
+            static_for<QX>([&](auto qq) {
+              constexpr int q = decltype(qq)::value, ss = k - q;
+              if constexpr (ss >= 0 && ss < W) {
+                t0[q] = fmar(v.x, taps.template get<C, 0, 0, ss>(), t0[q]);
+                t1[q] = fmar(v.x, taps.template get<C, 1, 0, ss>(), t1[q]);
+                t0[q] = fmar(v.y, taps.template get<C, 0, 1, ss>(), t0[q]);
+                t1[q] = fmar(v.y, taps.template get<C, 1, 1, ss>(), t1[q]);
               }
-            }
-          }
+            });
+          });
 #pragma unroll
           for (int q = 0; q < QX; ++q) {
-            bd[q * BHT] = t0[q];
-            bd[(TX + q) * BHT] = t1[q];
+            xdst[r][q * dq] = t0[q];
+            xdst[r][q * dq + d1] = t1[q];
           }
         }
-      } else {
-        // ---- y-task on plane s - 1: two runs along the column, into the ring
-        const R* colp = B + ((u + 1) & 1) * HB + yo;
-        R y0, y1;
-        if constexpr (KB == 0) {
-          wav_step<R, Op>([&](int ss, int c) { return colp[c * TH + ss]; }, y0, y1);
-        } else {
-          using C = WavCoef<Op>;
-          y0 = y1 = R(0);
-#pragma unroll
-          for (int ss = 0; ss < W; ++ss) {
-            if (ss > 0 && ss % KB == 0) __builtin_amdgcn_sched_barrier(0);
-            const R a = colp[ss], b = colp[TH + ss];
-            y0 = fmar(a, C::template c<R>(0, 0, ss), y0);
-            y1 = fmar(a, C::template c<R>(1, 0, ss), y1);
-            y0 = fmar(b, C::template c<R>(0, 1, ss), y0);
-            y1 = fmar(b, C::template c<R>(1, 1, ss), y1);
-          }
-        }
-        ring[0][(u + NP - 1) % NP] = y0;
-        ring[1][(u + NP - 1) % NP] = y1;
-        // ---- z: after the second value of an input step, the output step
-        // whose window (planes s - 16 .. s - 1) is complete
-        if (u % 2 == 0) {  // static after unrolling
-#pragma unroll
-          for (int b = 0; b < 2; ++b) {
-            R o0, o1;
-            wav_step<R, Op>([&](int ss, int c) { return ring[b][(u + 2 * ss + c) % NP]; }, o0, o1);
-            if (p.flags & F_A) {
-              o0 = o0 * p.a0;
-              o1 = o1 * p.a0;
-            }
-            outv[b][0] = o0;
-            outv[b][1] = o1;
-          }
-          if constexpr (ME) {
-            if (s >= NP && out_ok) {
-#pragma unroll
-              for (int b = 0; b < 2; ++b)
-#pragma unroll
-                for (int zbd = 0; zbd < 2; ++zbd) {
-                  R* yp = ya + zo + zbd * ozb + oxy + b * oyb;
-                  R v = outv[b][zbd];
-                  if (p.flags & F_AY) v = fmar(p.a_y, *yp, v);
-                  *yp = v;
-                }
-            }
-          }
-        }
-      }
-      if (u % 2 == 0) {  // static after unrolling
-        const bool em = s >= NP;  // uniform: an output step is complete
-        if constexpr (!ME) {
-          // stored by every wave; the x-waves', the invalid lanes' and (before
-          // plane 16) every value dropped
-          const __amdgpu_buffer_rsrc_t r0 = span_rsrc(ya + zo, em ? ps_out : 0);
-          const __amdgpu_buffer_rsrc_t r1 = span_rsrc(ya + zo + ozb, em ? ps_out : 0);
-#pragma unroll
-          for (int b = 0; b < 2; ++b) {
-            const int boff = out_ok ? (int)((oxy + b * oyb) * (long)sizeof(R)) : kOffNone;
-            plane_st<R, NTS>(r0, boff, outv[b][0]);
-            plane_st<R, NTS>(r1, boff, outv[b][1]);
-          }
-        }
-        zo += em ? zstep : 0;
       }
       __syncthreads();
-      if (s + 1 == nsteps) return;  // the last output step is stored
+      // ---- y-tasks on both planes, into the ring
+      auto ytask = [&](auto b0) {  // y-bands b0 .. b0 + NB - 1
+        constexpr int B0 = decltype(b0)::value;
+#pragma unroll
+        for (int c = 0; c < 2; ++c) {
+          R y[NB];
+#pragma unroll
+          for (int b = 0; b < NB; ++b) y[b] = R(0);
+          static_for<W>([&](auto sv) {
+            constexpr int ss = decltype(sv)::value;
+            const P2 v = ycol[c * PB + ss];
+            static_for<NB>([&](auto bb) {
+              constexpr int b = decltype(bb)::value;
+              y[b] = fmar(v.x, taps.template get<C, B0 + b, 0, ss>(), y[b]);
+              y[b] = fmar(v.y, taps.template get<C, B0 + b, 1, ss>(), y[b]);
+            });
+          });
+#pragma unroll
+          for (int b = 0; b < NB; ++b) ring[b][u][c] = y[b];
+        }
+      };
+      if (HB == 1 || band == 0)
+        ytask(std::integral_constant<int, 0>{});
+      else if constexpr (HB == 2)
+        ytask(std::integral_constant<int, 1>{});
+      // ---- z: the output step whose window is input steps s - 7 .. s
+      const bool em = s >= W - 1;  // uniform
+      R outv[NB][2];
+#pragma unroll
+      for (int b = 0; b < NB; ++b) {
+        R o0 = R(0), o1 = R(0);
+        static_for<W>([&](auto sv) {
+          constexpr int ss = decltype(sv)::value;
+          const R v0 = ring[b][(u + 1 + ss) % W][0], v1 = ring[b][(u + 1 + ss) % W][1];
+          o0 = fmar(v0, taps.template get<C, 0, 0, ss>(), o0);
+          o1 = fmar(v0, taps.template get<C, 1, 0, ss>(), o1);
+          o0 = fmar(v1, taps.template get<C, 0, 1, ss>(), o0);
+          o1 = fmar(v1, taps.template get<C, 1, 1, ss>(), o1);
+        });
+        if (p.flags & F_A) {
+          o0 = o0 * p.a0;
+          o1 = o1 * p.a0;
+        }
+        outv[b][0] = o0;
+        outv[b][1] = o1;
+      }
+      if constexpr (ME) {
+        if (em && out_ok) {
+#pragma unroll
+          for (int b = 0; b < NB; ++b)
+#pragma unroll
+            for (int zbd = 0; zbd < 2; ++zbd) {
+              R* yp = ya + zo + zbd * ozb + oxy + b * oyb;
+              R v = outv[b][zbd];
+              if (p.flags & F_AY) v = fmar(p.a_y, *yp, v);
+              *yp = v;
+            }
+        }
+      } else {
+        const __amdgpu_buffer_rsrc_t r0 = span_rsrc(ya + zo, em ? ps_out : 0);
+        const __amdgpu_buffer_rsrc_t r1 = span_rsrc(ya + zo + ozb, em ? ps_out : 0);
+        const int boff = out_ok ? (int)(oxy * (long)sizeof(R)) : kOffNone;
+#pragma unroll
+        for (int b = 0; b < NB; ++b) {
+          const int sb_off = (int)(b * oyb * (long)sizeof(R));
+          plane_st<R>(r0, boff, outv[b][0], sb_off);
+          plane_st<R>(r1, boff, outv[b][1], sb_off);
+        }
+      }
+      zo += em ? zstep : 0;
+      if (s + 1 == nsteps) return;
     }
   }
 }

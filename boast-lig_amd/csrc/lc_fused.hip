@@ -225,11 +225,10 @@ int select_variant(int prec, int form, int id, const Box3& b) {
   }
   v = env_variant("LIBCONV_WAV3D_VARIANT", wav_variant_count());
   if (v >= 0) return v;
-  // the plane-at-a-time kernel (its outputs go through 32-bit buffer
-  // records): FP32 on 16 x 8 steps, FP64 on 8 x 8 steps with two outputs per
-  // x-task (on 64^3 pairs 17% faster than the step-at-a-time kernel, on 96^3
-  // within 4% either way); else one z-step per slide
-  if (wav_plane_fits(b, prec) && 4L * b.ny[0] * b.ny[1] * prec <= kPlaneMax) return prec == 4 ? 7 : 16;
+  // the pair-wise kernel (its outputs go through 32-bit buffer records): the
+  // block that the model in lc_fused_wav.hip expects to be fastest on this
+  // grid; else one z-step per slide
+  if (wav_plane_fits(b, prec) && 4L * b.ny[0] * b.ny[1] * prec <= kPlaneMax) return wav_default_variant(prec, form, b);
   return 5;
 }
 

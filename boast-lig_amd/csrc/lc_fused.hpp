@@ -61,24 +61,25 @@ __device__ __forceinline__ __amdgpu_buffer_rsrc_t plane_rsrc(const R* xa, long s
   return span_rsrc(xa + (s2 >= 0 ? (long)s2 * sxy : 0), s2 >= 0 ? sxy : 0);
 }
 
-// element at byte offset `boff` of the plane; kOffNone reads zero
+// element at byte offset `boff` (+ a uniform `soff`) of the plane; kOffNone
+// reads zero
 template <typename R>
-__device__ __forceinline__ R plane_ld(__amdgpu_buffer_rsrc_t rs, int boff) {
+__device__ __forceinline__ R plane_ld(__amdgpu_buffer_rsrc_t rs, int boff, int soff = 0) {
   if constexpr (sizeof(R) == 8)
-    return __builtin_bit_cast(double, __builtin_amdgcn_raw_buffer_load_b64(rs, boff, 0, 0));
+    return __builtin_bit_cast(double, __builtin_amdgcn_raw_buffer_load_b64(rs, boff, soff, 0));
   else
-    return __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(rs, boff, 0, 0));
+    return __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(rs, boff, soff, 0));
 }
 
-// store t at byte offset `boff` of the plane (kOffNone, or a record count
+// store t at byte offset `boff` (+ a uniform `soff`) of the plane (kOffNone, or a record count
 // of 0: the store is dropped); nt: streaming (non-temporal) store
 template <typename R, bool NT = false>
-__device__ __forceinline__ void plane_st(__amdgpu_buffer_rsrc_t rs, int boff, R t) {
+__device__ __forceinline__ void plane_st(__amdgpu_buffer_rsrc_t rs, int boff, R t, int soff = 0) {
   typedef unsigned int u32x2 __attribute__((__vector_size__(2 * sizeof(unsigned int))));
   if constexpr (sizeof(R) == 8)
-    __builtin_amdgcn_raw_buffer_store_b64(__builtin_bit_cast(u32x2, t), rs, boff, 0, NT ? 2 : 0);
+    __builtin_amdgcn_raw_buffer_store_b64(__builtin_bit_cast(u32x2, t), rs, boff, soff, NT ? 2 : 0);
   else
-    __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(unsigned int, t), rs, boff, 0, NT ? 2 : 0);
+    __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(unsigned int, t), rs, boff, soff, NT ? 2 : 0);
 }
 
 template <typename R>
@@ -94,6 +95,7 @@ struct FusedArgs {
   long nti, nto;
   int narr;
   int tiles_x, tiles_y, zchunk;  // zchunk = outputs per block along z
+  int tile_x, tile_y;            // tile of a kernel that takes it at run time
   R a0, a1, a2, a_x, a_y;
   int flags;
   double* part;  // 3 sets of per-block energies (sum3d) or null

@@ -51,35 +51,37 @@ __global__ __launch_bounds__(2 * TX * TY) __attribute__((amdgpu_waves_per_eu(WPE
   sepw3d_body<R, Op, TX, TY, QX, BZ, AD>(p, tile % p.tiles_x, tile / p.tiles_x, zc, 0, lds);
 }
 
-// the plane-at-a-time form (lc_body_wavq.hpp): x-waves and y-waves, one
-// barrier per input plane
-template <typename R, class Op, int TX, int TY, int QX, int PD, int WPE, int KB>
-__global__ __launch_bounds__((WavqGeo<R, Op, TX, TY, QX>::NT)) __attribute__((amdgpu_waves_per_eu(WPE))) void wavq_fused(
-    FusedArgs<R> p) {
-  __shared__ __align__(16) unsigned char lds[WavqGeo<R, Op, TX, TY, QX>::lds_bytes()];
-  int bx, by, zc, arr;
-  block_coords(p.tiles_x, bx, by, zc, arr);
-  if (p.flags & F_AY)
-    wavq_body<R, Op, TX, TY, QX, PD, true, false, KB>(p, bx, by, zc, arr, lds);
-  else
-    wavq_body<R, Op, TX, TY, QX, PD, false, false, KB>(p, bx, by, zc, arr, lds);
-}
-
-template <typename R, class Op, int TX, int TY, int QX, int PD, int WPE, int KB>
-__global__ __launch_bounds__((WavqGeo<R, Op, TX, TY, QX>::NT)) __attribute__((amdgpu_waves_per_eu(WPE))) void wavq_batch(
-    const FusedArgs<R>* __restrict__ tab, const int* __restrict__ first, int count) {
-  const int lin = xcd_linear();
-  const int o = batch_item(first, count, lin);
-  const FusedArgs<R> p = tab[o];
-  const int local = lin - first[o];
-  const int tiles = p.tiles_x * p.tiles_y;
-  const int tile = local % tiles, zc = local / tiles;
-  __shared__ __align__(16) unsigned char lds[WavqGeo<R, Op, TX, TY, QX>::lds_bytes()];
-  if (p.flags & F_AY)
-    wavq_body<R, Op, TX, TY, QX, PD, true, false, KB>(p, tile % p.tiles_x, tile / p.tiles_x, zc, 0, lds);
-  else
-    wavq_body<R, Op, TX, TY, QX, PD, false, false, KB>(p, tile % p.tiles_x, tile / p.tiles_x, zc, 0, lds);
-}
+// the pair-wise form (lc_body_wavq.hpp): blocks for NG groups of TX x TY output
+// steps, QX outputs per x-task, PD planes of prefetch, 4 WPE waves per EU, KB + 1
+// lanes per y-task.  *_acc: with the a_y y term (ME), apart because the union
+// of both bodies spills.
+#define LC_WAVQ_ATTR                                                                         \
+  template <typename R, class Op, int NG, int TX, int TY, int QX, int PD, int WPE, int KB>   \
+  __global__ __launch_bounds__((WavqBlock{NG * TX * TY, QX, KB + 1}.nt()))                   \
+  __attribute__((amdgpu_waves_per_eu(4 * WPE)))
+#define LC_WAVQ_KERNELS(SINGLE, BATCH, ME)                                                                  \
+  LC_WAVQ_ATTR void SINGLE(FusedArgs<R> p) {                                                                \
+    constexpr WavqBlock kB{NG * TX * TY, QX, KB + 1};                                                       \
+    __shared__ __align__(16) unsigned char lds[kB.lds(sizeof(R))];                                          \
+    int bx, by, zc, arr;                                                                                    \
+    block_coords(p.tiles_x, bx, by, zc, arr);                                                               \
+    wavq_body<R, Op, kB.S, QX, kB.HB, PD / 2, ME>(p, bx, by, zc, arr, lds);                                 \
+  }                                                                                                         \
+  LC_WAVQ_ATTR void BATCH(const FusedArgs<R>* __restrict__ tab, const int* __restrict__ first, int count) { \
+    constexpr WavqBlock kB{NG * TX * TY, QX, KB + 1};                                                       \
+    const int lin = xcd_linear();                                                                           \
+    const int o = batch_item(first, count, lin);                                                            \
+    const FusedArgs<R> p = tab[o];                                                                          \
+    const int local = lin - first[o];                                                                       \
+    const int tiles = p.tiles_x * p.tiles_y;                                                                \
+    const int tile = local % tiles, zc = local / tiles;                                                     \
+    __shared__ __align__(16) unsigned char lds[kB.lds(sizeof(R))];                                          \
+    wavq_body<R, Op, kB.S, QX, kB.HB, PD / 2, ME>(p, tile % p.tiles_x, tile / p.tiles_x, zc, 0, lds);       \
+  }
+LC_WAVQ_KERNELS(wavq_fused, wavq_batch, false)
+LC_WAVQ_KERNELS(wavq_acc, wavq_batch_acc, true)
+#undef LC_WAVQ_KERNELS
+#undef LC_WAVQ_ATTR
 
 // ====================================================================== host
 // Compiled variants: tile TX x TY steps, QX outputs per x-task, BZ steps per
@@ -90,16 +92,32 @@ __global__ __launch_bounds__((WavqGeo<R, Op, TX, TY, QX>::NT)) __attribute__((am
   X(0, 16, 8, 4, 2, 2, 1, 0) X(1, 8, 8, 4, 2, 2, 1, 0) X(2, 32, 4, 4, 2, 2, 1, 0) X(3, 16, 8, 4, 1, 1, 1, 0) \
   X(4, 16, 8, 4, 1, 1, 2, 0) X(5, 16, 8, 4, 1, 1, 1, -2) X(6, 16, 8, 4, 2, 2, 1, -2)
 
-// plane-at-a-time variants: tile TX x TY steps, QX outputs per x-task, PD
-// planes of prefetch, waves per EU, z chunks as above, scheduling fence
-// interval of the filter reads (0: none)
-#define LC_WAVQ_VARIANTS(X)                                                                                  \
-  X(7, 16, 8, 4, 2, 1, -2, 0) X(8, 16, 8, 4, 2, 1, -3, 0) X(9, 32, 8, 4, 2, 1, -2, 0)                           \
-  X(10, 16, 16, 4, 2, 1, -2, 0) X(11, 16, 8, 4, 4, 1, -2, 0) X(12, 16, 8, 4, 2, 4, -2, 2)                        \
-  X(13, 16, 16, 4, 2, 4, -2, 2) X(14, 16, 8, 4, 2, 4, -2, 1) X(15, 16, 8, 4, 2, 1, -2, 2)                         \
-  X(16, 8, 8, 2, 2, 1, -2, 0) X(17, 8, 8, 2, 2, 4, -2, 1)
+// pair-wise variants: NG groups of TX x TY output steps per block (the tile is
+// any shape of up to NG TX TY steps, picked per grid by wav_pick), QX outputs
+// per x-task, PD planes of prefetch, WPE times four waves per EU (at most 128
+// VGPRs), KB = 1: two lanes per y-task
+#define LC_WAVQ_VARIANTS(X)                                                                      \
+  X(7, 1, 16, 8, 4, 2, 1, 0) X(8, 2, 16, 8, 4, 2, 1, 0) X(9, 4, 16, 8, 4, 2, 1, 0)                  \
+  X(10, 4, 8, 8, 2, 2, 1, 0) X(11, 1, 8, 8, 2, 2, 1, 1) X(12, 2, 8, 8, 2, 2, 1, 1)                   \
+  X(13, 8, 8, 8, 2, 2, 1, 0) X(14, 1, 8, 8, 2, 2, 1, 0) X(15, 1, 16, 8, 4, 2, 1, 1)                  \
+  X(16, 2, 8, 8, 2, 2, 1, 0) X(17, 1, 8, 4, 2, 2, 1, 1)
 
 int wav_variant_count() { return 18; }
+
+// entries 16 and 17 exist in FP64 only (they were shapes of FP64's 16-byte
+// pieces; tables tuned for FP32 never hold them)
+template <typename R>
+constexpr bool wavq_takes(int v) { return sizeof(R) == 8 || v < 16; }
+
+static bool wavq_block(int v, WavqBlock* b) {
+  switch (v) {
+#define X(I, NG, TX, TY, QX, PD, WPE, KB) \
+  case I: *b = WavqBlock{NG * TX * TY, QX, KB + 1}; return true;
+    LC_WAVQ_VARIANTS(X)
+#undef X
+  }
+  return false;
+}
 
 // output planes reached through 32-bit buffer records (the plane-at-a-time
 // variants store with buffer stores)
@@ -122,10 +140,10 @@ std::string wav_kernel_name(int prec, int form, int id, int v, bool batch) {
     break;
     LC_WAV_VARIANTS(X)
 #undef X
-#define X(I, TX, TY, QX, PD, WPE, ZC, KB)                                                                   \
+#define X(I, NG, TX, TY, QX, PD, WPE, KB)                                                                   \
   case I:                                                                                                   \
-    snprintf(buf, sizeof buf, "%s<%s, lc::%s, %d, %d, %d, %d, %d, %d>", batch ? "wavq_batch" : "wavq_fused", r, op, \
-             TX, TY, QX, PD, WPE, KB);                                                                      \
+    snprintf(buf, sizeof buf, "%s<%s, lc::%s, %d, %d, %d, %d, %d, %d, %d>", batch ? "wavq_batch" : "wavq_fused", r, \
+             op, NG, TX, TY, QX, PD, WPE, KB);                                                              \
     break;
     LC_WAVQ_VARIANTS(X)
 #undef X
@@ -189,19 +207,155 @@ static int wav_zchunk(long tiles, int narr, int nout) {
   return pick_zchunk(tiles, nout, std::max(narr, 1), std::max(1, Op::W / 2), num_cu());
 }
 
-template <typename R, class Op, int TX, int TY, int QX, int PD, int WPE, int ZC, int KB>
+// ---- tile and z chunk of the pair-wise kernels
+// Cycles of one block-step: the issue of its FMAs (x-tasks 32 QX, y-tasks
+// 128 / HB per wave of four cycles, over four SIMDs), its bytes at the CU's
+// share of the copy rate (9.3 bytes per cycle; rows and runs each cost most of
+// a 128-byte line more than they hold), and its serial chain (tile write, x,
+// y, z with a barrier between).  lat is a fit to blocks alone on their CU
+// (33 x 57 x 24 pairs, us per step in FP64 / FP32: QX 4 1.36 / 1.0, QX 2 1.21,
+// two lanes per y-task 1.06 / 0.73).
+struct WavCost {
+  double fma, mem, lat;
+};
+static WavCost wav_cost(const WavqBlock& k, const WavqShape& g, int rs) {
+  const double rd = 2.0 * g.nr * (2 * (g.tx + 7) * rs + 96), own = 8.0 * g.tx * g.ty * rs;
+  const double wr = 8.0 * g.ty * (g.tx * rs + 48);
+  WavCost c;
+  c.fma = 32.0 * k.QX * ((g.xtasks(k.QX) + 63) / 64) + 128.0 * ((2 * g.tx * g.ty + 63) / 64);
+  c.mem = (0.5 * (rd + own) + wr) / 9.3;  // about half of the halo reads hit L2
+  c.lat = rs == 8 ? 1900 + 3.7 * (32 * k.QX + 128 / k.HB) : 900 + 4.8 * (32 * k.QX + 128 / k.HB);
+  return c;
+}
+struct WavPick {
+  int tx = 0, ty = 0, zchunk = 0;
+  double t = 1e300;
+};
+// candidate tiles of a w0 x w1 grid: the extents split into equal parts
+template <typename F>
+static void wav_tiles(const WavqBlock& k, int w0, int w1, int rs, F&& f) {
+  for (int ny = 1, ty = 0; ny <= w1; ++ny) {
+    const int y = (w1 + ny - 1) / ny;
+    if (y == ty || y > k.S) continue;
+    ty = y;
+    for (int nx = (w0 * ty + k.S - 1) / k.S, tx = 0; nx <= w0; ++nx) {
+      const int x = (w0 + nx - 1) / nx;
+      if (x == tx) continue;
+      tx = x;
+      const WavqShape g(tx, ty, k.QX);
+      if (k.fits(g, rs)) f(g, (long)nx * ny);
+      if (tx <= 4) break;
+    }
+    if (ty <= 4) break;
+  }
+}
+// Single calls: the tile and z chunk with the least (steps) x (time per step).
+// A chunk of c output steps takes c + 7 input steps; a step takes the serial
+// chain while a CU has one block and the blocks' FMAs (at half of their issue
+// rate, measured at 96^3 and 112^3 pairs) or bytes beyond: all blocks start
+// together, so most halo reads hit L2 and the bytes count half.
+static WavPick wav_pick(const WavqBlock& k, int w0, int w1, int nz, int narr, int rs) {
+  WavPick best;
+  const long ncu = num_cu();
+  const int occ = std::max(1, 1024 / k.nt());  // blocks per CU: 128 VGPRs, four waves per SIMD
+  wav_tiles(k, w0, w1, rs, [&](const WavqShape& g, long tiles) {
+    const WavCost c = wav_cost(k, g, rs);
+    const double full = std::max((rs == 8 ? 2.1 : 1.7) * c.fma, 0.52 * c.mem);
+    auto consider = [&](long chunks) {
+      if (chunks < 1 || chunks > nz) return;
+      const int zc = (int)((nz + chunks - 1) / chunks);
+      const long blocks = tiles * narr * ((nz + zc - 1) / zc);
+      const long per = (blocks + ncu - 1) / ncu;
+      const double rounds = per <= occ ? 1.0 : (double)blocks / (ncu * occ);
+      const double t = (zc + 7) * rounds * std::max(c.lat, std::min<long>(per, occ) * full);
+      if (t < best.t) best = WavPick{g.tx, g.ty, zc, t};
+    };
+    for (int q = 1; q <= 2 * occ; ++q) consider(q * ncu / (tiles * narr));
+    consider(1);
+    consider(nz);
+  });
+  return best;
+}
+// The picks of recent shapes (the search takes some 10 us), per host thread.
+static WavPick wav_pick_cached(int v, const WavqBlock& k, int w0, int w1, int nz, int narr, int rs) {
+  struct Entry {
+    int key[6];
+    WavPick p;
+  };
+  constexpr int kEntries = 64;
+  static thread_local Entry cache[kEntries];  // zero-initialised: no variant 0 here
+  const int key[6] = {v, w0, w1, nz, narr, rs};
+  unsigned h = 0;
+  for (int q : key) h = h * 31u + (unsigned)q;
+  Entry& e = cache[h % kEntries];
+  if (!std::equal(key, key + 6, e.key)) {
+    e.p = wav_pick(k, w0, w1, nz, narr, rs);
+    std::copy(key, key + 6, e.key);
+  }
+  return e.p;
+}
+
+// The variant a call takes by default: of the block for 128 output steps and
+// the two-lane block for 64 the one the model expects to be faster.  Larger
+// blocks were not faster at any single grid tried (16^3 to 112^3 pairs); FP64
+// with two outputs per x-task is within 6% of four.
+int wav_default_variant(int prec, int form, const Box3& b) {
+  const int lo = form == FORM_IDWT ? Idwt<Sym8Rec>::LO : Dwt<Sym8Dec>::LO;
+  const FDim d0 = fdim(b.n[0], b.bc[0], b.nx[0], b.ny[0], lo, lo + 7), d1 = fdim(b.n[1], b.bc[1], b.nx[1], b.ny[1], lo, lo + 7),
+             d2 = fdim(b.n[2], b.bc[2], b.nx[2], b.ny[2], lo, lo + 7);
+  static const int f64[] = {16, 11}, f32[] = {7, 11};
+  int best = 5;
+  double t = 1e300;
+  for (int v : prec == 4 ? f32 : f64) {
+    WavqBlock k;
+    if (!wavq_block(v, &k)) continue;
+    const WavPick p = wav_pick_cached(v, k, d0.nout, d1.nout, d2.nout, 1, prec);
+    // a synthesis tile takes two loads per pair, which the block of half the
+    // tile hides better (64^3 pairs, FP64: 31.8 against 33.2 us)
+    const double pt = p.t * (form == FORM_IDWT && k.HB == 1 ? 1.06 : 1.0);
+    if (pt < t) { t = pt; best = v; }
+  }
+  return best;
+}
+
+// The variant of a batch stage whose largest item would take `single` by
+// itself: a stage that fills every CU is bound by bytes, so it takes the block
+// with the widest tiles, in FP64 512 output steps, in FP32 (more blocks per
+// CU) 256.  128 orbitals of 24..96 pairs, DWT stage: FP64 1.55 / 1.34 / 1.25
+// ms for 128 / 256 / 512 steps, FP32 0.90 / 0.78 / 0.83.
+int wav_batch_variant(int prec, int single, const Box3* b, int count) {
+  if (single < 7) return single;  // a tuned or environment choice of the step-at-a-time form
+  long steps = 0;
+  for (int i = 0; i < count; ++i) {
+    if (!wavq_fits(b[i], prec)) return single;
+    steps += (long)b[i].ny[0] * b[i].ny[1];
+  }
+  const int v = prec == 4 ? 10 : 9;
+  WavqBlock k;
+  return wavq_block(v, &k) && steps >= (long)k.S * num_cu() * std::max(1, 1024 / k.nt()) ? v : single;
+}
+
+template <int V, typename R, class Op, int NG, int TX, int TY, int QX, int PD, int WPE, int KB>
 static hipError_t launch_wavq(const Box3& b, int narr, const R* x, R* y, R a, R a_y, hipStream_t st) {
-  if constexpr (!wavq_shape_ok<R, TX, TY, QX>()) {
-    return hipErrorInvalidValue;  // a shape of the other precision
+  if constexpr (!wavq_takes<R>(V)) {
+    return hipErrorInvalidValue;
   } else {
   if (!wavq_fits(b, sizeof(R))) return hipErrorInvalidValue;
-  FusedArgs<R> p = wav_args<R, Op, TX, TY, QX, 1, 1>(b, narr, x, y, a, a_y);
-  const long tiles = (long)p.tiles_x * p.tiles_y;
-  p.zchunk = wav_zchunk<Op, ZC>(tiles, narr, p.d2.nout);
-  const int zch = (p.d2.nout + p.zchunk - 1) / p.zchunk;
   if (narr == 0) return hipSuccess;
-  dim3 grid((unsigned)tiles, (unsigned)zch, (unsigned)narr);
-  wavq_fused<R, Op, TX, TY, QX, PD, WPE, KB><<<grid, WavqGeo<R, Op, TX, TY, QX>::NT, 0, st>>>(p);
+  constexpr WavqBlock kB{NG * TX * TY, QX, KB + 1};
+  FusedArgs<R> p = wav_args<R, Op, TX, TY, QX, 1, 1>(b, narr, x, y, a, a_y);
+  const WavPick k = wav_pick_cached(V, kB, p.d0.nout, p.d1.nout, p.d2.nout, narr, sizeof(R));
+  p.tile_x = k.tx;
+  p.tile_y = k.ty;
+  p.tiles_x = (p.d0.nout + k.tx - 1) / k.tx;
+  p.tiles_y = (p.d1.nout + k.ty - 1) / k.ty;
+  p.zchunk = k.zchunk;
+  const int zch = (p.d2.nout + p.zchunk - 1) / p.zchunk;
+  dim3 grid((unsigned)(p.tiles_x * p.tiles_y), (unsigned)zch, (unsigned)narr);
+  if (p.flags & F_AY)
+    wavq_acc<R, Op, NG, TX, TY, QX, PD, WPE, KB><<<grid, kB.nt(), 0, st>>>(p);
+  else
+    wavq_fused<R, Op, NG, TX, TY, QX, PD, WPE, KB><<<grid, kB.nt(), 0, st>>>(p);
   return hipGetLastError();
   }
 }
@@ -214,8 +368,8 @@ static hipError_t sepw3d_variant(int v, const Box3& b, int narr, const R* x, R* 
   case I: return launch_sepw3d<R, Op, TX, TY, QX, BZ, AD, WPE, ZC>(b, narr, x, y, a, a_y, st);
     LC_WAV_VARIANTS(X)
 #undef X
-#define X(I, TX, TY, QX, PD, WPE, ZC, KB) \
-  case I: return launch_wavq<R, Op, TX, TY, QX, PD, WPE, ZC, KB>(b, narr, x, y, a, a_y, st);
+#define X(I, NG, TX, TY, QX, PD, WPE, KB) \
+  case I: return launch_wavq<I, R, Op, NG, TX, TY, QX, PD, WPE, KB>(b, narr, x, y, a, a_y, st);
     LC_WAVQ_VARIANTS(X)
 #undef X
   }
@@ -249,13 +403,29 @@ static hipError_t wav_stage_build(const BatchItem<R>* it, int count, BatchStage*
   std::vector<FusedArgs<R>> tab(count);
   std::vector<int> first(count + 1, 0);
   long tiles_all = 0;
+  WavqBlock k{};
+  const bool pairwise = wavq_block(s->variant, &k);
   for (int o = 0; o < count; ++o)
     if (!wav_plane_fits(it[o].b, sizeof(R))) return hipErrorInvalidValue;
   for (int o = 0; o < count; ++o) {
-    tab[o] = wav_args<R, Op, TX, TY, QX, BZ, AD>(it[o].b, 1, it[o].x, it[o].y, (R)it[o].a[0], (R)it[o].a_y);
+    FusedArgs<R>& p = tab[o];
+    p = wav_args<R, Op, TX, TY, QX, BZ, AD>(it[o].b, 1, it[o].x, it[o].y, (R)it[o].a[0], (R)it[o].a_y);
+    if (p.flags & F_AY) s->any_acc = true;
+    if (pairwise) {
+      // a full chip: the tile with the least bytes and (half hidden) FMAs
+      double best = 1e300;
+      wav_tiles(k, p.d0.nout, p.d1.nout, sizeof(R), [&](const WavqShape& g, long tiles) {
+        const WavCost c = wav_cost(k, g, sizeof(R));
+        const double t = tiles * (c.mem + 0.5 * c.fma);
+        if (t < best) { best = t; p.tile_x = g.tx; p.tile_y = g.ty; }
+      });
+      p.tiles_x = (p.d0.nout + p.tile_x - 1) / p.tile_x;
+      p.tiles_y = (p.d1.nout + p.tile_y - 1) / p.tile_y;
+    }
     tiles_all += (long)tab[o].tiles_x * tab[o].tiles_y;
   }
-  const long want = 2L * num_cu();
+  // two blocks per CU (pair-wise: what fills four waves per SIMD)
+  const long want = (pairwise ? std::max(1, 1024 / k.nt()) : 2) * (long)num_cu();
   const long chunks = std::max(1L, (want + tiles_all - 1) / std::max(1L, tiles_all));
   long total = 0;
   for (int o = 0; o < count; ++o) {
@@ -279,9 +449,9 @@ static hipError_t wav_stage_t(bool build, const BatchItem<R>* it, int count, Bat
   case I: return wav_stage_build<R, Op, TX, TY, QX, BZ, AD, WPE>(it, count, s);
       LC_WAV_VARIANTS(X)
 #undef X
-#define X(I, TX, TY, QX, PD, WPE, ZC, KB)                                  \
+#define X(I, NG, TX, TY, QX, PD, WPE, KB)                                  \
   case I:                                                                  \
-    if (!wavq_shape_ok<R, TX, TY, QX>()) return hipErrorInvalidValue;     \
+    if (!wavq_takes<R>(I)) return hipErrorInvalidValue;                    \
     for (int o = 0; o < count; ++o)                                        \
       if (!wavq_fits(it[o].b, sizeof(R))) return hipErrorInvalidValue;     \
     return wav_stage_build<R, Op, TX, TY, QX, 1, 1, WPE>(it, count, s);
@@ -299,13 +469,17 @@ static hipError_t wav_stage_t(bool build, const BatchItem<R>* it, int count, Bat
     break;
     LC_WAV_VARIANTS(X)
 #undef X
-#define X(I, TX, TY, QX, PD, WPE, ZC, KB)                                                                 \
+#define X(I, NG, TX, TY, QX, PD, WPE, KB)                                                                 \
   case I:                                                                                                 \
-    if constexpr (wavq_shape_ok<R, TX, TY, QX>())                                                          \
-      wavq_batch<R, Op, TX, TY, QX, PD, WPE, KB><<<s->blocks, WavqGeo<R, Op, TX, TY, QX>::NT, 0, st>>>(    \
-          tab, s->first, s->count);                                                                       \
-    else                                                                                                  \
+    if constexpr (wavq_takes<R>(I)) {                                                                     \
+      constexpr int nt = WavqBlock{NG * TX * TY, QX, KB + 1}.nt();                                        \
+      if (s->any_acc)                                                                                     \
+        wavq_batch_acc<R, Op, NG, TX, TY, QX, PD, WPE, KB><<<s->blocks, nt, 0, st>>>(tab, s->first, s->count); \
+      else                                                                                                \
+        wavq_batch<R, Op, NG, TX, TY, QX, PD, WPE, KB><<<s->blocks, nt, 0, st>>>(tab, s->first, s->count); \
+    } else {                                                                                              \
       return hipErrorInvalidValue;                                                                        \
+    }                                                                                                     \
     break;
     LC_WAVQ_VARIANTS(X)
 #undef X

@@ -27,7 +27,8 @@ struct SweepArgs {
   int ox, oy;     // logical index of the first stored input / output step
   int i_first;    // first output step (-up for grow, else 0)
   int nout;       // number of output steps
-  int chunk;      // outputs per lane chunk (strided kernel; set by launcher)
+  int chunk;      // outputs per block and line (set by launcher)
+  int cblocks;    // blocks over the lines / columns (set by launcher)
   R a, a_x, a_y;
   int flags;      // F_A | F_AX | F_AY | F_DOT
   double* dot_part;  // per-block FP64 partials of <x, a f(x)> (or null)
@@ -144,6 +145,7 @@ struct BatchStage {
   double* part = nullptr;    // device: BK_SUM energy partials, 3 per block
   double** dots = nullptr;   // device: BK_SUM energy destinations per item
   bool any_dot = false;
+  bool any_acc = false;      // wavelets: some item has a_y != 0
 };
 // copies the argument table and block prefix to new device buffers
 hipError_t batch_upload(const void* tab, size_t tab_bytes, const int* first, int count, BatchStage* s);
@@ -166,6 +168,8 @@ enum Form : int { FORM_SEP = 0, FORM_SUM = 1, FORM_DWT = 2, FORM_IDWT = 3 };
 int variant_count(int form);          // single-call variants
 bool has_batch_form(int form, int v);  // the variant also has a batched kernel
 int wav_variant_count();
+int wav_default_variant(int prec, int form, const Box3& b);
+int wav_batch_variant(int prec, int single, const Box3* b, int count);
 // variant a call of this shape uses: tuner table, else environment, else default
 int select_variant(int prec, int form, int id, const Box3& b);
 // tuner table lookup (lc_tune.cpp): -1 when the shape was not tuned
