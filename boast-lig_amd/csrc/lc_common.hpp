@@ -89,18 +89,16 @@ struct WSplit {
 // Common interface:
 //   LO, UP, W        step offsets of the input window, W = UP - LO + 1
 //   IN, OUT          values per input / output step
-//   compute(win, o)  win[s][c], s = 0..W-1 (step i+LO+s), c < IN
+//   step(s, w, o)    adds window step s (step i+LO+s, values w[c], c < IN) to
+//                    the OUT accumulators o; s = 0 .. W-1 in order
 //   DOT              the operator supports the dot_in / a_x terms
 template <class F>
 struct Conv {
   static constexpr int LO = F::LO, UP = F::UP, W = F::N, IN = 1, OUT = 1;
   static constexpr bool DOT = true;
   template <typename R>
-  __device__ __forceinline__ static void compute(const R (*win)[1], R* out) {
-    R t = R(0);
-#pragma unroll
-    for (int s = 0; s < W; ++s) t = fmar(win[s][0], tap<R, F>(s), t);
-    out[0] = t;
+  __device__ __forceinline__ static void step(int s, const R* w, R* o) {
+    o[0] = fmar(w[0], tap<R, F>(s), o[0]);
   }
 };
 
@@ -109,17 +107,11 @@ struct Dwt {  // input (s_2j, s_2j+1), output (L_i, H_i)
   static constexpr int LO = S::LO, UP = S::UP, W = S::W, IN = 2, OUT = 2;
   static constexpr bool DOT = false;
   template <typename R>
-  __device__ __forceinline__ static void compute(const R (*win)[2], R* out) {
-    R lt = R(0), ht = R(0);
-#pragma unroll
-    for (int s = 0; s < W; ++s) {
-      lt = fmar(win[s][0], S::template le<R>(s), lt);
-      ht = fmar(win[s][0], S::template he<R>(s), ht);
-      lt = fmar(win[s][1], S::template lo<R>(s), lt);
-      ht = fmar(win[s][1], S::template ho<R>(s), ht);
-    }
-    out[0] = lt;
-    out[1] = ht;
+  __device__ __forceinline__ static void step(int s, const R* w, R* o) {
+    o[0] = fmar(w[0], S::template le<R>(s), o[0]);
+    o[1] = fmar(w[0], S::template he<R>(s), o[1]);
+    o[0] = fmar(w[1], S::template lo<R>(s), o[0]);
+    o[1] = fmar(w[1], S::template ho<R>(s), o[1]);
   }
 };
 
@@ -128,17 +120,11 @@ struct Idwt {  // input (L_j, H_j), output (s_2i, s_2i+1)
   static constexpr int LO = S::LO, UP = S::UP, W = S::W, IN = 2, OUT = 2;
   static constexpr bool DOT = false;
   template <typename R>
-  __device__ __forceinline__ static void compute(const R (*win)[2], R* out) {
-    R et = R(0), ot = R(0);
-#pragma unroll
-    for (int s = 0; s < W; ++s) {
-      et = fmar(win[s][0], S::template lo<R>(s), et);
-      ot = fmar(win[s][0], S::template le<R>(s), ot);
-      et = fmar(win[s][1], S::template ho<R>(s), et);
-      ot = fmar(win[s][1], S::template he<R>(s), ot);
-    }
-    out[0] = et;
-    out[1] = ot;
+  __device__ __forceinline__ static void step(int s, const R* w, R* o) {
+    o[0] = fmar(w[0], S::template lo<R>(s), o[0]);
+    o[1] = fmar(w[0], S::template le<R>(s), o[1]);
+    o[0] = fmar(w[1], S::template ho<R>(s), o[0]);
+    o[1] = fmar(w[1], S::template he<R>(s), o[1]);
   }
 };
 

@@ -4,16 +4,29 @@
 // synthesis) along one dimension of an array seen as (L, line, R) with L
 // the product of the faster dims and R the product of the slower dims
 // (the libconv 1D dispatcher's ndat_left / ndat_right,
-// BigDFT/GenericConvolution2.rb:1701-1766).  Two kernels:
+// BigDFT/GenericConvolution2.rb:1701-1766).  Two kernels, one plan: a block
+// stages a tile of lines -- every line's input steps for a chunk of outputs,
+// halo included -- in LDS with all of its loads in flight at once, and every
+// lane then computes Q consecutive outputs of one line, each LDS value feeding
+// all of its outputs.
 //
-//   sweep_strided  L > 1: one lane per (l, r) column, consecutive lanes on
-//                  consecutive l so every load and store is coalesced; the
-//                  lane walks a chunk of the line with a register ring of W
-//                  input steps, so each input value is loaded once per chunk.
-//   sweep_contig   L == 1 (the processed dim is the contiguous one): a group
-//                  of lanes stages a line segment plus its filter halo in LDS
-//                  with coalesced loads, then every lane computes Q
-//                  consecutive outputs from a register window.
+//   sweep_strided  L > 1: the tile is [step][column], consecutive lanes on
+//                  consecutive columns in every phase, so loads and stores
+//                  are coalesced and the LDS is free of bank conflicts;
+//   sweep_contig   L == 1 (the processed dim is the contiguous one): the tile
+//                  is [line][step] with an odd row stride, filled along the
+//                  lines and read with consecutive lanes on consecutive lines;
+//                  the outputs go back through the LDS to be stored along the
+//                  lines.
+//
+// What bounds them: latency.  A sweep moves two values per output and the
+// arrays of one orbital are 2..130 MB, so a launch lasts a few memory round
+// trips; what counts is how many loads are in flight (here a block's whole
+// tile, 12..20 loads per lane) and that every CU has its blocks in the first
+// wave.  The form before this kept one load per lane in flight per step (a
+// register ring along the line): 27 us for a 128^3 FP64 second-derivative
+// sweep with its energy along a strided dim, 19 us along the contiguous one
+// (bank conflicts on a third of its LDS cycles).
 //
 // Epilogue per output (ConvolutionFilter#post_process_and_store_values,
 // GenericConvolution2.rb:173-203): t *= a; dot += x_i t; t += a_x x_i;
@@ -21,6 +34,9 @@
 // carries an input value (grow borders skip them).  dot is accumulated in
 // FP64 whatever the storage precision, per block, then summed in a fixed
 // order by a one-block kernel (deterministic).
+#include <type_traits>
+
+#include "lc_fused.hpp"
 #include "lc_kernels.hpp"
 
 namespace lc {
@@ -41,188 +57,246 @@ __device__ __forceinline__ double block_sum(double v, double* red) {
   return s;
 }
 
+// The input steps of a block's chunk: element offset (in line strides) of
+// component c of step j, or -1 where x is zero; steps past jmax are never used
+// and may lie outside x (shrink).  near: a periodic chunk within one wrap of
+// the line, where a compare replaces the modulo.
 template <int K, int BC, typename R>
-__device__ __forceinline__ R load_step(const R* __restrict__ xb, long L, int j, int c, int n, int nx,
-                                       int ox) {
-  if (BC == PER) {
-    return xb[in_elem<K>(pmod(j, n), c, nx) * L];
-  } else if (BC == GROW) {
-    const bool ok = (j >= 0) & (j < n);
-    const R v = xb[in_elem<K>(ok ? j : 0, c, nx) * L];
-    return ok ? v : R(0);
-  } else {
-    return xb[in_elem<K>(j - ox, c, nx) * L];
+struct SweepSrc {
+  int n, nx, ox, jmax;
+  bool near;
+  __device__ __forceinline__ SweepSrc(const SweepArgs<R>& p, int jmin, int jmax_)
+      : n(p.n), nx(p.nx), ox(p.ox), jmax(jmax_), near(jmin >= -p.n && jmax_ < 2 * p.n) {}
+  __device__ __forceinline__ long at(int j, int c) const {
+    if (j > jmax) return -1;
+    if (BC == PER) {
+      int w = j;
+      if (near) {
+        w += w < 0 ? n : 0;
+        w -= w >= n ? n : 0;
+      } else {
+        w = pmod(j, n);
+      }
+      return in_elem<K>(w, c, nx);
+    }
+    if (BC == GROW) return (j >= 0) & (j < n) ? in_elem<K>(j, c, nx) : -1;
+    return in_elem<K>(j - ox, c, nx);
   }
-}
+};
+
+// Q consecutive outputs from the LDS values v(c, s), s = 0 .. Q + W - 2 (the
+// input steps of the first output's window onwards): every accumulator takes
+// its terms in the order of Op::compute.  xc[q]: the value at the output's own
+// step (operators with the dot / a_x terms).
+template <typename R, class Op, int Q>
+struct SweepTask {
+  R o[Q][Op::OUT];
+  R xc[Q];
+  template <class V>
+  __device__ __forceinline__ void run(const V& v) {
+#pragma unroll
+    for (int q = 0; q < Q; ++q) {
+      xc[q] = R(0);
+#pragma unroll
+      for (int c = 0; c < Op::OUT; ++c) o[q][c] = R(0);
+    }
+#pragma unroll
+    for (int k = 0; k < Q + Op::W - 1; ++k) {
+      R w[Op::IN];
+#pragma unroll
+      for (int c = 0; c < Op::IN; ++c) w[c] = v(c, k);
+#pragma unroll
+      for (int q = 0; q < Q; ++q) {
+        const int s = k - q;
+        if (s >= 0 && s < Op::W) {
+          Op::step(s, w, o[q]);
+          if (Op::DOT && s == -Op::LO) xc[q] = w[0];
+        }
+      }
+    }
+  }
+  // the epilogue up to the a_y term of output step i = i0 + q
+  template <int BC>
+  __device__ __forceinline__ void finish(const SweepArgs<R>& p, int q, int i, bool want_dot, double& dot) {
+    if (p.flags & F_A) {
+#pragma unroll
+      for (int c = 0; c < Op::OUT; ++c) o[q][c] = o[q][c] * p.a;
+    }
+    if (Op::DOT) {
+      const bool has_x = BC != GROW || (i >= 0 && i < p.n);
+      if (has_x) {
+        if (want_dot) dot = fmar((double)xc[q], (double)o[q][0], dot);
+        if (p.flags & F_AX) o[q][0] = fmar(xc[q], p.a_x, o[q][0]);
+      }
+    }
+  }
+};
+
+// Tile of both kernels: 256 lanes, C columns (or lines) of 256 / C lanes that
+// take Q outputs each, so a chunk of up to CH outputs and NS input steps.
+// 32 columns: a row of the tile is 256 bytes in FP64 and a full line in FP32,
+// whose chunk would halve (and its halo reads double) with 64.
+constexpr int kSweepCols = 32;
+template <typename R, class Op, int Q>
+struct SweepGeo {
+  static constexpr int C = kSweepCols, G = 256 / C, CH = G * Q, NS = CH + Op::W - 1;
+  static constexpr int NL = (Op::IN * NS + G - 1) / G;  // strided: loads per lane
+  // contiguous: a row holds IN runs of NS steps (or OUT runs of CH outputs)
+  static constexpr int ROW = (Op::IN * NS > Op::OUT * CH ? Op::IN * NS : Op::OUT * CH) | 1;
+};
 
 // ---------------------------------------------------------------- strided
-template <typename R, class Op, int BC>
+template <typename R, class Op, int BC, int Q>
 __global__ __launch_bounds__(256) void sweep_strided(SweepArgs<R> p) {
-  constexpr int K = KindOf<Op>::v;
-  constexpr int W = Op::W, IN = Op::IN, OUT = Op::OUT, LO = Op::LO, UP = Op::UP;
+  using G = SweepGeo<R, Op, Q>;
+  constexpr int K = KindOf<Op>::v, C = G::C;
+  __shared__ R tile[Op::IN * G::NS * C];
   __shared__ double red[4];
-  const long col = (long)blockIdx.x * blockDim.x + threadIdx.x;
+  const int tc = threadIdx.x % C, tg = threadIdx.x / C;
+  // arrays of a call lie line_in * nr (line_out * nr) apart, so a line's place
+  // follows from its number in the whole call
+  const int bc = (int)(blockIdx.x % (unsigned)p.cblocks), bk = (int)(blockIdx.x / (unsigned)p.cblocks);
+  const long col = (long)bc * C + tc;
   const bool active = col < p.ncols;
+  const long line = !active ? 0 : p.ncols <= 0x7fffffffL ? (int)col / (int)p.L : col / p.L;
+  const long l = active ? col - line * p.L : 0;
+  const R* __restrict__ xb = p.x + line * p.line_in + l;
+  R* __restrict__ yb = p.y + line * p.line_out + l;
+  const int i0 = p.i_first + bk * p.chunk;
+  const int i1 = min(i0 + p.chunk, p.i_first + p.nout);
+  const SweepSrc<K, BC, R> src(p, i0 + Op::LO, i1 - 1 + Op::UP);
+  // row e of the tile: component e / NS of step i0 + LO + e % NS
+  R val[G::NL];
+#pragma unroll
+  for (int k = 0; k < G::NL; ++k) {
+    const int e = tg + k * G::G, c = e / G::NS;
+    const long at = c < Op::IN && active ? src.at(i0 + Op::LO + (e - c * G::NS), c) : -1;
+    val[k] = at >= 0 ? xb[at * p.L] : R(0);
+  }
+  // the lane's outputs, and the y values its a_y term needs
+  const int ib = i0 + tg * Q;
+  R yv[Q][Op::OUT];
+  if (p.flags & F_AY) {
+#pragma unroll
+    for (int q = 0; q < Q; ++q)
+#pragma unroll
+      for (int c = 0; c < Op::OUT; ++c)
+        yv[q][c] = active && ib + q < i1 ? yb[out_elem<K>(ib + q - p.oy, c, p.ny) * p.L] : R(0);
+  }
+#pragma unroll
+  for (int k = 0; k < G::NL; ++k) {
+    const int e = tg + k * G::G;
+    if ((k + 1) * G::G <= Op::IN * G::NS || e < Op::IN * G::NS) tile[e * C + tc] = val[k];
+  }
+  __syncthreads();
   double dot = 0.0;
-  if (active) {
-    const long l = col % p.L;
-    const long rest = col / p.L;
-    const long r = rest % p.nr;
-    const int arr = (int)(rest / p.nr);
-    const R* __restrict__ xb = p.x + arr * p.nti + r * p.line_in + l;
-    R* __restrict__ yb = p.y + arr * p.nto + r * p.line_out + l;
-    const bool want_dot = Op::DOT && (p.flags & F_DOT) && arr == p.narr - 1;
-    const int i0 = p.i_first + (int)blockIdx.y * p.chunk;
-    const int i1 = min(i0 + p.chunk, p.i_first + p.nout);
-    R win[W][IN];
-    // ring slot of step j is (j - (i0 + LO)) mod W; prefill W-1 steps
-    int jp = BC == PER ? pmod(i0 + LO, p.n) : 0;
+  if (active && ib < i1) {
+    const bool want_dot = Op::DOT && (p.flags & F_DOT) && line >= (p.narr - 1) * p.nr;
+    SweepTask<R, Op, Q> t;
+    const R* base = tile + tg * Q * C + tc;
+    t.run([&](int c, int k) { return base[(c * G::NS + k) * C]; });
 #pragma unroll
-    for (int s = 0; s < W - 1; ++s) {
-      const int j = i0 + LO + s;
+    for (int q = 0; q < Q; ++q) {
+      const int i = ib + q;
+      if (i < i1) {
+        t.template finish<BC>(p, q, i, want_dot, dot);
 #pragma unroll
-      for (int c = 0; c < IN; ++c) {
-        if (BC == PER)
-          win[s][c] = xb[in_elem<K>(jp, c, p.nx) * p.L];
-        else
-          win[s][c] = load_step<K, BC>(xb, p.L, j, c, p.n, p.nx, p.ox);
-      }
-      if (BC == PER) { ++jp; if (jp == p.n) jp = 0; }
-    }
-    for (int base = i0; base < i1; base += W) {
-#pragma unroll
-      for (int u = 0; u < W; ++u) {
-        const int i = base + u;
-        if (i < i1) {
-          const int j = i + UP;
-          const int sl = (u + W - 1) % W;
-#pragma unroll
-          for (int c = 0; c < IN; ++c) {
-            if (BC == PER)
-              win[sl][c] = xb[in_elem<K>(jp, c, p.nx) * p.L];
-            else
-              win[sl][c] = load_step<K, BC>(xb, p.L, j, c, p.n, p.nx, p.ox);
-          }
-          if (BC == PER) { ++jp; if (jp == p.n) jp = 0; }
-          R w2[W][IN];
-#pragma unroll
-          for (int s = 0; s < W; ++s)
-#pragma unroll
-            for (int c = 0; c < IN; ++c) w2[s][c] = win[(u + s) % W][c];
-          R o[OUT];
-          Op::compute(w2, o);
-          if (p.flags & F_A) {
-#pragma unroll
-            for (int c = 0; c < OUT; ++c) o[c] = o[c] * p.a;
-          }
-          if (Op::DOT) {
-            const bool has_x = BC != GROW || (i >= 0 && i < p.n);
-            if (has_x) {
-              const R xc = w2[-LO][0];
-              if (want_dot) dot = fmar((double)xc, (double)o[0], dot);
-              if (p.flags & F_AX) o[0] = fmar(xc, p.a_x, o[0]);
-            }
-          }
-#pragma unroll
-          for (int c = 0; c < OUT; ++c) {
-            R* yp = yb + out_elem<K>(i - p.oy, c, p.ny) * p.L;
-            if (p.flags & F_AY) o[c] = fmar(p.a_y, *yp, o[c]);
-            *yp = o[c];
-          }
+        for (int c = 0; c < Op::OUT; ++c) {
+          R o = t.o[q][c];
+          if (p.flags & F_AY) o = fmar(p.a_y, yv[q][c], o);
+          yb[out_elem<K>(i - p.oy, c, p.ny) * p.L] = o;
         }
       }
     }
   }
   if (p.dot_part) {
     const double s = block_sum<R>(dot, red);
-    if (threadIdx.x == 0) p.dot_part[blockIdx.y * gridDim.x + blockIdx.x] = s;
+    if (threadIdx.x == 0) p.dot_part[blockIdx.x] = s;
   }
 }
 
 // ---------------------------------------------------------------- contiguous
-// Q outputs per lane, TPL = 2^tpl_log2 lanes per line segment, 256/TPL lines
-// per block; LDS holds, per line, the NS = TPL*Q + W - 1 input steps of the
-// segment, one array per input component.
 template <typename R, class Op, int BC, int Q>
-__global__ __launch_bounds__(256) void sweep_contig(SweepArgs<R> p, int tpl_log2) {
-  constexpr int K = KindOf<Op>::v;
-  constexpr int W = Op::W, IN = Op::IN, OUT = Op::OUT, LO = Op::LO;
-  extern __shared__ __align__(16) unsigned char smem_raw[];
-  R* sm = reinterpret_cast<R*>(smem_raw);
+__global__ __launch_bounds__(256) void sweep_contig(SweepArgs<R> p) {
+  using G = SweepGeo<R, Op, Q>;
+  constexpr int K = KindOf<Op>::v, C = G::C;
+  __shared__ R tile[C * G::ROW];
   __shared__ double red[4];
-  const int TPL = 1 << tpl_log2;
-  const int LPB = 256 >> tpl_log2;
-  const int seg = TPL * Q;
-  const int NS = seg + W - 1;
-  const int tl = threadIdx.x & (TPL - 1);
-  const int lnb = threadIdx.x >> tpl_log2;
-  const long line = (long)blockIdx.x * LPB + lnb;
-  const bool active = line < p.ncols;
-  const int i0 = p.i_first + (int)blockIdx.y * seg;
-  const int iend = p.i_first + p.nout;
-  const long r = active ? line % p.nr : 0;
-  const int arr = active ? (int)(line / p.nr) : 0;
-  const R* __restrict__ xb = p.x + arr * p.nti + r * p.line_in;
-  R* __restrict__ yb = p.y + arr * p.nto + r * p.line_out;
-  if (active) {
-    // the last segment may extend past the last output: its steps beyond
-    // iend - 1 + UP are never used and may lie outside x (shrink), so they
-    // are not loaded
-    const int jmax = iend - 1 + Op::UP;
-    for (int e = tl; e < NS * IN; e += TPL) {
-      int s, c;
-      if (K == KDWT) { s = e >> 1; c = e & 1; }      // interleaved sample pairs
-      else if (K == KIDWT) { c = e / NS; s = e - c * NS; }  // L block then H block
-      else { s = e; c = 0; }
-      const int j = i0 + LO + s;
-      sm[(c * LPB + lnb) * NS + s] = j <= jmax ? load_step<K, BC>(xb, 1, j, c, p.n, p.nx, p.ox) : R(0);
+  const int bc = (int)(blockIdx.x % (unsigned)p.cblocks), bk = (int)(blockIdx.x / (unsigned)p.cblocks);
+  const int i0 = p.i_first + bk * p.chunk;
+  const int i1 = min(i0 + p.chunk, p.i_first + p.nout);
+  const SweepSrc<K, BC, R> src(p, i0 + Op::LO, i1 - 1 + Op::UP);
+  const long line0 = (long)bc * C;
+  // filled 64 lanes along a line: 4 lines per pass
+  constexpr int NX = (Op::IN * G::NS + 63) / 64, NY = C / 4;
+  const int lx = threadIdx.x & 63, ly = threadIdx.x >> 6;
+  R val[NX * NY];
+#pragma unroll
+  for (int b = 0; b < NY; ++b) {
+    const long line = line0 + ly + 4 * b;
+    const bool act = line < p.ncols;
+    const R* __restrict__ xb = p.x + (act ? line * p.line_in : 0);
+#pragma unroll
+    for (int a = 0; a < NX; ++a) {
+      const int e = lx + 64 * a;  // memory order: pairs (DWT), bands (IDWT)
+      const int c = K == KDWT ? e & 1 : e / G::NS, s = K == KDWT ? e >> 1 : e - c * G::NS;
+      const long at = act && e < Op::IN * G::NS ? src.at(i0 + Op::LO + s, c) : -1;
+      val[b * NX + a] = at >= 0 ? xb[at] : R(0);
     }
   }
+#pragma unroll
+  for (int b = 0; b < NY; ++b)
+#pragma unroll
+    for (int a = 0; a < NX; ++a) {
+      const int e = lx + 64 * a;
+      const int c = K == KDWT ? e & 1 : e / G::NS, s = K == KDWT ? e >> 1 : e - c * G::NS;
+      if (64 * (a + 1) <= Op::IN * G::NS || e < Op::IN * G::NS)
+        tile[(ly + 4 * b) * G::ROW + c * G::NS + s] = val[b * NX + a];
+    }
   __syncthreads();
+  // lane -> line tc, outputs ib .. ib + Q - 1
+  const int tc = threadIdx.x % C, tg = threadIdx.x / C;
+  const long line = line0 + tc;
+  const int ib = i0 + tg * Q;
   double dot = 0.0;
-  if (active) {
-    const bool want_dot = Op::DOT && (p.flags & F_DOT) && arr == p.narr - 1;
-    const int ib = i0 + tl * Q;
-    R win[Q + W - 1][IN];
+  SweepTask<R, Op, Q> t;
+  {
+    const R* base = tile + tc * G::ROW + tg * Q;
+    t.run([&](int c, int k) { return base[c * G::NS + k]; });
+    const bool want_dot = Op::DOT && (p.flags & F_DOT) && line < p.ncols && line >= (p.narr - 1) * p.nr;
 #pragma unroll
-    for (int s = 0; s < Q + W - 1; ++s)
+    for (int q = 0; q < Q; ++q)
+      if (ib + q < i1) t.template finish<BC>(p, q, ib + q, want_dot, dot);
+  }
+  __syncthreads();
+  // outputs back through the tile, in memory order along the line
 #pragma unroll
-      for (int c = 0; c < IN; ++c) win[s][c] = sm[(c * LPB + lnb) * NS + tl * Q + s];
+  for (int q = 0; q < Q; ++q)
 #pragma unroll
-    for (int q = 0; q < Q; ++q) {
-      const int i = ib + q;
-      if (i < iend) {
-        R w2[W][IN];
+    for (int c = 0; c < Op::OUT; ++c)
+      tile[tc * G::ROW + (K == KIDWT ? 2 * (tg * Q + q) + c : c * G::CH + tg * Q + q)] = t.o[q][c];
+  __syncthreads();
+  constexpr int OX = (Op::OUT * G::CH + 63) / 64;
 #pragma unroll
-        for (int s = 0; s < W; ++s)
+  for (int b = 0; b < NY; ++b) {
+    const long ln = line0 + ly + 4 * b;
+    if (ln >= p.ncols) break;
+    R* __restrict__ yb = p.y + ln * p.line_out;
 #pragma unroll
-          for (int c = 0; c < IN; ++c) w2[s][c] = win[q + s][c];
-        R o[OUT];
-        Op::compute(w2, o);
-        if (p.flags & F_A) {
-#pragma unroll
-          for (int c = 0; c < OUT; ++c) o[c] = o[c] * p.a;
-        }
-        if (Op::DOT) {
-          const bool has_x = BC != GROW || (i >= 0 && i < p.n);
-          if (has_x) {
-            const R xc = w2[-LO][0];
-            if (want_dot) dot = fmar((double)xc, (double)o[0], dot);
-            if (p.flags & F_AX) o[0] = fmar(xc, p.a_x, o[0]);
-          }
-        }
-#pragma unroll
-        for (int c = 0; c < OUT; ++c) {
-          R* yp = yb + out_elem<K>(i - p.oy, c, p.ny);
-          if (p.flags & F_AY) o[c] = fmar(p.a_y, *yp, o[c]);
-          *yp = o[c];
-        }
+    for (int a = 0; a < OX; ++a) {
+      const int e = lx + 64 * a;
+      const int c = K == KIDWT ? e & 1 : e / G::CH, i = i0 + (K == KIDWT ? e >> 1 : e - c * G::CH);
+      if (e < Op::OUT * G::CH && i < i1) {
+        R* yp = yb + out_elem<K>(i - p.oy, c, p.ny);
+        R o = tile[(ly + 4 * b) * G::ROW + e];
+        if (p.flags & F_AY) o = fmar(p.a_y, *yp, o);
+        *yp = o;
       }
     }
   }
   if (p.dot_part) {
     const double s = block_sum<R>(dot, red);
-    if (threadIdx.x == 0) p.dot_part[blockIdx.y * gridDim.x + blockIdx.x] = s;
+    if (threadIdx.x == 0) p.dot_part[blockIdx.x] = s;
   }
 }
 
@@ -269,43 +343,59 @@ __global__ __launch_bounds__(kPartThreads) void sum_partials(const double* __res
 }
 
 // ---------------------------------------------------------------- launcher
+// Launch shape: the largest chunk (outputs per lane Q in 2, 4, 8, 16) whose
+// blocks still number four per CU -- halo rows cost reads, few blocks leave
+// CUs idle in a launch that lasts one round of blocks -- and chunks of equal
+// length.  The wavelets' tiles are twice as deep per output step: Q up to 8
+// (sym8) and 4 (windows of 16 pairs).
+struct SweepPlan {
+  int q, chunk;
+  long cblocks, blocks;
+};
+template <typename R>
+static SweepPlan sweep_plan(const SweepArgs<R>& p, int in, int W) {
+  constexpr int C = kSweepCols, G = 256 / C;
+  SweepPlan s;
+  s.cblocks = (p.ncols + C - 1) / C;
+  s.q = in == 1 ? 16 : W > 8 ? 4 : 8;
+  while (s.q > 2 && s.cblocks * ((p.nout + G * s.q - 1) / (G * s.q)) < 4L * num_cu()) s.q /= 2;
+  const int n = (p.nout + G * s.q - 1) / (G * s.q);
+  s.chunk = (p.nout + n - 1) / n;
+  s.blocks = s.cblocks * n;
+  return s;
+}
+
 template <typename R, class Op, int BC>
 static hipError_t run_sweep(const SweepArgs<R>& a0, hipStream_t st, double* dot_out) {
   SweepArgs<R> p = a0;
-  constexpr int Q = 4;
   if (p.ncols == 0 || p.nout == 0) {
     if (dot_out) return hipMemsetAsync(dot_out, 0, sizeof(double), st);
     return hipSuccess;
   }
-  dim3 grid;
-  hipError_t e;
-  if (p.L == 1) {
-    int lg = 2;
-    while (lg < 6 && (1 << lg) * Q < p.nout) ++lg;
-    const int TPL = 1 << lg, LPB = 256 >> lg, seg = TPL * Q;
-    const int NS = seg + Op::W - 1;
-    grid = dim3((unsigned)((p.ncols + LPB - 1) / LPB), (unsigned)((p.nout + seg - 1) / seg));
-    const size_t sh = (size_t)LPB * NS * Op::IN * sizeof(R);
-    if (!p.dot_part) {
-      sweep_contig<R, Op, BC, Q><<<grid, 256, sh, st>>>(p, lg);
-    } else {
-      sweep_contig<R, Op, BC, Q><<<grid, 256, sh, st>>>(p, lg);
-    }
-  } else {
-    // chunk so that the grid holds ~8 waves per CU while chunks stay >= 2W
-    const long waves_cols = (p.ncols + 63) / 64;
-    int nchunk = (int)((8L * 256 + waves_cols - 1) / waves_cols);
-    int maxchunk = p.nout / (2 * Op::W);
-    if (nchunk > maxchunk) nchunk = maxchunk;
-    if (nchunk < 1) nchunk = 1;
-    p.chunk = (p.nout + nchunk - 1) / nchunk;
-    grid = dim3((unsigned)((p.ncols + 255) / 256), (unsigned)((p.nout + p.chunk - 1) / p.chunk));
-    sweep_strided<R, Op, BC><<<grid, 256, 0, st>>>(p);
+  const SweepPlan s = sweep_plan(p, Op::IN, Op::W);
+  if (s.blocks > 0x7fffffffL) return hipErrorInvalidValue;
+  p.chunk = s.chunk;
+  p.cblocks = (int)s.cblocks;
+  auto launch = [&](auto q) {
+    constexpr int Q = decltype(q)::value;
+    if (p.L == 1)
+      sweep_contig<R, Op, BC, Q><<<(unsigned)s.blocks, 256, 0, st>>>(p);
+    else
+      sweep_strided<R, Op, BC, Q><<<(unsigned)s.blocks, 256, 0, st>>>(p);
+  };
+  constexpr int QM = Op::IN == 1 ? 16 : Op::W > 8 ? 4 : 8;
+  if constexpr (QM >= 16) {
+    if (s.q == 16) launch(std::integral_constant<int, 16>{});
   }
-  e = hipGetLastError();
+  if constexpr (QM >= 8) {
+    if (s.q == 8) launch(std::integral_constant<int, 8>{});
+  }
+  if (s.q == 4) launch(std::integral_constant<int, 4>{});
+  if (s.q == 2) launch(std::integral_constant<int, 2>{});
+  hipError_t e = hipGetLastError();
   if (e != hipSuccess) return e;
   if (p.dot_part && dot_out) {
-    sum_partials<<<1, kPartThreads, 0, st>>>(p.dot_part, (long)grid.x * grid.y, dot_out, 1, 0);
+    sum_partials<<<1, kPartThreads, 0, st>>>(p.dot_part, s.blocks, dot_out, 1, 0);
     e = hipGetLastError();
   }
   return e;
@@ -313,13 +403,7 @@ static hipError_t run_sweep(const SweepArgs<R>& a0, hipStream_t st, double* dot_
 
 template <typename R>
 long sweep_partials_needed(const SweepArgs<R>& p, int W) {
-  if (p.L == 1) {
-    int lg = 2;
-    while (lg < 6 && (1 << lg) * 4 < p.nout) ++lg;
-    const int LPB = 256 >> lg, seg = (1 << lg) * 4;
-    return ((p.ncols + LPB - 1) / LPB) * (long)((p.nout + seg - 1) / seg);
-  }
-  return ((p.ncols + 255) / 256) * (long)p.nout;  // upper bound (chunk >= 1)
+  return sweep_plan(p, 1, W).blocks;  // only the filters form partials
 }
 
 template <typename R, class Op>
