@@ -278,14 +278,72 @@ hipError_t sep3d_fused_run(int id, const Box3& b, int narr, const R* x, R* y, R 
 }
 
 // ====================================================================== batches
-hipError_t batch_upload(const void* tab, size_t tab_bytes, const int* first, int count, BatchStage* s) {
+hipError_t batch_order(const std::vector<long>& blocks, const std::vector<long>& steps, std::vector<int>* order,
+                       std::vector<int>* first, BatchStage* s) {
+  const int count = (int)blocks.size();
+  long total = 0;
+  for (int i = 0; i < count; ++i) total += blocks[i];
+  if (total > 0x7fffffffL) return hipErrorInvalidValue;
+  order->resize(count);
+  for (int i = 0; i < count; ++i) (*order)[i] = i;
+  s->blocks = s->grid = (int)total;
+  s->by_xcd = false;
+  // items to XCDs, the most work first, to the least loaded one
+  std::vector<int> big(*order);
+  std::stable_sort(big.begin(), big.end(),
+                   [&](int a, int b) { return (double)blocks[a] * steps[a] > (double)blocks[b] * steps[b]; });
+  std::vector<int> list[8];
+  double load[8] = {};
+  long nb[8] = {};
+  for (int i : big) {
+    int x = 0;
+    for (int k = 1; k < 8; ++k)
+      if (load[k] < load[x]) x = k;
+    load[x] += (double)blocks[i] * steps[i];
+    nb[x] += blocks[i];
+    list[x].push_back(i);
+  }
+  // the other order: one contiguous run of blocks per XCD (xcd_linear)
+  double run[8] = {};
+  long at = 0;
+  for (int i = 0; i < count; ++i)
+    for (long e = at + blocks[i]; at < e;) {
+      const long per = total / 8, rem = total % 8;
+      const int x = (int)(at < rem * (per + 1) ? at / (per + 1) : rem + (at - rem * (per + 1)) / std::max(per, 1L));
+      const long end = std::min(e, (x + 1) * per + std::min<long>(x + 1, rem));
+      run[x] += (double)(end - at) * steps[i];
+      at = end;
+    }
+  // whole items per XCD unless they leave the XCDs more uneven than the runs
+  // do (few items): an XCD that ends late costs more than halo lines that miss
+  const double most = *std::max_element(load, load + 8), most_run = *std::max_element(run, run + 8);
+  const long grid = 8 * *std::max_element(nb, nb + 8);
+  int xs[9] = {};
+  if (most <= 1.06 * most_run && grid <= 0x7fffffffL) {
+    int k = 0;
+    for (int x = 0; x < 8; ++x) {
+      std::stable_sort(list[x].begin(), list[x].end(), [&](int a, int b) { return steps[a] > steps[b]; });
+      xs[x] = k;
+      for (int i : list[x]) (*order)[k++] = i;
+    }
+    xs[8] = k;
+    s->by_xcd = true;
+    s->grid = (int)grid;
+  }
+  first->assign(1, 0);
+  for (int i : *order) first->push_back(first->back() + (int)blocks[i]);
+  first->insert(first->end(), xs, xs + 9);
+  return hipSuccess;
+}
+
+hipError_t batch_upload(const void* tab, size_t tab_bytes, const std::vector<int>& first, BatchStage* s) {
   hipError_t e = hipMalloc(&s->tab, std::max<size_t>(tab_bytes, 1));
   if (e != hipSuccess) return e;
-  e = hipMalloc(reinterpret_cast<void**>(&s->first), sizeof(int) * (count + 1));
+  e = hipMalloc(reinterpret_cast<void**>(&s->first), sizeof(int) * first.size());
   if (e != hipSuccess) return e;
   e = hipMemcpy(s->tab, tab, tab_bytes, hipMemcpyHostToDevice);
   if (e != hipSuccess) return e;
-  return hipMemcpy(s->first, first, sizeof(int) * (count + 1), hipMemcpyHostToDevice);
+  return hipMemcpy(s->first, first.data(), sizeof(int) * first.size(), hipMemcpyHostToDevice);
 }
 
 void batch_stage_free(BatchStage* s) {

@@ -131,11 +131,19 @@ __device__ __forceinline__ void block_coords(int tiles_x, int& bx, int& by, int&
 }
 
 // Batched forms: one launch over the blocks of `count` independent operator
-// applications.  first[o] is the first block of application o (first[count]
-// = total); the block finds its application by binary search, then its
-// (tile, z chunk) inside it.  Applications are ordered tiles-fastest, so the
-// XCD-contiguous order of block_coords keeps each application's tiles on
-// few XCDs.
+// applications.  first[o] is the first block of application o of the table
+// (first[count] = total); the block finds its application by binary search,
+// then its (tile, z chunk) inside it, tiles fastest.
+//
+// With xs, XCD x serves the applications xs[x] .. xs[x + 1] - 1, one after the
+// other in table order: the host deals them to the XCDs by work and sorts each
+// XCD's by the length of their march (batch_order), so the blocks that run
+// together started together and stay together: neighbouring tiles read their
+// common halo lines within a few steps of each other, while those are in that
+// XCD's L2.  (One contiguous run of blocks per XCD, the order without xs, lets
+// blocks of unequal length drift apart: the wavelet stage of 128 orbitals read
+// 2.1 times its input and took 1.29 ms against 1.10 ms; sorted by total work
+// instead of march length it took 1.25 ms.)
 __device__ __forceinline__ int batch_item(const int* __restrict__ first, int count, int lin) {
   int lo = 0, hi = count - 1;
   while (lo < hi) {
@@ -150,6 +158,24 @@ __device__ __forceinline__ int xcd_linear() {
   const int xcd = lin & 7, k = lin >> 3;
   const int per = nb >> 3, rem = nb & 7;
   return xcd < rem ? xcd * (per + 1) + k : rem * (per + 1) + (xcd - rem) * per + k;
+}
+
+// the application o and the block `local` of it that this block serves; false:
+// none (the grid holds the longest XCD's blocks for every XCD)
+__device__ __forceinline__ bool batch_block(const BatchOrder& b, int& o, int& local) {
+  if (b.xs) {
+    const int x = blockIdx.x & 7, k = blockIdx.x >> 3;
+    const int i0 = b.xs[x], i1 = b.xs[x + 1];
+    const int lin = b.first[i0] + k;
+    if (i0 == i1 || lin >= b.first[i1]) return false;
+    o = i0 + batch_item(b.first + i0, i1 - i0, lin);
+    local = lin - b.first[o];
+  } else {
+    const int lin = xcd_linear();
+    o = batch_item(b.first, b.count, lin);
+    local = lin - b.first[o];
+  }
+  return true;
 }
 
 // ------------------------------------------------------------ host helpers

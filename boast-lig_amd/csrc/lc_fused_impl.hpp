@@ -47,11 +47,10 @@ __global__ __launch_bounds__(TX * TY / CPT) __attribute__((amdgpu_waves_per_eu(W
 
 template <typename R, class F, int TX, int TY, int CPT, int QX, int BZ, int HD, int WPE>
 __global__ __launch_bounds__(TX * TY / CPT) __attribute__((amdgpu_waves_per_eu(WPE))) void sum3d_batch(
-    const FusedArgs<R>* __restrict__ tab, const int* __restrict__ first, int count) {
-  const int lin = xcd_linear();
-  const int o = batch_item(first, count, lin);
+    const FusedArgs<R>* __restrict__ tab, BatchOrder ord) {
+  int o, local;
+  if (!batch_block(ord, o, local)) return;
   const FusedArgs<R> p = tab[o];
-  const int local = lin - first[o];
   const int tiles = p.tiles_x * p.tiles_y;
   const int tile = local % tiles, zc = local / tiles;
   const int bx = tile % p.tiles_x, by = tile / p.tiles_x;
@@ -61,11 +60,10 @@ __global__ __launch_bounds__(TX * TY / CPT) __attribute__((amdgpu_waves_per_eu(W
 
 template <typename R, class F, int TX, int TY, int CPT, int QX, int BZ, int AD, int WPE>
 __global__ __launch_bounds__(TX * TY / CPT) __attribute__((amdgpu_waves_per_eu(WPE))) void sep3d_batch(
-    const FusedArgs<R>* __restrict__ tab, const int* __restrict__ first, int count) {
-  const int lin = xcd_linear();
-  const int o = batch_item(first, count, lin);
+    const FusedArgs<R>* __restrict__ tab, BatchOrder ord) {
+  int o, local;
+  if (!batch_block(ord, o, local)) return;
   const FusedArgs<R> p = tab[o];
-  const int local = lin - first[o];
   const int tiles = p.tiles_x * p.tiles_y;
   const int tile = local % tiles, zc = local / tiles;
   __shared__ __align__(16) unsigned char lds[sep3d_lds_bytes<R, F, TX, TY, CPT, QX, BZ, AD>()];
@@ -147,11 +145,10 @@ __global__ __launch_bounds__(TX * TY) __attribute__((amdgpu_waves_per_eu(WPE))) 
 
 template <typename R, class F, int TX, int TY, int QX, int QY, int QZ, int WPE, int KC>
 __global__ __launch_bounds__(TX * TY) __attribute__((amdgpu_waves_per_eu(WPE))) void sum3d2_batch(
-    const FusedArgs<R>* __restrict__ tab, const int* __restrict__ first, int count) {
-  const int lin = xcd_linear();
-  const int o = batch_item(first, count, lin);
+    const FusedArgs<R>* __restrict__ tab, BatchOrder ord) {
+  int o, local;
+  if (!batch_block(ord, o, local)) return;
   const FusedArgs<R> p = tab[o];
-  const int local = lin - first[o];
   const int tiles = p.tiles_x * p.tiles_y;
   const int tile = local % tiles, zc = local / tiles;
   __shared__ __align__(16) unsigned char lds[Sum2Geo<R, F, TX, TY, QX, QY, QZ>::lds_bytes()];
@@ -178,11 +175,10 @@ __global__ __launch_bounds__(TX * TY) __attribute__((amdgpu_waves_per_eu(WPE))) 
 
 template <typename R, class F, int TX, int TY, int QX, int QY, int QZ, int WPE, int KC, int PW>
 __global__ __launch_bounds__(TX * TY) __attribute__((amdgpu_waves_per_eu(WPE))) void sum3d2w_batch(
-    const FusedArgs<R>* __restrict__ tab, const int* __restrict__ first, int count) {
-  const int lin = xcd_linear();
-  const int o = batch_item(first, count, lin);
+    const FusedArgs<R>* __restrict__ tab, BatchOrder ord) {
+  int o, local;
+  if (!batch_block(ord, o, local)) return;
   const FusedArgs<R> p = tab[o];
-  const int local = lin - first[o];
   const int tiles = p.tiles_x * p.tiles_y;
   const int tile = local % tiles, zc = local / tiles;
   __shared__ __align__(16) unsigned char lds[Sum2Geo<R, F, TX, TY, QX, QY, QZ>::lds_bytes()];
@@ -264,11 +260,10 @@ __global__ __launch_bounds__(TX * TY) __attribute__((amdgpu_waves_per_eu(WPE))) 
 
 template <typename R, class F, int TX, int TY, int QX, int QY, int QZ, int WPE, int PH>
 __global__ __launch_bounds__(TX * TY) __attribute__((amdgpu_waves_per_eu(WPE))) void sumt_batch(
-    const FusedArgs<R>* __restrict__ tab, const int* __restrict__ first, int count) {
-  const int lin = xcd_linear();
-  const int o = batch_item(first, count, lin);
+    const FusedArgs<R>* __restrict__ tab, BatchOrder ord) {
+  int o, local;
+  if (!batch_block(ord, o, local)) return;
   const FusedArgs<R> p = tab[o];
-  const int local = lin - first[o];
   const int tiles = p.tiles_x * p.tiles_y;
   const int tile = local % tiles, zc = local / tiles;
   __shared__ __align__(16) unsigned char lds[Sum2Geo<R, F, TX, TY, QX, QY, QZ>::lds_bytes()];
@@ -332,11 +327,10 @@ __global__ __launch_bounds__(TX * TY) __attribute__((amdgpu_waves_per_eu(WPE))) 
 
 template <typename R, class F, int TX, int TY, int QX, int QY, int PD, int U, int WPE>
 __global__ __launch_bounds__(TX * TY) __attribute__((amdgpu_waves_per_eu(WPE))) void sump_batch(
-    const FusedArgs<R>* __restrict__ tab, const int* __restrict__ first, int count) {
-  const int lin = xcd_linear();
-  const int o = batch_item(first, count, lin);
+    const FusedArgs<R>* __restrict__ tab, BatchOrder ord) {
+  int o, local;
+  if (!batch_block(ord, o, local)) return;
   const FusedArgs<R> p = tab[o];
-  const int local = lin - first[o];
   const int tiles = p.tiles_x * p.tiles_y;
   const int tile = local % tiles, zc = local / tiles;
   __shared__ __align__(16) unsigned char lds[SumpGeo<R, F, TX, TY, QX, QY, PD, U>::lds_bytes()];
@@ -410,11 +404,10 @@ __global__ __launch_bounds__(TX * TY) __attribute__((amdgpu_waves_per_eu(WPE))) 
 
 template <typename R, class F, int TX, int TY, int QX, int QY, int QZ, int WPE, int PD>
 __global__ __launch_bounds__(TX * TY) __attribute__((amdgpu_waves_per_eu(WPE))) void sep3d2_batch(
-    const FusedArgs<R>* __restrict__ tab, const int* __restrict__ first, int count) {
-  const int lin = xcd_linear();
-  const int o = batch_item(first, count, lin);
+    const FusedArgs<R>* __restrict__ tab, BatchOrder ord) {
+  int o, local;
+  if (!batch_block(ord, o, local)) return;
   const FusedArgs<R> p = tab[o];
-  const int local = lin - first[o];
   const int tiles = p.tiles_x * p.tiles_y;
   const int tile = local % tiles, zc = local / tiles;
   __shared__ __align__(16) unsigned char lds[Sep2Geo<R, F, TX, TY, QX, QY, QZ, PD>::lds_bytes()];
@@ -488,11 +481,10 @@ __global__ __launch_bounds__(TX * TY) __attribute__((amdgpu_waves_per_eu(WPE))) 
 
 template <typename R, class F, int TX, int TY, int QX, int QY, int PD, int WPE>
 __global__ __launch_bounds__(TX * TY) __attribute__((amdgpu_waves_per_eu(WPE))) void sepp_batch(
-    const FusedArgs<R>* __restrict__ tab, const int* __restrict__ first, int count) {
-  const int lin = xcd_linear();
-  const int o = batch_item(first, count, lin);
+    const FusedArgs<R>* __restrict__ tab, BatchOrder ord) {
+  int o, local;
+  if (!batch_block(ord, o, local)) return;
   const FusedArgs<R> p = tab[o];
-  const int local = lin - first[o];
   const int tiles = p.tiles_x * p.tiles_y;
   const int tile = local % tiles, zc = local / tiles;
   __shared__ __align__(16) unsigned char lds[SeppGeo<R, F, TX, TY, QX, QY, PD>::lds_bytes()];
@@ -525,7 +517,7 @@ hipError_t launch_sepp_batch(const FusedArgs<R>* tab, const BatchStage* s, hipSt
   if constexpr (!sepp_filter<F>()) {
     return hipErrorInvalidValue;
   } else {
-    sepp_batch<R, F, TX, TY, QX, QY, PD, WPE><<<s->blocks, TX * TY, 0, st>>>(tab, s->first, s->count);
+    sepp_batch<R, F, TX, TY, QX, QY, PD, WPE><<<s->grid, TX * TY, 0, st>>>(tab, batch_order_of(s));
     return hipSuccess;
   }
 }
@@ -542,12 +534,10 @@ __attribute__((amdgpu_waves_per_eu(WPE))) void sepr_fused(FusedArgs<R> p) {
 
 template <typename R, class F, int TX, int TY, int QX, int QY, int PD, int WPE>
 __global__ __launch_bounds__((SeprGeo<R, F, TX, TY, QX, QY, PD>::NT))
-__attribute__((amdgpu_waves_per_eu(WPE))) void sepr_batch(const FusedArgs<R>* __restrict__ tab,
-                                                           const int* __restrict__ first, int count) {
-  const int lin = xcd_linear();
-  const int o = batch_item(first, count, lin);
+__attribute__((amdgpu_waves_per_eu(WPE))) void sepr_batch(const FusedArgs<R>* __restrict__ tab, BatchOrder ord) {
+  int o, local;
+  if (!batch_block(ord, o, local)) return;
   const FusedArgs<R> p = tab[o];
-  const int local = lin - first[o];
   const int tiles = p.tiles_x * p.tiles_y;
   const int tile = local % tiles, zc = local / tiles;
   __shared__ __align__(16) unsigned char lds[SeprGeo<R, F, TX, TY, QX, QY, PD>::lds_bytes()];
@@ -577,7 +567,7 @@ hipError_t launch_sepr_batch(const FusedArgs<R>* tab, const BatchStage* s, hipSt
     return hipErrorInvalidValue;
   } else {
     sepr_batch<R, F, TX, TY, QX, QY, PD, WPE>
-        <<<s->blocks, SeprGeo<R, F, TX, TY, QX, QY, PD>::NT, 0, st>>>(tab, s->first, s->count);
+        <<<s->grid, SeprGeo<R, F, TX, TY, QX, QY, PD>::NT, 0, st>>>(tab, batch_order_of(s));
     return hipSuccess;
   }
 }
@@ -597,12 +587,10 @@ __attribute__((amdgpu_waves_per_eu(WPE))) void sepq_fused(FusedArgs<R> p) {
 
 template <typename R, class F, int TX, int TY, int QX, int QY, int PD, int WPE>
 __global__ __launch_bounds__((SepqGeo<R, F, TX, TY, QX, QY, PD>::NT))
-__attribute__((amdgpu_waves_per_eu(WPE))) void sepq_batch(const FusedArgs<R>* __restrict__ tab,
-                                                           const int* __restrict__ first, int count) {
-  const int lin = xcd_linear();
-  const int o = batch_item(first, count, lin);
+__attribute__((amdgpu_waves_per_eu(WPE))) void sepq_batch(const FusedArgs<R>* __restrict__ tab, BatchOrder ord) {
+  int o, local;
+  if (!batch_block(ord, o, local)) return;
   const FusedArgs<R> p = tab[o];
-  const int local = lin - first[o];
   const int tiles = p.tiles_x * p.tiles_y;
   const int tile = local % tiles, zc = local / tiles;
   __shared__ __align__(16) unsigned char lds[SepqGeo<R, F, TX, TY, QX, QY, PD>::lds_bytes()];
@@ -638,7 +626,7 @@ hipError_t launch_sepq_batch(const FusedArgs<R>* tab, const BatchStage* s, hipSt
     return hipErrorInvalidValue;
   } else {
     sepq_batch<R, F, TX, TY, QX, QY, PD, WPE>
-        <<<s->blocks, SepqGeo<R, F, TX, TY, QX, QY, PD>::NT, 0, st>>>(tab, s->first, s->count);
+        <<<s->grid, SepqGeo<R, F, TX, TY, QX, QY, PD>::NT, 0, st>>>(tab, batch_order_of(s));
     return hipSuccess;
   }
 }
@@ -806,8 +794,6 @@ bool items_fit(const BatchItem<R>* it, int count) {  // planes within the buffer
 template <typename R, class F, int TX, int TY>
 hipError_t fused_stage_build(int kind, const BatchItem<R>* it, int count, BatchStage* s) {
   std::vector<FusedArgs<R>> tab(count);
-  std::vector<int> first(count + 1, 0);
-  std::vector<double*> dots(count, nullptr);
   long tiles_all = 0;
   for (int o = 0; o < count; ++o) {
     const Box3& b = it[o].b;
@@ -828,36 +814,40 @@ hipError_t fused_stage_build(int kind, const BatchItem<R>* it, int count, BatchS
       p.flags = (p.a_x != R(0) ? F_AX : 0) | (p.a_y != R(0) ? F_AY : 0) | (it[o].dot ? F_DOT : 0);
     else
       p.flags = (p.a0 != R(1) ? F_A : 0) | (p.a_y != R(0) ? F_AY : 0);
-    dots[o] = it[o].dot;
     if (it[o].dot) s->any_dot = true;
     tiles_all += (long)p.tiles_x * p.tiles_y;
   }
   // the same number of z chunks for every item: enough blocks for ~2 per CU
   const long chunks = std::max(1L, (2L * num_cu() + tiles_all - 1) / std::max(1L, tiles_all));
-  long total = 0;
+  std::vector<long> blocks(count), steps(count);
   for (int o = 0; o < count; ++o) {
     FusedArgs<R>& p = tab[o];
     const long c = std::max(1L, std::min<long>(chunks, std::max(1, p.d2.nout / (4 * F::N))));
     p.zchunk = std::max(1, (int)((p.d2.nout + c - 1) / c));
-    const long nb = (long)p.tiles_x * p.tiles_y * ((p.d2.nout + p.zchunk - 1) / p.zchunk);
-    first[o] = (int)total;
-    p.nparts = nb;
-    total += nb;
+    blocks[o] = (long)p.tiles_x * p.tiles_y * ((p.d2.nout + p.zchunk - 1) / p.zchunk);
+    steps[o] = p.zchunk + F::N - 1;
+    p.nparts = blocks[o];
   }
-  first[count] = (int)total;
-  if (total > 0x7fffffffL) return hipErrorInvalidValue;
-  s->blocks = (int)total;
+  std::vector<int> order, first;
+  hipError_t e = batch_order(blocks, steps, &order, &first, s);
+  if (e != hipSuccess) return e;
+  std::vector<FusedArgs<R>> sorted;
+  std::vector<double*> dots;
+  for (int i : order) {
+    sorted.push_back(tab[i]);
+    dots.push_back(it[i].dot);
+  }
   if (kind == BK_SUM && s->any_dot) {
-    hipError_t e = hipMalloc(reinterpret_cast<void**>(&s->part), sizeof(double) * 3 * std::max(total, 1L));
+    e = hipMalloc(reinterpret_cast<void**>(&s->part), sizeof(double) * 3 * std::max(s->blocks, 1));
     if (e != hipSuccess) return e;
-    for (int o = 0; o < count; ++o)
-      if (it[o].dot) tab[o].part = s->part + 3L * first[o];
+    for (int k = 0; k < count; ++k)
+      if (dots[k]) sorted[k].part = s->part + 3L * first[k];
     e = hipMalloc(reinterpret_cast<void**>(&s->dots), sizeof(double*) * count);
     if (e != hipSuccess) return e;
     e = hipMemcpy(s->dots, dots.data(), sizeof(double*) * count, hipMemcpyHostToDevice);
     if (e != hipSuccess) return e;
   }
-  return batch_upload(tab.data(), sizeof(FusedArgs<R>) * count, first.data(), count, s);
+  return batch_upload(sorted.data(), sizeof(FusedArgs<R>) * count, first, s);
 }
 
 template <typename R, class F>
@@ -920,32 +910,32 @@ hipError_t fused_stage_t(bool build, int kind, const BatchItem<R>* it, int count
     switch (s->variant) {
 #define X(I, TX, TY, CPT, QX, BZ, HD, WPE)                                                                   \
   case I:                                                                                              \
-    sum3d_batch<R, F, TX, TY, CPT, QX, BZ, HD, WPE><<<s->blocks, TX * TY / CPT, 0, st>>>(tab, s->first, s->count); \
+    sum3d_batch<R, F, TX, TY, CPT, QX, BZ, HD, WPE><<<s->grid, TX * TY / CPT, 0, st>>>(tab, batch_order_of(s)); \
     break;
       LC_SUM_VARIANTS(X)
 #undef X
 #define X(I, TX, TY, QX, QY, QZ, WPE, KC, ZC)                                                         \
   case I:                                                                                            \
-    sum3d2_batch<R, F, TX, TY, QX, QY, QZ, WPE, KC><<<s->blocks, TX * TY, 0, st>>>(tab, s->first, s->count); \
+    sum3d2_batch<R, F, TX, TY, QX, QY, QZ, WPE, KC><<<s->grid, TX * TY, 0, st>>>(tab, batch_order_of(s)); \
     break;
       LC_SUM2_VARIANTS(X)
 #undef X
 #define X(I, TX, TY, QX, QY, PD, U, WPE, ZC)                                                         \
   case I:                                                                                            \
-    sump_batch<R, F, TX, TY, QX, QY, PD, U, WPE><<<s->blocks, TX * TY, 0, st>>>(tab, s->first, s->count); \
+    sump_batch<R, F, TX, TY, QX, QY, PD, U, WPE><<<s->grid, TX * TY, 0, st>>>(tab, batch_order_of(s)); \
     break;
       LC_SUMP_VARIANTS(X)
 #undef X
 #define X(I, TX, TY, QX, QY, QZ, WPE, KC, ZC, PW)                                                     \
   case I:                                                                                            \
-    sum3d2w_batch<R, F, TX, TY, QX, QY, QZ, WPE, KC, PW><<<s->blocks, TX * TY, 0, st>>>(tab, s->first, s->count); \
+    sum3d2w_batch<R, F, TX, TY, QX, QY, QZ, WPE, KC, PW><<<s->grid, TX * TY, 0, st>>>(tab, batch_order_of(s)); \
     break;
       LC_SUM2W_VARIANTS(X)
 #undef X
 #define X(I, TX, TY, QX, QY, QZ, WPE, ZC, PH)                                                        \
   case I:                                                                                            \
     if constexpr (sumt_filter<F>()) {                                                                \
-      sumt_batch<R, F, TX, TY, QX, QY, QZ, WPE, PH><<<s->blocks, TX * TY, 0, st>>>(tab, s->first, s->count); \
+      sumt_batch<R, F, TX, TY, QX, QY, QZ, WPE, PH><<<s->grid, TX * TY, 0, st>>>(tab, batch_order_of(s)); \
       break;                                                                                         \
     } else {                                                                                         \
       return hipErrorInvalidValue;                                                                   \
@@ -961,13 +951,13 @@ hipError_t fused_stage_t(bool build, int kind, const BatchItem<R>* it, int count
     switch (s->variant) {
 #define X(I, TX, TY, CPT, QX, BZ, AD, WPE)                                                                   \
   case I:                                                                                              \
-    sep3d_batch<R, F, TX, TY, CPT, QX, BZ, AD, WPE><<<s->blocks, TX * TY / CPT, 0, st>>>(tab, s->first, s->count); \
+    sep3d_batch<R, F, TX, TY, CPT, QX, BZ, AD, WPE><<<s->grid, TX * TY / CPT, 0, st>>>(tab, batch_order_of(s)); \
     break;
       LC_SEP_VARIANTS(X)
 #undef X
 #define X(I, TX, TY, QX, QY, QZ, WPE, ZC, PD)                                                                 \
   case I:                                                                                            \
-    sep3d2_batch<R, F, TX, TY, QX, QY, QZ, WPE, PD><<<s->blocks, TX * TY, 0, st>>>(tab, s->first, s->count); \
+    sep3d2_batch<R, F, TX, TY, QX, QY, QZ, WPE, PD><<<s->grid, TX * TY, 0, st>>>(tab, batch_order_of(s)); \
     break;
       LC_SEP2_VARIANTS(X)
 #undef X

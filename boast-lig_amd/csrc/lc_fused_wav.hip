@@ -40,11 +40,10 @@ __global__ __launch_bounds__(2 * TX * TY) __attribute__((amdgpu_waves_per_eu(WPE
 
 template <typename R, class Op, int TX, int TY, int QX, int BZ, int AD, int WPE>
 __global__ __launch_bounds__(2 * TX * TY) __attribute__((amdgpu_waves_per_eu(WPE))) void sepw3d_batch(
-    const FusedArgs<R>* __restrict__ tab, const int* __restrict__ first, int count) {
-  const int lin = xcd_linear();
-  const int o = batch_item(first, count, lin);
+    const FusedArgs<R>* __restrict__ tab, BatchOrder ord) {
+  int o, local;
+  if (!batch_block(ord, o, local)) return;
   const FusedArgs<R> p = tab[o];
-  const int local = lin - first[o];
   const int tiles = p.tiles_x * p.tiles_y;
   const int tile = local % tiles, zc = local / tiles;
   __shared__ __align__(16) unsigned char lds[sepw3d_lds_bytes<R, Op, TX, TY, QX, BZ, AD>()];
@@ -67,12 +66,11 @@ __global__ __launch_bounds__(2 * TX * TY) __attribute__((amdgpu_waves_per_eu(WPE
     block_coords(p.tiles_x, bx, by, zc, arr);                                                               \
     wavq_body<R, Op, kB.S, QX, kB.HB, PD / 2, ME>(p, bx, by, zc, arr, lds);                                 \
   }                                                                                                         \
-  LC_WAVQ_ATTR void BATCH(const FusedArgs<R>* __restrict__ tab, const int* __restrict__ first, int count) { \
+  LC_WAVQ_ATTR void BATCH(const FusedArgs<R>* __restrict__ tab, BatchOrder ord) {                           \
     constexpr WavqBlock kB{NG * TX * TY, QX, KB + 1};                                                       \
-    const int lin = xcd_linear();                                                                           \
-    const int o = batch_item(first, count, lin);                                                            \
+    int o, local;                                                                                           \
+    if (!batch_block(ord, o, local)) return;                                                                \
     const FusedArgs<R> p = tab[o];                                                                          \
-    const int local = lin - first[o];                                                                       \
     const int tiles = p.tiles_x * p.tiles_y;                                                                \
     const int tile = local % tiles, zc = local / tiles;                                                     \
     __shared__ __align__(16) unsigned char lds[kB.lds(sizeof(R))];                                          \
@@ -401,7 +399,6 @@ hipError_t sepw3d(int kind, int id, const Box3& b, int narr, const R* x, R* y, R
 template <typename R, class Op, int TX, int TY, int QX, int BZ, int AD, int WPE>
 static hipError_t wav_stage_build(const BatchItem<R>* it, int count, BatchStage* s) {
   std::vector<FusedArgs<R>> tab(count);
-  std::vector<int> first(count + 1, 0);
   long tiles_all = 0;
   WavqBlock k{};
   const bool pairwise = wavq_block(s->variant, &k);
@@ -427,18 +424,20 @@ static hipError_t wav_stage_build(const BatchItem<R>* it, int count, BatchStage*
   // two blocks per CU (pair-wise: what fills four waves per SIMD)
   const long want = (pairwise ? std::max(1, 1024 / k.nt()) : 2) * (long)num_cu();
   const long chunks = std::max(1L, (want + tiles_all - 1) / std::max(1L, tiles_all));
-  long total = 0;
+  std::vector<long> blocks(count), steps(count);
   for (int o = 0; o < count; ++o) {
     FusedArgs<R>& p = tab[o];
     const long c = std::max(1L, std::min<long>(chunks, std::max(1, p.d2.nout / (2 * Op::W))));
     p.zchunk = (int)((p.d2.nout + c - 1) / c);
-    first[o] = (int)total;
-    total += (long)p.tiles_x * p.tiles_y * ((p.d2.nout + p.zchunk - 1) / p.zchunk);
+    blocks[o] = (long)p.tiles_x * p.tiles_y * ((p.d2.nout + p.zchunk - 1) / p.zchunk);
+    steps[o] = p.zchunk + Op::W - 1;
   }
-  first[count] = (int)total;
-  if (total > 0x7fffffffL) return hipErrorInvalidValue;
-  s->blocks = (int)total;
-  return batch_upload(tab.data(), sizeof(FusedArgs<R>) * count, first.data(), count, s);
+  std::vector<int> order, first;
+  const hipError_t e = batch_order(blocks, steps, &order, &first, s);
+  if (e != hipSuccess) return e;
+  std::vector<FusedArgs<R>> sorted;
+  for (int i : order) sorted.push_back(tab[i]);
+  return batch_upload(sorted.data(), sizeof(FusedArgs<R>) * count, first, s);
 }
 
 template <typename R, class Op>
@@ -465,7 +464,7 @@ static hipError_t wav_stage_t(bool build, const BatchItem<R>* it, int count, Bat
   switch (s->variant) {
 #define X(I, TX, TY, QX, BZ, AD, WPE, ZC)                                                                     \
   case I:                                                                                           \
-    sepw3d_batch<R, Op, TX, TY, QX, BZ, AD, WPE><<<s->blocks, 2 * TX * TY, 0, st>>>(tab, s->first, s->count); \
+    sepw3d_batch<R, Op, TX, TY, QX, BZ, AD, WPE><<<s->grid, 2 * TX * TY, 0, st>>>(tab, batch_order_of(s)); \
     break;
     LC_WAV_VARIANTS(X)
 #undef X
@@ -474,9 +473,9 @@ static hipError_t wav_stage_t(bool build, const BatchItem<R>* it, int count, Bat
     if constexpr (wavq_takes<R>(I)) {                                                                     \
       constexpr int nt = WavqBlock{NG * TX * TY, QX, KB + 1}.nt();                                        \
       if (s->any_acc)                                                                                     \
-        wavq_batch_acc<R, Op, NG, TX, TY, QX, PD, WPE, KB><<<s->blocks, nt, 0, st>>>(tab, s->first, s->count); \
+        wavq_batch_acc<R, Op, NG, TX, TY, QX, PD, WPE, KB><<<s->grid, nt, 0, st>>>(tab, batch_order_of(s)); \
       else                                                                                                \
-        wavq_batch<R, Op, NG, TX, TY, QX, PD, WPE, KB><<<s->blocks, nt, 0, st>>>(tab, s->first, s->count); \
+        wavq_batch<R, Op, NG, TX, TY, QX, PD, WPE, KB><<<s->grid, nt, 0, st>>>(tab, batch_order_of(s)); \
     } else {                                                                                              \
       return hipErrorInvalidValue;                                                                        \
     }                                                                                                     \

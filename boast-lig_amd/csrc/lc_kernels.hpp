@@ -137,18 +137,35 @@ struct BatchItem {
   double a_x, a_y;
   double* dot;       // BK_SUM: device pointer to 3 energies, or null
 };
+// block -> application map of a batched launch (batch_block, lc_fused.hpp)
+struct BatchOrder {
+  const int* first;  // device: first block of every table entry (count + 1)
+  const int* xs;     // device: first table entry of every XCD (9), or null
+  int count;
+};
 struct BatchStage {
   int kind = 0, id = 0, bc = 0, count = 0, blocks = 0;
+  int grid = 0;              // blocks of the launch
+  bool by_xcd = false;       // the table is dealt to the XCDs
   int variant = 0;           // kernel variant of the stage (tuner index)
   void* tab = nullptr;       // device table of per-item kernel arguments
-  int* first = nullptr;      // device: first block of every item (count + 1)
+  int* first = nullptr;      // device: first block of every entry (count + 1), then the XCDs' entries (9)
   double* part = nullptr;    // device: BK_SUM energy partials, 3 per block
   double** dots = nullptr;   // device: BK_SUM energy destinations per item
   bool any_dot = false;
   bool any_acc = false;      // wavelets: some item has a_y != 0
 };
-// copies the argument table and block prefix to new device buffers
-hipError_t batch_upload(const void* tab, size_t tab_bytes, const int* first, int count, BatchStage* s);
+inline BatchOrder batch_order_of(const BatchStage* s) {
+  return BatchOrder{s->first, s->by_xcd ? s->first + s->count + 1 : nullptr, s->count};
+}
+// the order of a stage's table: entry k of the table is item order[k]; first
+// and the stage's blocks and grid follow.  blocks[i], steps[i]: the blocks of
+// item i and the length of their march.
+hipError_t batch_order(const std::vector<long>& blocks, const std::vector<long>& steps, std::vector<int>* order,
+                       std::vector<int>* first, BatchStage* s);
+// copies the argument table and block prefix (with the XCDs' entries) to new
+// device buffers
+hipError_t batch_upload(const void* tab, size_t tab_bytes, const std::vector<int>& first, BatchStage* s);
 void batch_stage_free(BatchStage* s);
 // build (allocating, synchronous) or launch (stream-ordered, no host work)
 template <typename R>
