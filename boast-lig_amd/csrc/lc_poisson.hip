@@ -293,28 +293,30 @@ __global__ __launch_bounds__(kPThreads) void grad_point_kernel(PGeom g, int segs
 }
 
 // ------------------------------------------------------------ z-marching form
-// div_u_i and nabla_u as one z march per TX x TY tile of output columns.  Per
-// plane z the tiles of the inputs (the tile plus an M-point halo along x, and
-// along y where a y-derivative is taken) go to LDS from registers loaded two
-// planes ahead; every lane owns one output column, takes its x- and
-// y-stencils from LDS and the z-stencil of the last input from a register
-// window of its column along z.  Each input value is read from HBM about
-// once, and the stencil reads hit LDS, not L2.
+// Every operator as one z march per tile of 32 x TY output columns.  Per plane
+// z the tiles of the inputs (the tile plus an M-point halo along x, and along y
+// where a y-derivative is taken) go to LDS from registers loaded one plane
+// ahead; every lane owns two neighbouring columns (i0, i0 + 1): their x- and
+// y-stencils read the LDS a pair at a time, their z-stencil of the last input
+// comes from a register window of both columns along z.
+//
+// What bounds it (256^3, order 16, FP64): LDS reads.  With one column per lane
+// and 8-byte reads, div_u_i with cc read 85 values per output (five stencils of
+// 17 taps) and the LDS was busy 62% of the kernel: 282 us.  A pair of columns
+// takes 9 reads of 16 bytes for both x-stencils and 17 for both y-stencils,
+// 30.5 per output, at twice the bytes per clock: 240 us.  What is left is the
+// overlap: order 16 in FP64 keeps 2 x 17 window values and asks for two waves
+// per SIMD (at four it spills: 585 us).
 //
 // Non-periodic borders: an output within M points of the border uses the
 // shifted row on inputs 0 .. 2m or n - 1 - 2m .. n - 1.  A tile holding such
 // outputs along x or y shifts its LDS window to [0, T + 2m) or
 // [n - T - 2m, n), which holds every input its outputs use, and its border
 // lanes read their row from LDS too (the rows are copied to LDS once).  On a
-// non-periodic z the 2m border planes are left to the one-point kernels, and
-// the march covers planes m .. n - m - 1.  Taps, order and operations equal
-// pderiv's, so both forms give identical bits.
+// non-periodic z the window of the column stays on planes 0 .. 2m (the last
+// 2m + 1 planes) for the border planes, which take their rows from LDS.  Taps,
+// order and operations equal pderiv's, so all forms give identical bits.
 constexpr int kZTX = 32;
-// tile rows (every mode): 16 rows read half the y-halo rows per output that
-// 8 rows do (update_rhopol at 256^3, order 16: 0.207 -> 0.184 ms; div_u_i
-// with cc 0.285 -> 0.277 ms)
-template <int MODE>
-constexpr int pz_ty() { return 16; }
 
 // MODE 0: div_u_i, 1: div_u_i with cc, 2..5: the gradient family (GE_*).
 // Derivatives taken of input k (X, Y in LDS; Z in the register window).
@@ -328,9 +330,11 @@ struct PNeed {
 template <typename R, int NORD, int TY>
 struct PzGeo {
   static constexpr int M = NORD / 2, W = NORD + 1;
-  static constexpr int NT = kZTX * TY;  // lanes: one output column each
-  static constexpr int TWP = (kZTX + 2 * M) | 1, TH = TY + 2 * M;
-  static constexpr int TSZ = TH * TWP + 1;  // one tile plus a spare slot
+  static constexpr int NT = kZTX / 2 * TY;  // lanes: two output columns each
+  // even row stride (a pair never straddles 16 bytes), with a spare column for
+  // tiles whose window starts at an odd distance from their first output
+  static constexpr int TWP = (kZTX + 2 * M + 2) & ~1, TH = TY + 2 * M;
+  static constexpr int TSZ = TH * TWP + 2;  // one tile plus a spare slot
   static constexpr int nload(bool x, bool y) { return (TY + (y ? 2 * M : 0)) * (kZTX + (x ? 2 * M : 0)); }
   static constexpr int nlane(bool x, bool y) { return (nload(x, y) + NT - 1) / NT; }
 };
@@ -345,18 +349,17 @@ __device__ __forceinline__ int pz_window(int o0, int t, int m, int n, bool per) 
   return o0 - m;
 }
 
-// the lane's entries of input k's tile: LDS slot and element offset in a plane
-template <typename R, int NORD, int MODE, int K>
-struct PzTile {
-  using G = PzGeo<R, NORD, pz_ty<MODE>()>;
-  using N = PNeed<MODE, K>;
-  static constexpr int NL = N::TILE ? G::nlane(N::X, N::Y) : 0;
-  int slot[NL > 0 ? NL : 1], boff[NL > 0 ? NL : 1];
-  R val[2][NL > 0 ? NL : 1];  // two planes in flight
-  __device__ __forceinline__ void init(const PGeom& g, int X0, int Y0, int wx0, int wy0, int t) {
+// a lane's entries of a tile that holds an x and / or a y halo: LDS slot and
+// byte offset in a plane (the inputs with the same halos share them)
+template <typename R, int NORD, int TY, bool X, bool Y>
+struct PzMap {
+  using G = PzGeo<R, NORD, TY>;
+  static constexpr int NL = G::nlane(X, Y);
+  int slot[NL], boff[NL];
+  __device__ __forceinline__ void init(const PGeom& g, int X0, int Y0, int wx0, int wy0, int sh, int t) {
     constexpr int M = G::M;
-    constexpr int NC = kZTX + (N::X ? 2 * M : 0), NLD = G::nload(N::X, N::Y);
-    const int rx0 = N::X ? wx0 : X0, ry0 = N::Y ? wy0 : Y0;  // region origin
+    constexpr int NC = kZTX + (X ? 2 * M : 0), NLD = G::nload(X, Y);
+    const int rx0 = X ? wx0 : X0, ry0 = Y ? wy0 : Y0;  // region origin
 #pragma unroll
     for (int j = 0; j < NL; ++j) {
       const int e = t + j * G::NT;
@@ -364,169 +367,357 @@ struct PzTile {
       const int sx = g.per0 ? pmod(gx, g.n0) : gx, sy = g.per1 ? pmod(gy, g.n1) : gy;
       // on a non-periodic dim only [0, n) is ever read
       const bool in = e < NLD && sx >= 0 && sx < g.n0 && sy >= 0 && sy < g.n1;
-      slot[j] = in ? (gy - wy0) * G::TWP + (gx - wx0) : G::TSZ - 1;
+      slot[j] = in ? (gy - wy0) * G::TWP + (gx - wx0) + sh : G::TSZ - 1;
       boff[j] = plane_boff<R>(in ? sx + g.n0 * sy : -1);
     }
   }
-  __device__ __forceinline__ void load(int b, const R* u, long plane, int s2) {
+};
+// input k's tile values of one plane in flight
+template <typename R, class Map>
+struct PzTile {
+  R val[Map::NL];
+  __device__ __forceinline__ void load(const Map& m, const R* u, long plane, int s2) {
     const __amdgpu_buffer_rsrc_t rs = plane_rsrc(u, plane, s2);
 #pragma unroll
-    for (int j = 0; j < NL; ++j) val[b][j] = plane_ld<R>(rs, boff[j]);
+    for (int j = 0; j < Map::NL; ++j) val[j] = plane_ld<R>(rs, m.boff[j]);
   }
-  __device__ __forceinline__ void store(int b, R* T) const {
+  __device__ __forceinline__ void store(const Map& m, R* T) const {
 #pragma unroll
-    for (int j = 0; j < NL; ++j) T[slot[j]] = val[b][j];
+    for (int j = 0; j < Map::NL; ++j) T[m.slot[j]] = val[j];
   }
 };
 
-// waves per SIMD asked of the compiler: 4 (<= 128 VGPRs; the FP64 form with
-// cc at order 16 spills three values at that budget, on its 16-row tiles)
+// two neighbouring values in LDS (aligned to the pair, where M is even), and
+// of a global array (aligned like one)
+template <typename R>
+struct Pz2;
+template <> struct Pz2<double> { using T = double2; };
+template <> struct Pz2<float> { using T = float2; };
+template <typename R>
+__device__ __forceinline__ typename Pz2<R>::T pz_ld2(__amdgpu_buffer_rsrc_t rs, int boff) {
+  using T = typename Pz2<R>::T;
+  if constexpr (sizeof(R) == 8)
+    return __builtin_bit_cast(T, __builtin_amdgcn_raw_buffer_load_b128(rs, boff, 0, 0));
+  else
+    return __builtin_bit_cast(T, __builtin_amdgcn_raw_buffer_load_b64(rs, boff, 0, 0));
+}
+template <typename R>
+struct PzMem;
+template <> struct PzMem<double> { typedef double T __attribute__((ext_vector_type(2), aligned(8))); };
+template <> struct PzMem<float> { typedef float T __attribute__((ext_vector_type(2), aligned(4))); };
+template <typename R>
+__device__ __forceinline__ void pz_put(R* base, long p, const R* v, bool both) {
+  if (both) {
+    typename PzMem<R>::T q;
+    q.x = v[0];
+    q.y = v[1];
+    *reinterpret_cast<typename PzMem<R>::T*>(base + p) = q;
+  } else {
+    base[p] = v[0];
+  }
+}
+template <typename R>
+__device__ __forceinline__ void pz_get(const R* base, long p, R* v, bool both) {
+  if (both) {
+    const typename PzMem<R>::T q = *reinterpret_cast<const typename PzMem<R>::T*>(base + p);
+    v[0] = q.x;
+    v[1] = q.y;
+  } else {
+    v[0] = base[p];
+    v[1] = R(0);
+  }
+}
+
+// grad_epilogue for the points p and (both) p + 1
 template <typename R, int MODE>
-constexpr int pz_waves() { return 4; }
+__device__ __forceinline__ double grad_epilogue2(const GradEpi<R>& e, long np, long p, bool both, R (*d)[2]) {
+  if constexpr (MODE == GE_GRAD || MODE == GE_SQUARE) {
+    R q[2];
+#pragma unroll
+    for (int k = 0; k < 2; ++k) q[k] = (d[0][k] * d[0][k] + d[1][k] * d[1][k]) + d[2][k] * d[2][k];
+    if constexpr (MODE == GE_GRAD) {
+#pragma unroll
+      for (int c = 0; c < 3; ++c) pz_put(e.du + c * np, p, d[c], both);
+      if (e.du2) pz_put(e.du2, p, q, both);  // uniform branch
+    } else {
+      pz_put(e.du2, p, q, both);
+    }
+    return 0.0;
+  } else if constexpr (MODE == GE_EPS) {
+    R ep[2];
+    pz_get(e.eps, p, ep, both);
+#pragma unroll
+    for (int c = 0; c < 3; ++c) {
+      const R o[2] = {d[c][0] * ep[0], d[c][1] * ep[1]};
+      pz_put(e.du + c * np, p, o, both);
+    }
+    return 0.0;
+  } else {
+    double s = grad_epilogue<R, MODE>(e, np, p, d[0][0], d[1][0], d[2][0]);
+    if (both) s += grad_epilogue<R, MODE>(e, np, p + 1, d[0][1], d[1][1], d[2][1]);
+    return s;
+  }
+}
 
-template <int MODE>
-constexpr int pz_nt() { return kZTX * pz_ty<MODE>(); }  // lanes of a z-march block
+// waves per SIMD asked of the compiler
+template <typename R, int NORD>
+constexpr int pz_waves() { return sizeof(R) == 8 && NORD == 16 ? 2 : 4; }
 
-template <typename R, int NORD, int MODE>
-__global__ __launch_bounds__(pz_nt<MODE>()) __attribute__((amdgpu_waves_per_eu(pz_waves<R, MODE>()))) void poisson_zm_kernel(
-    PGeom g, int tiles_x, int tiles, int zlo, int zhi, int zchunk, const R* __restrict__ u, R* __restrict__ o0,
-    R* __restrict__ o1, GradEpi<R> ep, R rh0, R rh1, R rh2) {
-  constexpr int TY = pz_ty<MODE>(), NT = pz_nt<MODE>();
+template <typename R, int NORD, int MODE, int TY>
+__global__ __launch_bounds__((PzGeo<R, NORD, TY>::NT))
+__attribute__((amdgpu_waves_per_eu(pz_waves<R, NORD>()))) void poisson_zm_kernel(
+    PGeom g, int tiles_x, int tiles, int zchunk, const R* __restrict__ u, R* __restrict__ o0, R* __restrict__ o1,
+    GradEpi<R> ep, R rh0, R rh1, R rh2) {
   using G = PzGeo<R, NORD, TY>;
-  constexpr int M = G::M, W = G::W, TWP = G::TWP, TSZ = G::TSZ;
+  constexpr int NT = G::NT, M = G::M, W = G::W, TWP = G::TWP, TSZ = G::TSZ;
   constexpr int NI = MODE >= GE_GRAD ? 1 : 3;
+  using T2 = typename Pz2<R>::T;
   __shared__ __align__(16) R lds[NI * TSZ];
   __shared__ R rows[W * W];  // every coefficient row (border lanes index it)
   for (int k = threadIdx.x; k < W * W; k += NT) rows[k] = prow<R, NORD>(k);
   const int lin = xcd_linear();
   const int tile = lin % tiles, zc = lin / tiles;
   const int X0 = (tile % tiles_x) * kZTX, Y0 = (tile / tiles_x) * TY;
-  const int zb = zlo + zc * zchunk, ze = min(zb + zchunk, zhi);
-  const int t = threadIdx.x, tx = t % kZTX, ty = t / kZTX;
+  const int zb = zc * zchunk, ze = min(zb + zchunk, g.n2);
+  const int t = threadIdx.x, tx = 2 * (t % (kZTX / 2)), ty = t / (kZTX / 2);
   const int i0 = X0 + tx, i1 = Y0 + ty;
-  const bool out_ok = i0 < g.n0 && i1 < g.n1;
+  const bool out_ok = i0 < g.n0 && i1 < g.n1, both = i0 + 1 < g.n0;
   const long plane = (long)g.n0 * g.n1;
   const R* uz = u + (NI - 1) * g.np;  // the input taken along z
   const int wx0 = pz_window(X0, kZTX, M, g.n0, g.per0), wy0 = pz_window(Y0, TY, M, g.n1, g.per1);
+  const int sh = (X0 - M - wx0) & 1;  // the centred stencils of a pair start on an even LDS column
 
-  // the lane's stencils in the LDS window: first tap (row / column) and
-  // coefficient row; border lanes of non-periodic dims take the shifted rows
-  const int lr = i1 - wy0, lc = i0 - wx0;
-  const bool bxl = !g.per0 && i0 < M, bxh = !g.per0 && i0 >= g.n0 - M;
-  const bool byl = !g.per1 && i1 < M, byh = !g.per1 && i1 >= g.n1 - M;
-  const int xs = (bxl ? 0 : bxh ? g.n0 - 1 - 2 * M : i0 - M) - wx0;
+  // the lane's stencils in the LDS window: row of its y, centred first columns;
+  // border lanes of non-periodic dims take the shifted rows
+  const int lr = i1 - wy0, lc = i0 - wx0 + sh;
+  const bool byl = !g.per1 && i1 < M, byh = !g.per1 && i1 >= g.n1 - M, by = byl || byh;
   const int ys = (byl ? 0 : byh ? g.n1 - 1 - 2 * M : i1 - M) - wy0;
-  const int xrow = (bxl ? i0 : bxh ? i0 - g.n0 + 2 * M + 1 : M) * W;  // first tap of the row
-  const int yrow = (byl ? i1 : byh ? i1 - g.n1 + 2 * M + 1 : M) * W;
-  const bool bx = bxl || bxh, by = byl || byh;
-
-  PzTile<R, NORD, MODE, 0> t0;
-  PzTile<R, NORD, MODE, 1> t1;
-  PzTile<R, NORD, MODE, 2> t2;
-  t0.init(g, X0, Y0, wx0, wy0, t);
-  if constexpr (NI == 3) {
-    t1.init(g, X0, Y0, wx0, wy0, t);
-    t2.init(g, X0, Y0, wx0, wy0, t);
+  const int yrow = (byl ? i1 : byh ? i1 - g.n1 + 2 * M + 1 : M) * W;  // first tap of the row
+  const bool bx = !g.per0 && (i0 < M || i0 + 1 >= g.n0 - M);
+  int xs[2], xrow[2];
+#pragma unroll
+  for (int e = 0; e < 2; ++e) {
+    const int i = i0 + e;
+    const bool l = !g.per0 && i < M, h = !g.per0 && i >= g.n0 - M;
+    // (the second column of a pair may lie past the grid: any row in the tile)
+    xs[e] = (l ? 0 : h ? g.n0 - 1 - 2 * M : i - M) - wx0 + sh;
+    xrow[e] = (l ? i : h ? min(i - g.n0 + 2 * M + 1, 2 * M) : M) * W;
   }
+
+  PzMap<R, NORD, TY, PNeed<MODE, 0>::X, PNeed<MODE, 0>::Y> m0;
+  PzMap<R, NORD, TY, PNeed<MODE, 1>::X, PNeed<MODE, 1>::Y> m1;  // inputs 1 and 2 (with cc the same halos)
+  m0.init(g, X0, Y0, wx0, wy0, sh, t);
+  if constexpr (NI == 3) m1.init(g, X0, Y0, wx0, wy0, sh, t);
+  PzTile<R, decltype(m0)> t0;
+  PzTile<R, decltype(m1)> t1, t2;
   FDim dz{};
   dz.n = g.n2; dz.nx = g.n2; dz.bc = g.per2 ? PER : FREE;
-  ZCursor zc_tile(dz, zb), zc_col(dz, zb - M);
-  auto load_tiles = [&](int b) {  // b static after unrolling
+  ZCursor zc_tile(dz, zb);
+  auto load_tiles = [&]() {
     const int s2 = zc_tile.src();
-    t0.load(b, u, plane, s2);
-    if constexpr (NI == 3) {
-      t1.load(b, u + g.np, plane, s2);
-      t2.load(b, u + 2 * g.np, plane, s2);
-    }
+    t0.load(m0, u, plane, s2);
+    if constexpr (NI == 3) t1.load(m1, u + g.np, plane, s2);
+    if constexpr (PNeed<MODE, 2>::TILE && NI == 3) t2.load(m1, u + 2 * g.np, plane, s2);
     zc_tile.next();
   };
-  const int cboff = plane_boff<R>(out_ok ? i0 + g.n0 * i1 : -1);
-  auto col_next = [&]() -> R {
-    const R v = plane_ld<R>(plane_rsrc(uz, plane, zc_col.src()), cboff);
-    zc_col.next();
-    return v;
-  };
-  // planes z + M (column) and z (tiles) are loaded two steps ahead of use
-  R win[W];
+  // (a pair whose second column lies past the grid is loaded one column
+  // earlier, so that no load runs past the plane)
+  const int cboff = plane_boff<R>(out_ok ? i0 + g.n0 * i1 - (both ? 0 : 1) : -1);
+  auto col_at = [&](const ZCursor& c) -> T2 { return pz_ld2<R>(plane_rsrc(uz, plane, c.src()), cboff); };
+  // the window: planes c, c + 1, .. of both columns (c moves past them)
+  auto load_window = [&](ZCursor& c, R (&win)[W][2]) {
+    T2 first[W];
 #pragma unroll
-  for (int k = 0; k < W - 1; ++k) win[k] = col_next();  // planes zb - M .. zb + M - 1
-  R nxt[2];
-  nxt[0] = col_next();
-  nxt[1] = col_next();
-  load_tiles(0);
-  load_tiles(1);
-
-  // x- / y-stencil of a tile at this lane (centred taps from scalar
-  // registers; the shifted border rows per lane)
-  auto sx = [&](const R* T) {
-    const R* v = T + lr * TWP + xs;
-    R s = R(0);
-    if (!bx) {
-#pragma unroll
-      for (int j = 0; j < W; ++j) s = fmar(prow<R, NORD>(M * W + j), v[j], s);
-    } else {
-#pragma unroll
-      for (int j = 0; j < W; ++j) s = fmar(rows[xrow + j], v[j], s);
+    for (int k = 0; k < W; ++k) {
+      first[k] = col_at(c);
+      c.next();
     }
-    return s;
+#pragma unroll
+    for (int k = 0; k < W; ++k) {
+      win[k][0] = both ? first[k].x : first[k].y;
+      win[k][1] = first[k].y;
+    }
   };
-  auto sy = [&](const R* T) {
+  load_tiles();
+
+  // order 16: six taps' LDS reads in flight at a time (all of them take more
+  // registers than there are)
+  auto fence = [&]() {
+    if constexpr (NORD == 16) __builtin_amdgcn_sched_barrier(0);
+  };
+  auto fence_at = [&](int j) {
+    if (j % 6 == 5) fence();
+  };
+  // x- / y-stencils of both columns from a tile (centred taps are constants;
+  // the shifted border rows come per lane)
+  auto sx = [&](const R* T, R* d) {
+    d[0] = d[1] = R(0);
+    if (!bx) {
+      const T2* v = reinterpret_cast<const T2*>(T + lr * TWP + (lc - M));
+#pragma unroll
+      for (int k = 0; k < W + 1; k += 2) {
+        const T2 q = v[k / 2];
+        const R e0 = q.x, e1 = q.y;
+        if (k < W) d[0] = fmar(prow<R, NORD>(M * W + k), e0, d[0]);
+        if (k > 0) d[1] = fmar(prow<R, NORD>(M * W + k - 1), e0, d[1]);
+        if (k + 1 < W) d[0] = fmar(prow<R, NORD>(M * W + k + 1), e1, d[0]);
+        d[1] = fmar(prow<R, NORD>(M * W + k), e1, d[1]);
+        if (k % 8 == 6) fence();
+      }
+    } else {
+      const R* v = T + lr * TWP;
+#pragma unroll
+      for (int e = 0; e < 2; ++e)
+#pragma unroll
+        for (int j = 0; j < W; ++j) {
+          d[e] = fmar(rows[xrow[e] + j], v[xs[e] + j], d[e]);
+          fence_at(j);
+        }
+    }
+    d[0] *= rh0;
+    d[1] *= rh0;
+    fence();
+  };
+  auto pair = [&](const R* v) -> T2 {  // columns lc, lc + 1 of a tile row
+    if constexpr (M % 2 == 0) {
+      return *reinterpret_cast<const T2*>(v);
+    } else {
+      T2 q;
+      q.x = v[0];
+      q.y = v[1];
+      return q;
+    }
+  };
+  auto sy = [&](const R* T, R* d) {
     const R* v = T + ys * TWP + lc;
-    R s = R(0);
+    d[0] = d[1] = R(0);
     if (!by) {
 #pragma unroll
-      for (int j = 0; j < W; ++j) s = fmar(prow<R, NORD>(M * W + j), v[j * TWP], s);
+      for (int j = 0; j < W; ++j) {
+        const T2 q = pair(v + j * TWP);
+        d[0] = fmar(prow<R, NORD>(M * W + j), q.x, d[0]);
+        d[1] = fmar(prow<R, NORD>(M * W + j), q.y, d[1]);
+        fence_at(j);
+      }
     } else {
 #pragma unroll
-      for (int j = 0; j < W; ++j) s = fmar(rows[yrow + j], v[j * TWP], s);
+      for (int j = 0; j < W; ++j) {
+        const T2 q = pair(v + j * TWP);
+        d[0] = fmar(rows[yrow + j], q.x, d[0]);
+        d[1] = fmar(rows[yrow + j], q.y, d[1]);
+        fence_at(j);
+      }
     }
-    return s;
+    d[0] *= rh1;
+    d[1] *= rh1;
+    fence();
   };
-  auto ctr = [&](const R* T) { return T[lr * TWP + lc]; };
 
   double sq = 0.0;  // update_rhopol: this lane's sum of res^2, z in order
-  auto step = [&](int z, int b) {  // b = (z - zb) & 1, static after unrolling
-    win[W - 1] = nxt[b];
-    t0.store(b, lds);
-    if constexpr (NI == 3) {
-      t1.store(b, lds + TSZ);
-      t2.store(b, lds + 2 * TSZ);
-    }
-    nxt[b] = col_next();
-    load_tiles(b);
+  // output plane z with the z-stencil zdot
+  auto step = [&](int z, auto zdot) {
+    t0.store(m0, lds);
+    if constexpr (NI == 3) t1.store(m1, lds + TSZ);
+    if constexpr (PNeed<MODE, 2>::TILE && NI == 3) t2.store(m1, lds + 2 * TSZ);
+    load_tiles();
     __syncthreads();
     if (out_ok) {
       const long p = (long)z * plane + i0 + (long)g.n0 * i1;
-      R dzv = R(0);
-#pragma unroll
-      for (int j = 0; j < W; ++j) dzv = fmar(prow<R, NORD>(M * W + j), win[j], dzv);
+      R dzv[2];
+      zdot(dzv);
+      dzv[0] *= rh2;
+      dzv[1] *= rh2;
+      fence();
       if constexpr (MODE >= GE_GRAD) {
-        const R dx = sx(lds) * rh0, dy = sy(lds) * rh1, dz2 = dzv * rh2;
-        sq += grad_epilogue<R, MODE>(ep, g.np, p, dx, dy, dz2);
+        R d[3][2];
+        sx(lds, d[0]);
+        sy(lds, d[1]);
+        d[2][0] = dzv[0];
+        d[2][1] = dzv[1];
+        sq += grad_epilogue2<R, MODE>(ep, g.np, p, both, d);
       } else {
-        const R dx = sx(lds) * rh0;
-        const R dy = sy(lds + TSZ) * rh1;
-        const R dz2 = dzv * rh2;
-        o0[p] = (dx + dy) + dz2;
+        R dx[2], dy[2], o[2];
+        sx(lds, dx);
+        sy(lds + TSZ, dy);
+#pragma unroll
+        for (int e = 0; e < 2; ++e) o[e] = (dx[e] + dy[e]) + dzv[e];
+        pz_put(o0, p, o, both);
         if constexpr (MODE == 1) {
-          const R x = ctr(lds), y = ctr(lds + TSZ), zv = win[M];
-          const R xy = sx(lds + TSZ) * rh0;
-          const R xz = sx(lds + 2 * TSZ) * rh0;
-          const R yz = sy(lds + 2 * TSZ) * rh1;
-          o1[p] = (((x * x) * dx + (y * y) * dy) + (zv * zv) * dz2) +
-                  R(2) * ((x * y * xy + x * zv * xz) + y * zv * yz);
+          R xy[2], xz[2], yz[2];
+          sx(lds + TSZ, xy);
+          sx(lds + 2 * TSZ, xz);
+          sy(lds + 2 * TSZ, yz);
+          const T2 cx = pair(lds + lr * TWP + lc);
+          const T2 cy = pair(lds + TSZ + lr * TWP + lc);
+          const T2 cz = pair(lds + 2 * TSZ + lr * TWP + lc);
+#pragma unroll
+          for (int e = 0; e < 2; ++e) {
+            const R x = e ? cx.y : cx.x, y = e ? cy.y : cy.x, zv = e ? cz.y : cz.x;
+            o[e] = (((x * x) * dx[e] + (y * y) * dy[e]) + (zv * zv) * dzv[e]) +
+                   R(2) * ((x * y * xy[e] + x * zv * xz[e]) + y * zv * yz[e]);
+          }
+          pz_put(o1, p, o, both);
         }
       }
     }
     __syncthreads();
-#pragma unroll
-    for (int k = 0; k < W - 1; ++k) win[k] = win[k + 1];
   };
-  for (int z = zb; z < ze; z += 4) {  // four steps per trip: static buffers
-    step(z, 0);
-    if (z + 1 < ze) step(z + 1, 1);
-    if (z + 2 < ze) step(z + 2, 0);
-    if (z + 3 < ze) step(z + 3, 1);
+  // a border plane of a non-periodic z: row `row` on the window's planes
+  auto border = [&](int z, const R (&win)[W][2], int row) {
+    step(z, [&](R* d) {
+      d[0] = d[1] = R(0);
+#pragma unroll
+      for (int j = 0; j < W; ++j) {
+        d[0] = fmar(rows[row * W + j], win[j][0], d[0]);
+        d[1] = fmar(rows[row * W + j], win[j][1], d[1]);
+        fence_at(j);
+      }
+    });
+  };
+  int z = zb;  // (the rows are read after the first step's barrier)
+  const int zl = g.per2 ? zb : min(ze, M), zh = g.per2 ? ze : min(ze, g.n2 - M);
+  if (z < zl) {  // the first M planes, on planes 0 .. 2M
+    ZCursor c(dz, 0);
+    R win[W][2];
+    load_window(c, win);
+    for (; z < zl; ++z) border(z, win, z);
+  }
+  if (z < zh) {
+    ZCursor c(dz, z - M);
+    R win[W][2];
+    load_window(c, win);
+    T2 nxt = col_at(c);
+    c.next();
+    for (;;) {
+#pragma unroll
+      for (int k = 0; k < 4; ++k) {  // four steps per trip: the window moves by renaming
+        step(z, [&](R* d) {
+          d[0] = d[1] = R(0);
+#pragma unroll
+          for (int j = 0; j < W; ++j) {
+            d[0] = fmar(prow<R, NORD>(M * W + j), win[j][0], d[0]);
+            d[1] = fmar(prow<R, NORD>(M * W + j), win[j][1], d[1]);
+          }
+        });
+        if (++z >= zh) goto high;
+#pragma unroll
+        for (int j = 0; j < W - 1; ++j) {
+          win[j][0] = win[j + 1][0];
+          win[j][1] = win[j + 1][1];
+        }
+        win[W - 1][0] = both ? nxt.x : nxt.y;
+        win[W - 1][1] = nxt.y;
+        nxt = col_at(c);
+        c.next();
+      }
+    }
+  }
+high:
+  if (z < ze) {  // the last M planes, on planes n - 1 - 2M .. n - 1
+    ZCursor c(dz, g.n2 - W);
+    R win[W][2];
+    load_window(c, win);
+    for (; z < ze; ++z) border(z, win, z - g.n2 + W);
   }
   if constexpr (MODE == GE_RHOPOL) {
     __shared__ double red[NT / 64];
@@ -578,35 +769,41 @@ hipError_t poisson_1d(int nord, int idim, const int* n, int bc, const R* u, R* d
   return hipGetLastError();
 }
 
-// z-march launch shape: tiles x z chunks of the planes zlo .. zhi - 1 (all,
-// or on a non-periodic z the planes off its border).  The chunks put at most
-// `resident` blocks (what one CU holds of the kernel) on any CU, so the grid
-// runs in one even round, yet at least one block per CU where the grid
-// allows; chunks no shorter than 2 stencil lengths.  False when the
-// one-point kernels must do all (LIBCONV_POISSON_POINT set, planes beyond
-// the buffer-record limit).
+// z-march launch shape: tiles x z chunks.  The chunks put at most `resident`
+// blocks (what one CU holds of the kernel) on any CU, so the grid runs in one
+// even round; a chunk repeats only the 2m column loads of its window, so
+// chunks go down to 6 planes for that, and to 2 when the grid would leave CUs
+// without a block (order 4 on 100 x 60 x 40: 11.6 us against 13.8 with 4).
+// False when the one-point kernels must do all (LIBCONV_POISSON_POINT set,
+// planes beyond the buffer-record limit).
 struct PzLaunch {
-  int tiles_x, tiles, zlo, zhi, zchunk;
+  int tiles_x, tiles, zchunk;
   unsigned blocks;
 };
-static bool pz_launch(const PGeom& g, int nord, int ty, int resident, PzLaunch& L) {
+static bool pz_launch(const PGeom& g, int ty, int resident, PzLaunch& L) {
   if (getenv("LIBCONV_POISSON_POINT")) return false;
   if ((long)g.n0 * g.n1 * 8 > kPlaneMax) return false;
-  const int m = nord / 2;
-  L.zlo = g.per2 ? 0 : m;
-  L.zhi = g.per2 ? g.n2 : g.n2 - m;
-  const int nz = L.zhi - L.zlo;  // >= 1: n >= nord + 1
   L.tiles_x = (g.n0 + kZTX - 1) / kZTX;
   const long tiles = (long)L.tiles_x * ((g.n1 + ty - 1) / ty);
-  long chunks = (long)std::max(1, resident) * num_cu() / tiles;
-  if (chunks * tiles < num_cu()) chunks = (num_cu() + tiles - 1) / tiles;
-  chunks = std::max(1L, std::min<long>(chunks, nz / (2 * (nord + 1))));
-  L.zchunk = (int)((nz + chunks - 1) / chunks);
-  const long nb = tiles * ((nz + L.zchunk - 1) / L.zchunk);
+  long chunks = std::min<long>((long)std::max(1, resident) * num_cu() / tiles, g.n2 / 6);
+  if (chunks * tiles < num_cu()) chunks = std::min<long>((num_cu() + tiles - 1) / tiles, g.n2 / 2);
+  chunks = std::max(1L, chunks);
+  L.zchunk = (int)((g.n2 + chunks - 1) / chunks);
+  const long nb = tiles * ((g.n2 + L.zchunk - 1) / L.zchunk);
   if (nb > 0x7fffffffL) return false;
   L.tiles = (int)tiles;
   L.blocks = (unsigned)nb;
   return true;
+}
+// tile rows: 16; 32 for the gradient operators of order 16, whose y halo is as
+// high as the tile (nabla_u_and_square at 256^3: FP64 151 us against 179, FP32
+// 68 against 93), where that still gives a CU two chunks of 16 planes.
+// div_u_i holds three tiles and gains nothing (FP64 257 against 240 us).
+template <int NO, int MODE>
+static constexpr bool pz_tall() { return NO == 16 && MODE >= GE_GRAD; }
+static bool pz_fills(const PGeom& g) {
+  const long tiles = (long)((g.n0 + kZTX - 1) / kZTX) * ((g.n1 + 31) / 32);
+  return tiles * (g.n2 / 16) >= 2L * num_cu();
 }
 
 // blocks of one z-march kernel that a CU holds (registers, LDS), cached
@@ -621,29 +818,26 @@ static int pz_resident() {
   return nb;
 }
 
-// one z-march launch; *done false when the one-point kernels must run
-template <typename R, int NO, int MODE>
-static hipError_t pz_run(const PGeom& g, const R* u, R* o0, R* o1, R r0, R r1, R r2, hipStream_t st,
-                         bool* done) {
+// one z-march launch; its blocks, or 0 when the one-point kernels must run;
+// dry: count only
+template <typename R, int NO, int MODE, int TY>
+static long pz_run_rows(const PGeom& g, const R* u, R* o0, R* o1, const GradEpi<R>& ep, R r0, R r1, R r2,
+                        hipStream_t st, bool dry) {
+  constexpr int NT = PzGeo<R, NO, TY>::NT;
   PzLaunch L;
-  *done = pz_launch(g, NO, pz_ty<MODE>(), pz_resident<poisson_zm_kernel<R, NO, MODE>, pz_nt<MODE>()>(), L);
-  if (!*done) return hipSuccess;
-  poisson_zm_kernel<R, NO, MODE><<<L.blocks, pz_nt<MODE>(), 0, st>>>(g, L.tiles_x, L.tiles, L.zlo, L.zhi, L.zchunk,
-                                                                     u, o0, o1, GradEpi<R>{}, r0, r1, r2);
-  return hipGetLastError();
+  if (!pz_launch(g, TY, pz_resident<poisson_zm_kernel<R, NO, MODE, TY>, NT>(), L)) return 0;
+  if (!dry)
+    poisson_zm_kernel<R, NO, MODE, TY><<<L.blocks, NT, 0, st>>>(g, L.tiles_x, L.tiles, L.zchunk, u, o0, o1, ep, r0,
+                                                                r1, r2);
+  return L.blocks;
 }
-
-// the planes of a non-periodic z the z march leaves out: 0 .. m - 1 and
-// n - m .. n - 1, as two one-point launches (g.z0 / g.nz select the planes)
-template <typename F>
-static void pz_border_planes(const PGeom& g, int nord, F&& launch) {
-  if (g.per2) return;
-  PGeom b = g;
-  b.nz = nord / 2;
-  b.z0 = 0;
-  launch(b);
-  b.z0 = g.n2 - nord / 2;
-  launch(b);
+template <typename R, int NO, int MODE>
+static long pz_run(const PGeom& g, const R* u, R* o0, R* o1, const GradEpi<R>& ep, R r0, R r1, R r2, hipStream_t st,
+                   bool dry) {
+  if constexpr (pz_tall<NO, MODE>()) {
+    if (pz_fills(g)) return pz_run_rows<R, NO, MODE, 32>(g, u, o0, o1, ep, r0, r1, r2, st, dry);
+  }
+  return pz_run_rows<R, NO, MODE, 16>(g, u, o0, o1, ep, r0, r1, r2, st, dry);
 }
 
 template <typename R>
@@ -655,48 +849,26 @@ hipError_t div_u_i(int geocode, const int* n, const R* u, R* du, R* cc, int nord
     LC_POISSON_DISPATCH(nord, (div_u_i_kernel<R, NO><<<pgrid(q), kPThreads, 0, st>>>(q, psegs(q), u, du, cc, r0, r1, r2)))
     return hipGetLastError();
   };
-  bool done = false;
-  hipError_t e = hipSuccess;
+  long done = 0;
   if (cc) {
-    LC_POISSON_DISPATCH(nord, (e = pz_run<R, NO, 1>(g, u, du, cc, r0, r1, r2, st, &done)))
+    LC_POISSON_DISPATCH(nord, (done = pz_run<R, NO, 1>(g, u, du, cc, GradEpi<R>{}, r0, r1, r2, st, false)))
   } else {
-    LC_POISSON_DISPATCH(nord, (e = pz_run<R, NO, 0>(g, u, du, cc, r0, r1, r2, st, &done)))
+    LC_POISSON_DISPATCH(nord, (done = pz_run<R, NO, 0>(g, u, du, cc, GradEpi<R>{}, r0, r1, r2, st, false)))
   }
-  if (e != hipSuccess) return e;
-  if (!done) return point(g);
-  pz_border_planes(g, nord, [&](const PGeom& q) { if (e == hipSuccess) e = point(q); });
-  return e;
+  return done ? hipGetLastError() : point(g);
 }
 
-// The launches of one gradient-family operator: the z march over the planes
-// off a non-periodic z border and the one-point kernels on the border planes,
-// or the one-point kernels on every plane.  Returns their block count, which
-// is the number of partial sums update_rhopol writes (ep.part[0 .. count));
-// dry: count only, nothing launched.
+// The launch of one gradient-family operator: the z march, or the one-point
+// kernel.  Returns its block count, which is the number of partial sums
+// update_rhopol writes (ep.part[0 .. count)); dry: count only.
 template <typename R, int NO, int MODE>
 static long grad_launch(const PGeom& g, const R* u, const GradEpi<R>& ep, R r0, R r1, R r2, hipStream_t st,
                         bool dry) {
-  long off = 0;
-  auto point = [&](const PGeom& q) {
-    const unsigned nb = pgrid(q);
-    if (!dry) {
-      GradEpi<R> e = ep;
-      if (e.part) e.part += off;
-      grad_point_kernel<R, NO, MODE><<<nb, kPThreads, 0, st>>>(q, psegs(q), u, e, r0, r1, r2);
-    }
-    off += nb;
-  };
-  PzLaunch L;
-  if (!pz_launch(g, NO, pz_ty<MODE>(), pz_resident<poisson_zm_kernel<R, NO, MODE>, pz_nt<MODE>()>(), L)) {
-    point(g);
-    return off;
-  }
-  if (!dry)
-    poisson_zm_kernel<R, NO, MODE><<<L.blocks, pz_nt<MODE>(), 0, st>>>(g, L.tiles_x, L.tiles, L.zlo, L.zhi,
-                                                                       L.zchunk, u, nullptr, nullptr, ep, r0, r1, r2);
-  off += L.blocks;
-  pz_border_planes(g, NO, point);
-  return off;
+  const long nb = pz_run<R, NO, MODE>(g, u, nullptr, nullptr, ep, r0, r1, r2, st, dry);
+  if (nb) return nb;
+  const unsigned np = pgrid(g);
+  if (!dry) grad_point_kernel<R, NO, MODE><<<np, kPThreads, 0, st>>>(g, psegs(g), u, ep, r0, r1, r2);
+  return np;
 }
 
 template <typename R, int MODE>
