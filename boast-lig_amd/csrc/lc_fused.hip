@@ -212,7 +212,7 @@ int select_variant(int prec, int form, int id, const Box3& b) {
       const int g = FMD::N - 1;  // outputs per dim: grow adds the filter length
       const long plane = (long)(b.bc[0] == GROW ? b.n[0] + g : b.n[0]) * (b.bc[1] == GROW ? b.n[1] + g : b.n[1]);
       if (prec == 8) return 62;
-      return plane >= 200L * 200 ? 68 : 41;
+      return plane >= 200L * 200 ? 68 : 60;
     }
     if (!fit) return prec == 4 ? 7 : 8;
     if (prec == 8) return 46;

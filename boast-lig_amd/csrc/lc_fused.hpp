@@ -202,6 +202,33 @@ inline int pick_zchunk(long tiles, int nz, int narr, int w, int ncu) {
   return (int)((nz + chunks - 1) / chunks);
 }
 
+// z chunk by the expected time of the busiest CU, in units of one plane of a
+// block alone on its CU.  A single block is bound by the latency of a plane's
+// barriers and loads, so the second one costs little, further ones their full
+// throughput share:
+//   time = fix + blk k + (chunk + pre) max(1, add + mul k)
+// with k blocks on the busiest CU, `pre` planes that a chunk repeats, `fix` the
+// launch and the first loads, `blk` a block's window prefill.  At most `cap`
+// blocks on a CU where the tiles allow, no chunk shorter than 4 planes, no more
+// than maxc chunks, chunks of whole steps of q planes.
+struct ZCost {
+  double fix, blk, pre, add, mul;
+};
+inline int cost_zchunk(const ZCost& m, long tiles, int nz, int narr, int cap, long maxc, int q, int ncu) {
+  const long per = std::max(1L, tiles * std::max(narr, 1));
+  const long kmax = std::max<long>(cap, (per + ncu - 1) / ncu);
+  int best = (std::max(1, nz) + q - 1) / q * q;
+  double bt = 1e300;
+  for (long c = 1; c <= std::max(1L, std::min<long>(maxc, nz / 4)); ++c) {
+    const int zc = (int)(((nz + c - 1) / c + q - 1) / q * q);
+    const long n = (nz + zc - 1) / zc, k = (n * per + ncu - 1) / ncu;
+    if (c > 1 && k > kmax) break;
+    const double t = m.fix + m.blk * k + (zc + m.pre) * std::max(1.0, m.add + m.mul * k);
+    if (t < bt) bt = t, best = zc;
+  }
+  return best;
+}
+
 inline int num_cu() {
   static int g_ncu = 0;
   if (!g_ncu) {

@@ -208,13 +208,16 @@ hipError_t launch_sum3d2(const Box3& b, int narr, const R* x, R* y, const double
   if (ZC == 0) {
     p.zchunk = pick_zchunk(tiles, p.d2.nout, std::max(narr, 1), F::N, num_cu());
   } else if (ZC < 0) {
-    // at most -ZC blocks on any CU, at least one where the grid allows
-    const long per = tiles * std::max(narr, 1);
-    long chunks = (long)(-ZC) * num_cu() / per;
-    if (chunks * per < num_cu()) chunks = (num_cu() + per - 1) / per;
-    chunks = std::max(1L, std::min<long>(chunks, std::max(1, p.d2.nout / 16)));
-    p.zchunk = (int)((p.d2.nout + chunks - 1) / chunks);
-    p.zchunk = (p.zchunk + QZ - 1) / QZ * QZ;
+    // at most -ZC blocks on any CU; no more partial sums than the scratch holds.
+    // A block's prefill (W - 1 column loads per lane) takes the time of about
+    // ten planes, three for each block more; two FP64 blocks on a CU run a
+    // plane in 1.6 times the time of one (fitted to 1 - 5 blocks per CU on
+    // 24^3 to 256^3).  Chunks of 16 planes and more, filling the CUs, took
+    // 26 us on 24^3, 22 on 100 x 90 x 110 and 32 on 143^3 in FP64; now 16
+    // (the host's launch rate), 18 and 29.
+    const ZCost m = sizeof(R) == 8 ? ZCost{13, 3.1, 0, 0, 0.8} : ZCost{9, 3, 0, 0, 0.58};
+    const long maxc = (long)fused_sum3d_parts(b, narr, F::LO, F::UP, F::N) / tiles;
+    p.zchunk = cost_zchunk(m, tiles, p.d2.nout, narr, -ZC, maxc, QZ, num_cu());
   } else {
     // a z chunk only costs the window prefill (W - 1 column loads per lane):
     // chunks down to ZC planes put ~8 blocks on every CU, and down to 16
@@ -433,15 +436,15 @@ int sep_plane_args(const Box3& b, int narr, const R* x, R* y, R a, R a_y, const 
   if (ZC == 0) {
     p.zchunk = pick_zchunk(tiles, p.d2.nout, std::max(narr, 1), F::N, num_cu());
   } else if (ZC < 0) {
-    // at most -ZC blocks on any CU: chunks = floor(-ZC CUs / tiles), so no
-    // CU holds one block more than the others (balance beats occupancy: 162
-    // tiles of 284 planes run 486 blocks of 95 planes 6% faster than 648 of
-    // 71), yet at least one block per CU where the grid allows
-    const long per = tiles * std::max(narr, 1);
-    long chunks = (long)(-ZC) * num_cu() / per;
-    if (chunks * per < num_cu()) chunks = (num_cu() + per - 1) / per;
-    chunks = std::max(1L, std::min<long>(chunks, std::max(1, p.d2.nout / (2 * F::N))));
-    p.zchunk = (int)((p.d2.nout + chunks - 1) / chunks);
+    // at most -ZC blocks on any CU (balance beats occupancy: 162 tiles of 284
+    // planes run 486 blocks of 95 planes 6% faster than 648 of 71).  A chunk
+    // repeats W - 1 planes; two FP64 blocks on a CU run a plane in 1.74 times
+    // the time of one, two FP32 ones in 1.55 (fitted to 1 - 5 blocks per CU on
+    // 24^3 to 256^3).  Chunks of 2 W planes and more left CUs idle on small
+    // grids: 37 us on 48^3, 32 on 100 x 90 x 110, 30 on 128^3 in FP64, 47 on
+    // 200^3 in FP32; now 16 (the host's launch rate), 20, 23 and 37.
+    const ZCost m = sizeof(R) == 8 ? ZCost{10, 0, F::N - 1, 0, 0.87} : ZCost{10, 0, F::N - 1, 0.15, 0.7};
+    p.zchunk = cost_zchunk(m, tiles, p.d2.nout, narr, -ZC, p.d2.nout, 1, num_cu());
   } else {
     // a chunk recomputes W - 1 filtered planes: shorter chunks buy occupancy
     const long per = tiles * std::max(narr, 1);
