@@ -212,7 +212,6 @@ __device__ __forceinline__ void sepp_body(const FusedArgs<R>& p, int bx, int by,
         if (out_ok) {
           R* yp = ya + (ocol + zo);
           if (p.flags & F_AY) sum = fmar(p.a_y, *yp, sum);
-          if (p.flags & F_POT) sum = pot_step(p, ocol + zo, sum);
           *yp = sum;
         }
         zo += syo;

@@ -81,14 +81,19 @@ struct SepqGeo {
   static_assert(W % 2 == 0 && W % PD == 0, "static ring and prefetch slots");
 };
 
-// ME: the epilogue reads or writes memory besides the output (F_AY, F_POT).
+// ME: the epilogue reads memory besides the output's place (F_AY).
 // Without (ME false) every wave issues the same memory operations in every
 // step: the y-waves' outputs are stored after the x/y branch, by all waves,
 // as buffer stores that drop the x-waves' and the invalid lanes' values (out
 // of range).  The compiler's wait counts are then exact, and a step waits for
 // the tile loads it uses, not for the previous step's stores.
 // NTS (ME false): streaming (non-temporal) output stores.
-template <typename R, class F, int TX, int TY, int QX, int QY, int PD, bool ME = true, bool NTS = false>
+// PT (ME false): the potential step in the same manner: rho += t^2, y = pot t.
+// Every wave issues the loads of pot and rho one step ahead of their use (two
+// or three steps ahead measured the same) and the store of rho beside that of
+// y; a null rho is a descriptor of no bytes.
+template <typename R, class F, int TX, int TY, int QX, int QY, int PD, bool ME = true, bool NTS = false,
+          bool PT = false>
 __device__ __forceinline__ void sepq_body(const FusedArgs<R>& p, int bx, int by, int zc, int arr,
                                           unsigned char* lds) {
   using G = SepqGeo<R, F, TX, TY, QX, QY, PD>;
@@ -143,6 +148,13 @@ __device__ __forceinline__ void sepq_body(const FusedArgs<R>& p, int bx, int by,
   const long syo = (long)p.d0.ny * p.d1.ny;
   long zo = (long)(zb - p.d2.oy) * syo;
   ZCursor zc_ld(p.d2, pfirst + PD + 1);
+  // byte offsets of this lane's outputs in their plane (none: the x-waves)
+  int yoff[QY];
+#pragma unroll
+  for (int i = 0; i < QY; ++i)
+    yoff[i] = (!xwave && xin && i < yrows) ? (int)((ocol + (long)i * p.d0.ny) * (long)sizeof(R)) : kOffNone;
+  // PT: pot and rho of the outputs of this step and of the next
+  R pv[2][QY], rv[2][QY];
 
   R ring[QY][W];
 #pragma unroll
@@ -172,6 +184,17 @@ __device__ __forceinline__ void sepq_body(const FusedArgs<R>& p, int bx, int by,
 #pragma unroll
         for (int j = 0; j < NAP; ++j) bq[j] = plane_ld<R>(rs, aoff[j]);
         zc_ld.next();
+        if constexpr (PT) {  // of the plane that step s + 1 stores
+          const bool in = s + 1 >= W && s + 1 < nsteps;  // uniform
+          const long zn = in ? (long)(zb + s + 1 - W - p.d2.oy) * syo : 0, no = in ? syo : 0;
+          const __amdgpu_buffer_rsrc_t rp = span_rsrc(p.pot + zn, no);
+          const __amdgpu_buffer_rsrc_t rr = span_rsrc(p.rho + zn, p.rho ? no : 0);
+#pragma unroll
+          for (int i = 0; i < QY; ++i) {
+            pv[(u + 1) & 1][i] = plane_ld<R>(rp, yoff[i]);
+            rv[(u + 1) & 1][i] = plane_ld<R>(rr, yoff[i]);
+          }
+        }
       }
       R outv[QY];  // ME false: the step's outputs of this lane
 #pragma unroll
@@ -230,7 +253,6 @@ __device__ __forceinline__ void sepq_body(const FusedArgs<R>& p, int bx, int by,
                 const long o = ocol + (long)i * p.d0.ny + zo;
                 R* yp = ya + o;
                 if (p.flags & F_AY) sum = fmar(p.a_y, *yp, sum);
-                if (p.flags & F_POT) sum = pot_step(p, o, sum);
                 *yp = sum;
               }
             }
@@ -251,10 +273,16 @@ __device__ __forceinline__ void sepq_body(const FusedArgs<R>& p, int bx, int by,
         // the outputs of planes s - W (before plane W: none), stored by every wave
         const bool em = s >= W;  // uniform
         const __amdgpu_buffer_rsrc_t ro = span_rsrc(ya + zo, em ? syo : 0);
+        if constexpr (PT) {
+          const __amdgpu_buffer_rsrc_t rr = span_rsrc(p.rho + zo, em && p.rho ? syo : 0);
 #pragma unroll
-        for (int i = 0; i < QY; ++i)
-          plane_st<R, NTS>(ro, (!xwave && xin && i < yrows) ? (int)((ocol + (long)i * p.d0.ny) * (long)sizeof(R)) : kOffNone,
-                      outv[i]);
+          for (int i = 0; i < QY; ++i) {
+            plane_st<R>(rr, yoff[i], fmar(outv[i], outv[i], rv[u & 1][i]));
+            outv[i] = pv[u & 1][i] * outv[i];
+          }
+        }
+#pragma unroll
+        for (int i = 0; i < QY; ++i) plane_st<R, NTS>(ro, yoff[i], outv[i]);
         zo += em ? syo : 0;
       }
       __syncthreads();

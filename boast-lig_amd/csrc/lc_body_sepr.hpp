@@ -186,7 +186,6 @@ __device__ __forceinline__ void sepr_body(const FusedArgs<R>& p, int bx, int by,
               const long o = ocol + (long)i * p.d0.ny + zo;
               R* yp = ya + o;
               if (p.flags & F_AY) sum = fmar(p.a_y, *yp, sum);
-              if (p.flags & F_POT) sum = pot_step(p, o, sum);
               *yp = sum;
             }
           }

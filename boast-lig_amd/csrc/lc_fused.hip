@@ -62,6 +62,10 @@ hipError_t fused_stage_t(bool build, int kind, const BatchItem<R>* it, int count
                                                  const R*, R*);                                          \
   extern template hipError_t fused_stage_t<R, F>(bool, int, const BatchItem<R>*, int, BatchStage*,       \
                                                  hipStream_t);
+extern template hipError_t launch_sepq_pot<double>(const Box3&, const double*, double*, double, hipStream_t,
+                                                   const double*, double*);
+extern template hipError_t launch_sepq_pot<float>(const Box3&, const float*, float*, float, hipStream_t,
+                                                  const float*, float*);
 LC_FUSED_EXTERN(double, FMD)
 LC_FUSED_EXTERN(double, FIMD)
 LC_FUSED_EXTERN(double, FD2)
@@ -269,11 +273,10 @@ hipError_t sep3d_fused_run(int id, const Box3& b, int narr, const R* x, R* y, R 
   int v = select_variant(sizeof(R), FORM_SEP, id, b);
   if (pot && v >= 5 && v <= 7)  // the wave-specialised forms have no potential step
     v = plane_fits(b, sizeof(R)) ? (sizeof(R) == 4 ? 28 : 33) : 12;
-  // with the potential step the 128-bit-LDS kernels take their general
-  // epilogue (stores inside the y-waves' branch, conservative wait counts):
-  // the pipelined kernel is faster there (the local Hamiltonian's 157^3
-  // magic filter: 0.203 against 0.226 ms for the whole chain)
-  if (pot && v >= 62 && v <= 72) v = sizeof(R) == 4 ? 41 : 45;
+  // nor have the pipelined, ring-owning and 128-bit-LDS forms: for these it
+  // is a kernel of its own
+  if (pot && v >= 37 && v <= 72 && id == OP_MD && narr == 1 && a_y == R(0))
+    return launch_sepq_pot<R>(b, x, y, a, st, pot, rho);
   return sep3d_fused_v<R>(v, id, b, narr, x, y, a, a_y, st, pot, rho);
 }
 

@@ -500,14 +500,13 @@ template <class F>
 constexpr bool sepp_filter() { return F::N == 16; }
 
 template <typename R, class F, int TX, int TY, int QX, int QY, int PD, int WPE, int ZC>
-hipError_t launch_sepp(const Box3& b, int narr, const R* x, R* y, R a, R a_y, hipStream_t st,
-                       const R* pot, R* rho) {
+hipError_t launch_sepp(const Box3& b, int narr, const R* x, R* y, R a, R a_y, hipStream_t st) {
   if constexpr (!sepp_filter<F>()) {
     return hipErrorInvalidValue;
   } else {
     if (!plane_fits(b, sizeof(R))) return hipErrorInvalidValue;
     FusedArgs<R> p;
-    const int zch = sep_plane_args<R, F, TX, TY, ZC>(b, narr, x, y, a, a_y, pot, rho, p);
+    const int zch = sep_plane_args<R, F, TX, TY, ZC>(b, narr, x, y, a, a_y, nullptr, nullptr, p);
     if (narr == 0) return hipSuccess;
     dim3 grid((unsigned)(p.tiles_x * p.tiles_y), (unsigned)zch, (unsigned)narr);
     sepp_fused<R, F, TX, TY, QX, QY, PD, WPE><<<grid, TX * TY, 0, st>>>(p);
@@ -548,14 +547,13 @@ __attribute__((amdgpu_waves_per_eu(WPE))) void sepr_batch(const FusedArgs<R>* __
 }
 
 template <typename R, class F, int TX, int TY, int QX, int QY, int PD, int WPE, int ZC>
-hipError_t launch_sepr(const Box3& b, int narr, const R* x, R* y, R a, R a_y, hipStream_t st,
-                       const R* pot, R* rho) {
+hipError_t launch_sepr(const Box3& b, int narr, const R* x, R* y, R a, R a_y, hipStream_t st) {
   if constexpr (!sepp_filter<F>()) {
     return hipErrorInvalidValue;
   } else {
     if (!plane_fits(b, sizeof(R))) return hipErrorInvalidValue;
     FusedArgs<R> p;
-    const int zch = sep_plane_args<R, F, TX, TY, ZC>(b, narr, x, y, a, a_y, pot, rho, p);
+    const int zch = sep_plane_args<R, F, TX, TY, ZC>(b, narr, x, y, a, a_y, nullptr, nullptr, p);
     if (narr == 0) return hipSuccess;
     dim3 grid((unsigned)(p.tiles_x * p.tiles_y), (unsigned)zch, (unsigned)narr);
     sepr_fused<R, F, TX, TY, QX, QY, PD, WPE>
@@ -582,7 +580,7 @@ __attribute__((amdgpu_waves_per_eu(WPE))) void sepq_fused(FusedArgs<R> p) {
   __shared__ __align__(16) unsigned char lds[SepqGeo<R, F, TX, TY, QX, QY, PD>::lds_bytes()];
   int bx, by, zc, arr;
   block_coords(p.tiles_x, bx, by, zc, arr);
-  if (p.flags & (F_AY | F_POT))
+  if (p.flags & F_AY)
     sepq_body<R, F, TX, TY, QX, QY, PD, true>(p, bx, by, zc, arr, lds);
   else
     sepq_body<R, F, TX, TY, QX, QY, PD, false>(p, bx, by, zc, arr, lds);
@@ -597,7 +595,7 @@ __attribute__((amdgpu_waves_per_eu(WPE))) void sepq_batch(const FusedArgs<R>* __
   const int tiles = p.tiles_x * p.tiles_y;
   const int tile = local % tiles, zc = local / tiles;
   __shared__ __align__(16) unsigned char lds[SepqGeo<R, F, TX, TY, QX, QY, PD>::lds_bytes()];
-  if (p.flags & (F_AY | F_POT))
+  if (p.flags & F_AY)
     sepq_body<R, F, TX, TY, QX, QY, PD, true>(p, tile % p.tiles_x, tile / p.tiles_x, zc, 0, lds);
   else
     sepq_body<R, F, TX, TY, QX, QY, PD, false>(p, tile % p.tiles_x, tile / p.tiles_x, zc, 0, lds);
@@ -607,14 +605,13 @@ template <typename R, class F, int TX, int TY, int QX, int QY>
 constexpr bool sepq_ok() { return sepp_filter<F>() && sepq_shape_ok<R, TX, TY, QX, QY>(); }
 
 template <typename R, class F, int TX, int TY, int QX, int QY, int PD, int WPE, int ZC>
-hipError_t launch_sepq(const Box3& b, int narr, const R* x, R* y, R a, R a_y, hipStream_t st,
-                       const R* pot, R* rho) {
+hipError_t launch_sepq(const Box3& b, int narr, const R* x, R* y, R a, R a_y, hipStream_t st) {
   if constexpr (!sepq_ok<R, F, TX, TY, QX, QY>()) {
     return hipErrorInvalidValue;
   } else {
     if (!plane_fits(b, sizeof(R))) return hipErrorInvalidValue;
     FusedArgs<R> p;
-    const int zch = sep_plane_args<R, F, TX, TY, ZC>(b, narr, x, y, a, a_y, pot, rho, p);
+    const int zch = sep_plane_args<R, F, TX, TY, ZC>(b, narr, x, y, a, a_y, nullptr, nullptr, p);
     if (narr == 0) return hipSuccess;
     dim3 grid((unsigned)(p.tiles_x * p.tiles_y), (unsigned)zch, (unsigned)narr);
     sepq_fused<R, F, TX, TY, QX, QY, PD, WPE>
@@ -632,6 +629,49 @@ hipError_t launch_sepq_batch(const FusedArgs<R>* tab, const BatchStage* s, hipSt
         <<<s->grid, SepqGeo<R, F, TX, TY, QX, QY, PD>::NT, 0, st>>>(tab, batch_order_of(s));
     return hipSuccess;
   }
+}
+
+// ---- magic filter with the potential step of the local Hamiltonian (one
+// array, a_y = 0): y = pot t, rho += t^2 of the filtered value t.
+// Bound: memory, five arrays (x, pot and rho read, y and rho written).  The
+// pipelined kernels' epilogue had loads and stores inside a branch and so
+// waits for everything in flight: 78 us on the 157^3 points of 64^3 pairs in
+// FP64 and 55 us in FP32 (69% of the wave cycles were waits).  This one: 53 us
+// (155 MB, 2.9 TB/s) and 36 us; deeper prefetch, tiles of 32 x 32 and more
+// blocks are no faster in FP64 (53 - 57 us).  In FP32 a block has four waves,
+// and two blocks per CU run a plane in little more time than one: 36 against
+// 45 us.
+template <typename R>
+struct PotTile {
+  static constexpr int TX = 32, TY = 16, QX = sizeof(R) == 8 ? 4 : 8, QY = sizeof(R) == 8 ? 2 : 4, PD = 2,
+                       WPE = sizeof(R) == 8 ? 4 : 2;
+};
+template <typename R>
+using PotGeo = SepqGeo<R, FMD, PotTile<R>::TX, PotTile<R>::TY, PotTile<R>::QX, PotTile<R>::QY, PotTile<R>::PD>;
+
+template <typename R>
+__global__ __launch_bounds__((PotGeo<R>::NT)) __attribute__((amdgpu_waves_per_eu(PotTile<R>::WPE))) void sepq_pot(
+    FusedArgs<R> p) {
+  using T = PotTile<R>;
+  __shared__ __align__(16) unsigned char lds[PotGeo<R>::lds_bytes()];
+  int bx, by, zc, arr;
+  block_coords(p.tiles_x, bx, by, zc, arr);
+  sepq_body<R, FMD, T::TX, T::TY, T::QX, T::QY, T::PD, false, false, true>(p, bx, by, zc, arr, lds);
+}
+
+template <typename R>
+hipError_t launch_sepq_pot(const Box3& b, const R* x, R* y, R a, hipStream_t st, const R* pot, R* rho) {
+  using T = PotTile<R>;
+  if (!plane_fits(b, sizeof(R))) return hipErrorInvalidValue;
+  FusedArgs<R> p;
+  int zch = sep_plane_args<R, FMD, T::TX, T::TY, -2>(b, 1, x, y, a, R(0), pot, rho, p);
+  if (sizeof(R) == 4) {
+    p.zchunk = cost_zchunk(ZCost{10, 0, FMD::N - 1, 0.15, 0.5}, (long)p.tiles_x * p.tiles_y, p.d2.nout, 1, 3,
+                           p.d2.nout, 1, num_cu());
+    zch = (p.d2.nout + p.zchunk - 1) / p.zchunk;
+  }
+  sepq_pot<R><<<dim3((unsigned)(p.tiles_x * p.tiles_y), (unsigned)zch), PotGeo<R>::NT, 0, st>>>(p);
+  return hipGetLastError();
 }
 
 // ====================================================================== variants
@@ -772,15 +812,15 @@ hipError_t sep3d_variant(int v, const Box3& b, int narr, const R* x, R* y, R a, 
     LC_SEP2_VARIANTS(X)
 #undef X
 #define X(I, TX, TY, QX, QY, PD, WPE, ZC) \
-  case I: return launch_sepp<R, F, TX, TY, QX, QY, PD, WPE, ZC>(b, narr, x, y, a, a_y, st, pot, rho);
+  case I: return pot ? hipErrorInvalidValue : launch_sepp<R, F, TX, TY, QX, QY, PD, WPE, ZC>(b, narr, x, y, a, a_y, st);
     LC_SEPP_VARIANTS(X)
 #undef X
 #define X(I, TX, TY, QX, QY, PD, WPE, ZC) \
-  case I: return launch_sepr<R, F, TX, TY, QX, QY, PD, WPE, ZC>(b, narr, x, y, a, a_y, st, pot, rho);
+  case I: return pot ? hipErrorInvalidValue : launch_sepr<R, F, TX, TY, QX, QY, PD, WPE, ZC>(b, narr, x, y, a, a_y, st);
     LC_SEPR_VARIANTS(X)
 #undef X
 #define X(I, TX, TY, QX, QY, PD, WPE, ZC) \
-  case I: return launch_sepq<R, F, TX, TY, QX, QY, PD, WPE, ZC>(b, narr, x, y, a, a_y, st, pot, rho);
+  case I: return pot ? hipErrorInvalidValue : launch_sepq<R, F, TX, TY, QX, QY, PD, WPE, ZC>(b, narr, x, y, a, a_y, st);
     LC_SEPQ_VARIANTS(X)
 #undef X
   }

@@ -71,3 +71,26 @@ def test_default_chunks_equal_general_forms(lc, gpu, monkeypatch, prec, bc):
                     terms = float((x.double() * t.double()).abs().sum())
                     # FP32: the products are of values rounded to FP32 in both forms alike
                     assert abs(float(da[d] - db[d])) <= 2 * 4096 * 2.0 ** -53 * terms, (n, d)
+
+
+@pytest.mark.parametrize('prec', [8, 4])
+def test_potential_step_equals_general_form(lc, gpu, monkeypatch, prec):
+    torch = gpu
+    dt = torch.float64 if prec == 8 else torch.float32
+    rng = np.random.default_rng(5 + prec)
+    for n in [(1, 1, 1), (2, 9, 3), (18, 3, 20), (33, 20, 41)]:
+        m = int(np.prod([2 * v + 29 for v in n]))
+        dev = lambda k: torch.from_numpy(rng.uniform(-1, 1, k)).to('cuda', dt)
+        psi, pot, rho0 = dev(8 * int(np.prod(n))), dev(m), dev(m)
+        work = torch.empty(lc.local_hamiltonian_work(n), dtype=dt, device='cuda')
+        for with_rho in (True, False):
+            got = []
+            for v in (None, '12'):
+                monkeypatch.delenv('LIBCONV_SEP3D_VARIANT', raising=False)
+                if v:
+                    monkeypatch.setenv('LIBCONV_SEP3D_VARIANT', v)
+                rho, h = rho0.clone(), torch.full_like(psi, float('nan'))
+                lc.local_hamiltonian(n, [-0.5, -0.4, -0.3], psi, h, pot, rho if with_rho else None, work)
+                got.append((h, rho))
+            torch.cuda.synchronize()
+            assert torch.equal(got[0][0], got[1][0]) and torch.equal(got[0][1], got[1][1]), (n, with_rho)
