@@ -511,11 +511,15 @@ int run_1ds(int fil, int d, const int* n, const int* bc, const int* nx, const in
     }
     scratch = static_cast<double*>(sc);
     dot3 = reinterpret_cast<double*>(static_cast<char*>(sc) + sbytes);
+    // three energies go straight to the caller's device array (a copy is a
+    // launch of its own: 2 us and the gap before it); with fewer dims the
+    // kernel's three values do not fit there
+    if (d == 3 && dot_dev_user) dot3 = dot_dev_user;
   }
   hipError_t e = sum3d<R>(fil, b, narr, ax.dev, ay.dev, a3, (R)a_x, (R)a_y, want_dot ? dot3 : nullptr,
                           st, scratch, sbytes);
   if (e != hipSuccess) return hip_fail(e, who);
-  if (want_dot && dot_dev_user)
+  if (want_dot && dot_dev_user && dot3 != dot_dev_user)
     HIPCHK(hipMemcpyAsync(dot_dev_user, dot3, d * sizeof(double), hipMemcpyDeviceToDevice, st));
   if (!device_api) {
     if (ay.host_in) HIPCHK(hipMemcpyAsync(y, ay.dev, (size_t)tout * narr * sizeof(R), hipMemcpyDeviceToHost, st));
