@@ -86,7 +86,7 @@ struct SweepSrc {
 
 // Q consecutive outputs from the LDS values v(c, s), s = 0 .. Q + W - 2 (the
 // input steps of the first output's window onwards): every accumulator takes
-// its terms in the order of Op::compute.  xc[q]: the value at the output's own
+// its terms in the order of Op::step.  xc[q]: the value at the output's own
 // step (operators with the dot / a_x terms).
 template <typename R, class Op, int Q>
 struct SweepTask {

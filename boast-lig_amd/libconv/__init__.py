@@ -18,6 +18,7 @@ missing library raises at import.
 import ctypes
 import os
 import time
+from array import array
 
 import numpy as np
 
@@ -126,6 +127,27 @@ def _ints(v):
     return a
 
 
+def _iv(v):
+    """A dims argument as a C int array, for the calls on device tensors: the
+    smallest of them last a few microseconds on the GPU, and a numpy array and
+    its pointer cost one each.  Whatever array('i') does not take goes through
+    _ints, with its conversions and errors."""
+    if type(v) in (list, tuple) and v:
+        try:
+            return (_I * len(v)).from_buffer(array('i', v))
+        except (TypeError, OverflowError):
+            pass
+    a = _ints(v)
+    if a.size != len(a):
+        raise TypeError('dims: one integer per dimension')
+    return (_I * len(a))(*a.ravel().tolist())
+
+
+def _addr(t):
+    """Address of a checked tensor, for a void pointer argument."""
+    return None if t is None else t.data_ptr()
+
+
 def _ptr(a):
     """Address of a numpy array or a torch tensor (device or host)."""
     if a is None:
@@ -137,8 +159,21 @@ def _ptr(a):
     raise TypeError('array argument must be a numpy array or a torch tensor')
 
 
+_DTYPE_NAMES = {}  # torch dtype -> its name (str() of one builds the string each time)
+
+
+def _dtype_name(a):
+    dt = a.dtype
+    s = _DTYPE_NAMES.get(dt) if type(dt).__module__ == 'torch' else None
+    if s is None:
+        s = str(dt)
+        if type(dt).__module__ == 'torch':
+            _DTYPE_NAMES[dt] = s
+    return s
+
+
 def _is_f32(a):
-    if hasattr(a, 'dtype') and str(a.dtype) in ('float32', 'torch.float32'):
+    if hasattr(a, 'dtype') and _dtype_name(a) in ('float32', 'torch.float32'):
         return True
     return False
 
@@ -297,7 +332,7 @@ def _dev(t, name, prec, count, optional=False):
     if not (hasattr(t, 'data_ptr') and hasattr(t, 'is_cuda') and hasattr(t, 'numel')):
         raise TypeError('%s must be a torch tensor on the GPU' % name)
     want = 'torch.float64' if prec in (8, 'dot') else 'torch.float32'
-    if str(t.dtype) != want:
+    if _dtype_name(t) != want:
         raise LibconvError('%s: dtype %s, expected %s' % (name, t.dtype, want))
     if not t.is_contiguous():
         raise LibconvError('%s: not contiguous' % name)
@@ -328,52 +363,48 @@ def _rc(rc):
 
 def conv_1d(fil, idim, n, bc, nx, ny, narr, x, y, a=1.0, a_x=0.0, a_y=0.0, dot=None, stream=None):
     """Device-pointer sweep (lc_conv_1d); dot: a float64 device tensor or None."""
-    n_, nx_, ny_ = _ints(n), _ints(nx), _ints(ny)
+    n_, nx_, ny_ = _iv(n), _iv(nx), _iv(ny)
     pr = _prec(x)
     ei, eo = _ext1(n_, nx_, ny_, idim) if 0 <= idim < len(n_) else (nx_, ny_)
     _dev(x, 'x', pr, _count(ei) * narr)
     _dev(y, 'y', pr, _count(eo) * narr)
     _dev(dot, 'dot', 'dot', 1, optional=True)
     _resident(x=x, y=y, dot=dot)
-    _rc(lib().lc_conv_1d(_prec(x), fil, len(n_), idim, n_.ctypes.data_as(_IP), bc,
-                         nx_.ctypes.data_as(_IP), ny_.ctypes.data_as(_IP), narr, _ptr(x), _ptr(y),
-                         a, a_x, a_y, _ptr(dot), _stream(stream)))
+    _rc(lib().lc_conv_1d(pr, fil, len(n_), idim, n_, bc, nx_, ny_, narr, _addr(x), _addr(y), a, a_x, a_y,
+                         _addr(dot), _stream(stream)))
 
 
 def wavelet_1d(wav, inverse, idim, n, bc, nx, ny, narr, x, y, a=1.0, a_y=0.0, stream=None):
-    n_, nx_, ny_ = _ints(n), _ints(nx), _ints(ny)
+    n_, nx_, ny_ = _iv(n), _iv(nx), _iv(ny)
     pr = _prec(x)
     ei, eo = _ext1(n_, nx_, ny_, idim) if 0 <= idim < len(n_) else (nx_, ny_)
     _dev(x, 'x', pr, _count(ei, 2) * narr)
     _dev(y, 'y', pr, _count(eo, 2) * narr)
     _resident(x=x, y=y)
-    _rc(lib().lc_wavelet_1d(_prec(x), wav, int(bool(inverse)), len(n_), idim, n_.ctypes.data_as(_IP),
-                            bc, nx_.ctypes.data_as(_IP), ny_.ctypes.data_as(_IP), narr, _ptr(x),
-                            _ptr(y), a, a_y, _stream(stream)))
+    _rc(lib().lc_wavelet_1d(pr, wav, int(bool(inverse)), len(n_), idim, n_, bc, nx_, ny_, narr, _addr(x),
+                            _addr(y), a, a_y, _stream(stream)))
 
 
 def conv_md(fil, n, bc, nx, ny, narr, x, y, a=1.0, a_x=0.0, a_y=0.0, stream=None):
-    n_, b_, nx_, ny_ = _ints(n), _ints(bc), _ints(nx), _ints(ny)
+    n_, b_, nx_, ny_ = _iv(n), _iv(bc), _iv(nx), _iv(ny)
     pr = _prec(x)
     _dev(x, 'x', pr, _count(nx_) * narr)
     _dev(y, 'y', pr, _count(ny_) * narr)
     _resident(x=x, y=y)
-    _rc(lib().lc_conv_md(_prec(x), fil, len(n_), n_.ctypes.data_as(_IP), b_.ctypes.data_as(_IP),
-                         nx_.ctypes.data_as(_IP), ny_.ctypes.data_as(_IP), narr, _ptr(x), _ptr(y),
-                         a, a_x, a_y, _stream(stream)))
+    _rc(lib().lc_conv_md(pr, fil, len(n_), n_, b_, nx_, ny_, narr, _addr(x), _addr(y), a, a_x, a_y,
+                         _stream(stream)))
 
 
 def conv_1ds(fil, n, bc, nx, ny, narr, a, a_x, a_y, x, y, dot=None, stream=None):
-    n_, b_, nx_, ny_ = _ints(n), _ints(bc), _ints(nx), _ints(ny)
+    n_, b_, nx_, ny_ = _iv(n), _iv(bc), _iv(nx), _iv(ny)
     pr = _prec(x)
     _dev(x, 'x', pr, _count(nx_) * narr)
     _dev(y, 'y', pr, _count(ny_) * narr)
     _dev(dot, 'dot', 'dot', len(n_), optional=True)
     _resident(x=x, y=y, dot=dot)
     av = np.ascontiguousarray(np.asarray(a, dtype=np.float64))
-    _rc(lib().lc_conv_1ds(_prec(x), fil, len(n_), n_.ctypes.data_as(_IP), b_.ctypes.data_as(_IP),
-                          nx_.ctypes.data_as(_IP), ny_.ctypes.data_as(_IP), narr,
-                          av.ctypes.data_as(_DP), a_x, a_y, _ptr(x), _ptr(y), _ptr(dot),
+    _rc(lib().lc_conv_1ds(pr, fil, len(n_), n_, b_, nx_, ny_, narr,
+                          av.ctypes.data_as(_DP), a_x, a_y, _addr(x), _addr(y), _addr(dot),
                           _stream(stream)))
 
 
@@ -381,35 +412,33 @@ def conv_1ds_noalloc(fil, n, bc, nx, ny, narr, a, a_x, a_y, x, y, dot=None, stre
     """conv_1ds through lc_conv_1ds_noalloc: the energy partials use the
     library's static device buffer, no allocation (calls on one GPU must not
     overlap)."""
-    n_, b_, nx_, ny_ = _ints(n), _ints(bc), _ints(nx), _ints(ny)
+    n_, b_, nx_, ny_ = _iv(n), _iv(bc), _iv(nx), _iv(ny)
     av = np.ascontiguousarray(np.asarray(a, dtype=np.float64))
     pr = _prec(x)
     _dev(x, 'x', pr, _count(nx_) * narr)
     _dev(y, 'y', pr, _count(ny_) * narr)
     _dev(dot, 'dot', 'dot', len(n_), optional=True)
     _resident(x=x, y=y, dot=dot)
-    _rc(lib().lc_conv_1ds_noalloc(pr, fil, len(n_), n_.ctypes.data_as(_IP), b_.ctypes.data_as(_IP),
-                                  nx_.ctypes.data_as(_IP), ny_.ctypes.data_as(_IP), narr,
-                                  av.ctypes.data_as(_DP), a_x, a_y, _ptr(x), _ptr(y), _ptr(dot),
+    _rc(lib().lc_conv_1ds_noalloc(pr, fil, len(n_), n_, b_, nx_, ny_, narr,
+                                  av.ctypes.data_as(_DP), a_x, a_y, _addr(x), _addr(y), _addr(dot),
                                   _stream(stream)))
 
 
 def wavelet_md(wav, inverse, n, bc, nx, ny, narr, x, y, a=1.0, a_y=0.0, stream=None):
-    n_, b_, nx_, ny_ = _ints(n), _ints(bc), _ints(nx), _ints(ny)
+    n_, b_, nx_, ny_ = _iv(n), _iv(bc), _iv(nx), _iv(ny)
     pr = _prec(x)
     _dev(x, 'x', pr, _count(nx_, 2) * narr)
     _dev(y, 'y', pr, _count(ny_, 2) * narr)
     _resident(x=x, y=y)
-    _rc(lib().lc_wavelet_md(_prec(x), wav, int(bool(inverse)), len(n_), n_.ctypes.data_as(_IP),
-                            b_.ctypes.data_as(_IP), nx_.ctypes.data_as(_IP), ny_.ctypes.data_as(_IP),
-                            narr, _ptr(x), _ptr(y), a, a_y, _stream(stream)))
+    _rc(lib().lc_wavelet_md(pr, wav, int(bool(inverse)), len(n_), n_, b_, nx_, ny_, narr, _addr(x), _addr(y),
+                            a, a_y, _stream(stream)))
 
 
 def local_hamiltonian_work(n):
     """Elements of the work array lc_local_hamiltonian needs for n pairs per dim."""
     L = lib()
     L.lc_local_hamiltonian_work.restype = ctypes.c_long
-    w = L.lc_local_hamiltonian_work(_ints(n).ctypes.data_as(_IP))
+    w = L.lc_local_hamiltonian_work(_iv(n))
     check()
     return int(w)
 
@@ -417,7 +446,7 @@ def local_hamiltonian_work(n):
 def local_hamiltonian(n, a, psig, hpsig, pot, rho, work, ekin=None, stream=None):
     """lc_local_hamiltonian on device tensors (libconv.f90:238-295): hpsig =
     DWT o (IMF o pot o MF + sum_d a_d D2_d) o IDWT psig, rho += psir^2."""
-    n_ = _ints(n)
+    n_ = _iv(n)
     av = np.ascontiguousarray(np.asarray(a, dtype=np.float64))
     pr = _prec(psig)
     ng = _count([2 * v for v in n_])
@@ -429,7 +458,7 @@ def local_hamiltonian(n, a, psig, hpsig, pot, rho, work, ekin=None, stream=None)
     _dev(work, 'work', pr, local_hamiltonian_work(n_))
     _dev(ekin, 'ekin', 'dot', 3, optional=True)
     _resident(psig=psig, hpsig=hpsig, pot=pot, rho=rho, work=work, ekin=ekin)
-    _rc(lib().lc_local_hamiltonian(_prec(psig), n_.ctypes.data_as(_IP), av.ctypes.data_as(_DP), _ptr(psig),
+    _rc(lib().lc_local_hamiltonian(pr, n_, av.ctypes.data_as(_DP), _ptr(psig),
                                    _ptr(hpsig), _ptr(pot), _ptr(rho), _ptr(work), _ptr(ekin),
                                    _stream(stream)))
 
@@ -444,7 +473,7 @@ def poisson_1d(nord, idim, n, bc, u, du, a=1.0, a_y=0.0, stream=None):
     _dev(u, 'u', pr, _count(n))
     _dev(du, 'du', pr, _count(n))
     _resident(u=u, du=du)
-    _rc(lib().lc_poisson_1d(_prec(u), nord, idim, _ints(n).ctypes.data_as(_IP), bc, _ptr(u), _ptr(du),
+    _rc(lib().lc_poisson_1d(pr, nord, idim, _iv(n), bc, _ptr(u), _ptr(du),
                             _D(a), _D(a_y), _stream(stream)))
 
 
@@ -459,7 +488,7 @@ def div_u_i(geocode, n, u, du, nord, h, cc=None, stream=None):
     _dev(du, 'du', pr, _count(n))
     _dev(cc, 'cc', pr, _count(n), optional=True)
     _resident(u=u, du=du, cc=cc)
-    _rc(lib().lc_div_u_i(_prec(u), geocode, _ints(n).ctypes.data_as(_IP), _ptr(u), _ptr(du), nord,
+    _rc(lib().lc_div_u_i(pr, geocode, _iv(n), _ptr(u), _ptr(du), nord,
                          hv.ctypes.data_as(_DP), _ptr(cc), _stream(stream)))
 
 
@@ -469,7 +498,7 @@ def nabla_u(geocode, n, u, du, nord, h, stream=None):
     _dev(u, 'u', pr, _count(n))
     _dev(du, 'du', pr, 3 * _count(n))
     _resident(u=u, du=du)
-    _rc(lib().lc_nabla_u(_prec(u), geocode, _ints(n).ctypes.data_as(_IP), _ptr(u), _ptr(du), nord,
+    _rc(lib().lc_nabla_u(pr, geocode, _iv(n), _ptr(u), _ptr(du), nord,
                          hv.ctypes.data_as(_DP), _stream(stream)))
 
 
