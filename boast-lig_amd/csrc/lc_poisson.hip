@@ -428,9 +428,29 @@ __device__ __forceinline__ void pz_get(const R* base, long p, R* v, bool both) {
   }
 }
 
+// update_rhopol's other inputs at the points p and (both) p + 1, loaded before
+// the stencils (loads and a store per point after them are two chained round
+// trips: order 16 at 256^3 FP64 203 us, now 168)
+template <typename R>
+struct RhoIn {
+  R d[6], rho[2];
+  __device__ __forceinline__ void load(const GradEpi<R>& e, long p, bool both) {
+    pz_get(e.dlogeps, 3 * p, d, true);
+    if (both) {
+      pz_get(e.dlogeps, 3 * p + 2, d + 2, true);
+      pz_get(e.dlogeps, 3 * p + 4, d + 4, true);
+    } else {
+      d[2] = e.dlogeps[3 * p + 2];
+      d[3] = d[4] = d[5] = R(0);
+    }
+    pz_get(e.rhopol, p, rho, both);
+  }
+};
+
 // grad_epilogue for the points p and (both) p + 1
 template <typename R, int MODE>
-__device__ __forceinline__ double grad_epilogue2(const GradEpi<R>& e, long np, long p, bool both, R (*d)[2]) {
+__device__ __forceinline__ double grad_epilogue2(const GradEpi<R>& e, const RhoIn<R>& in, long np, long p, bool both,
+                                                 R (*d)[2]) {
   if constexpr (MODE == GE_GRAD || MODE == GE_SQUARE) {
     R q[2];
 #pragma unroll
@@ -453,8 +473,18 @@ __device__ __forceinline__ double grad_epilogue2(const GradEpi<R>& e, long np, l
     }
     return 0.0;
   } else {
-    double s = grad_epilogue<R, MODE>(e, np, p, d[0][0], d[1][0], d[2][0]);
-    if (both) s += grad_epilogue<R, MODE>(e, np, p + 1, d[0][1], d[1][1], d[2][1]);
+    const R oneo4pi = (R)0.07957747154594766788444188168625718101722982287022822437383367203;  // 1 / (4 pi)
+    R o[2];
+    double s = 0.0;
+#pragma unroll
+    for (int k = 0; k < 2; ++k) {
+      R res = (in.d[3 * k] * d[0][k] + in.d[3 * k + 1] * d[1][k]) + in.d[3 * k + 2] * d[2][k];
+      res = res * oneo4pi;
+      res = (res - in.rho[k]) * e.eta;
+      o[k] = res + in.rho[k];
+      if (k == 0 || both) s += (double)(res * res);
+    }
+    pz_put(e.rhopol, p, o, both);
     return s;
   }
 }
@@ -629,12 +659,14 @@ __attribute__((amdgpu_waves_per_eu(pz_waves<R, NORD>()))) void poisson_zm_kernel
       dzv[1] *= rh2;
       fence();
       if constexpr (MODE >= GE_GRAD) {
+        RhoIn<R> in;
+        if constexpr (MODE == GE_RHOPOL) in.load(ep, p, both);
         R d[3][2];
         sx(lds, d[0]);
         sy(lds, d[1]);
         d[2][0] = dzv[0];
         d[2][1] = dzv[1];
-        sq += grad_epilogue2<R, MODE>(ep, g.np, p, both, d);
+        sq += grad_epilogue2<R, MODE>(ep, in, g.np, p, both, d);
       } else {
         R dx[2], dy[2], o[2];
         sx(lds, dx);
@@ -797,10 +829,11 @@ static bool pz_launch(const PGeom& g, int ty, int resident, PzLaunch& L) {
 }
 // tile rows: 16; 32 for the gradient operators of order 16, whose y halo is as
 // high as the tile (nabla_u_and_square at 256^3: FP64 151 us against 179, FP32
-// 68 against 93), where that still gives a CU two chunks of 16 planes.
+// 68 against 93), where that still gives a CU two chunks of 16 planes.  In FP64
+// the others' tall tiles are no faster (nabla_u_square 106 against 100 us).
 // div_u_i holds three tiles and gains nothing (FP64 257 against 240 us).
-template <int NO, int MODE>
-static constexpr bool pz_tall() { return NO == 16 && MODE >= GE_GRAD; }
+template <typename R, int NO, int MODE>
+static constexpr bool pz_tall() { return NO == 16 && (MODE == GE_GRAD || (sizeof(R) == 4 && MODE > GE_GRAD)); }
 static bool pz_fills(const PGeom& g) {
   const long tiles = (long)((g.n0 + kZTX - 1) / kZTX) * ((g.n1 + 31) / 32);
   return tiles * (g.n2 / 16) >= 2L * num_cu();
@@ -818,6 +851,21 @@ static int pz_resident() {
   return nb;
 }
 
+// Blocks per CU on arrays beyond the last-level cache, orders below 16 (order 16
+// has the registers or the work to be indifferent): longer chunks re-read
+// fewer window planes from memory.  256^3, all blocks that fit against this
+// many: FP64 order 4 div_u_i 112 -> 105 us, nabla_u 128 -> 122, with square 155
+// -> 149; FP32 order 8 nabla_u 59 -> 47, div_u_i 55 -> 46.  The operators that
+// gain nothing keep all (div_u_i with cc, three inputs in LDS: FP64 order 8 on
+// 200 x 150 x 180 59 us against 72; in FP32 those of four outputs or one).
+constexpr double kPzCached = 128e6;  // bytes of four arrays: half the cache
+template <typename R, int MODE>
+static int pz_stream_blocks(const GradEpi<R>& ep) {
+  if (MODE == 1) return 8;  // div_u_i with cc
+  if (sizeof(R) == 8) return MODE == GE_SQUARE ? 3 : 2;
+  return MODE == GE_SQUARE || MODE == GE_EPS || ep.du2 ? 8 : 3;
+}
+
 // one z-march launch; its blocks, or 0 when the one-point kernels must run;
 // dry: count only
 template <typename R, int NO, int MODE, int TY>
@@ -825,7 +873,9 @@ static long pz_run_rows(const PGeom& g, const R* u, R* o0, R* o1, const GradEpi<
                         hipStream_t st, bool dry) {
   constexpr int NT = PzGeo<R, NO, TY>::NT;
   PzLaunch L;
-  if (!pz_launch(g, TY, pz_resident<poisson_zm_kernel<R, NO, MODE, TY>, NT>(), L)) return 0;
+  int resident = pz_resident<poisson_zm_kernel<R, NO, MODE, TY>, NT>();
+  if (NO < 16 && 4.0 * sizeof(R) * g.np > kPzCached) resident = std::min(resident, pz_stream_blocks<R, MODE>(ep));
+  if (!pz_launch(g, TY, resident, L)) return 0;
   if (!dry)
     poisson_zm_kernel<R, NO, MODE, TY><<<L.blocks, NT, 0, st>>>(g, L.tiles_x, L.tiles, L.zchunk, u, o0, o1, ep, r0,
                                                                 r1, r2);
@@ -834,7 +884,7 @@ static long pz_run_rows(const PGeom& g, const R* u, R* o0, R* o1, const GradEpi<
 template <typename R, int NO, int MODE>
 static long pz_run(const PGeom& g, const R* u, R* o0, R* o1, const GradEpi<R>& ep, R r0, R r1, R r2, hipStream_t st,
                    bool dry) {
-  if constexpr (pz_tall<NO, MODE>()) {
+  if constexpr (pz_tall<R, NO, MODE>()) {
     if (pz_fills(g)) return pz_run_rows<R, NO, MODE, 32>(g, u, o0, o1, ep, r0, r1, r2, st, dry);
   }
   return pz_run_rows<R, NO, MODE, 16>(g, u, o0, o1, ep, r0, r1, r2, st, dry);
