@@ -7,8 +7,9 @@
 //   out[i][c'] = sum_{s<W} sum_{c<2} C[c'][c](s) * in[i + LO + s][c],
 // the split filters of WaveletFilterDecompose / WaveletFilterRecompose
 // (BigDFT/GenericConvolution2.rb:386-410, :453-462, :505-671).  The three
-// per-dim sweeps of the libconv composition (:2160-2240) become one pass:
-// per input z-step the two z-planes of the (TX+W-1) x (TY+W-1)-step tile go
+// per-dim sweeps of the libconv composition (:2160-2240) become one pass, in
+// two forms of equal bits: the pair-wise one (lc_body_wavq.hpp), and the
+// step-at-a-time one, which takes planes beyond 32-bit buffer records: per input z-step the two z-planes of the (TX+W-1) x (TY+W-1)-step tile go
 // to LDS, x-tasks filter rows into LDS, every lane filters one column along
 // y for both bands and feeds its register window along z, which emits both
 // z bands of the output step.  Data layout per dim (storage extents 2 nx and
@@ -117,7 +118,7 @@ static bool wavq_block(int v, WavqBlock* b) {
   return false;
 }
 
-// output planes reached through 32-bit buffer records (the plane-at-a-time
+// output planes reached through 32-bit buffer records (the pair-wise
 // variants store with buffer stores)
 static bool wavq_fits(const Box3& b, int prec) {
   return wav_plane_fits(b, prec) && 4L * b.ny[0] * b.ny[1] * prec <= kPlaneMax;
