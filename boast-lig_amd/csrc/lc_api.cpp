@@ -1171,8 +1171,9 @@ Box3 item_box(const lc_batch_item& u) {
   return b;
 }
 
-// variant of a new stage: the tuned one for its largest item's shape when it
-// has a batched form, else the default
+// variant of a new stage: the chosen one (tuned, or named by the environment)
+// for its largest item's shape, else the default, which for wavelets looks at
+// all items; when that has no batched form, the fastest that has one
 int stage_default_variant(const lc_batch_item* it, int count, int prec) {
   int big = 0;
   long most = -1;
@@ -1181,11 +1182,14 @@ int stage_default_variant(const lc_batch_item* it, int count, int prec) {
     if (p > most) { most = p; big = i; }
   }
   const int form = item_form(it[big]);
-  int v = select_variant(prec, form, it[big].op, item_box(it[big]));
-  if (form == FORM_DWT || form == FORM_IDWT) {
-    std::vector<Box3> boxes;
-    for (int i = 0; i < count; ++i) boxes.push_back(item_box(it[i]));
-    v = wav_batch_variant(prec, v, boxes.data(), count);
+  int v = chosen_variant(prec, form, it[big].op, item_box(it[big]));
+  if (v < 0) {
+    v = default_variant(prec, form, item_box(it[big]));
+    if (form == FORM_DWT || form == FORM_IDWT) {
+      std::vector<Box3> boxes;
+      for (int i = 0; i < count; ++i) boxes.push_back(item_box(it[i]));
+      v = wav_batch_variant(prec, v, boxes.data(), count);
+    }
   }
   if (has_batch_form(form, v)) return v;
   bool fit = true;

@@ -194,12 +194,8 @@ static int env_variant(const char* name, int nvar) {
   return v >= 0 && v < nvar ? v : -1;
 }
 
-int select_variant(int prec, int form, int id, const Box3& b) {
-  int v = tuned_variant(prec, form, id, b);
-  if (v >= 0) return v;
+int default_variant(int prec, int form, const Box3& b) {
   if (form == FORM_SUM || form == FORM_SEP) {
-    v = env_variant(form == FORM_SUM ? "LIBCONV_SUM3D_VARIANT" : "LIBCONV_SEP3D_VARIANT", variant_count(form));
-    if (v >= 0) return v;
     // defaults: the fastest variants on MI355X (MF in FP64: the 128-bit-LDS
     // kernel on 32 x 16 tiles, 4-10% ahead of the others from the 128^3
     // chain and the 157^3 magic filter of the local Hamiltonian at 64^3 pairs
@@ -227,13 +223,24 @@ int select_variant(int prec, int form, int id, const Box3& b) {
     const long kplane = (long)(b.bc[0] == GROW ? b.n[0] + gk : b.n[0]) * (b.bc[1] == GROW ? b.n[1] + gk : b.n[1]);
     return kplane >= 150L * 150 ? 31 : 32;
   }
-  v = env_variant("LIBCONV_WAV3D_VARIANT", wav_variant_count());
-  if (v >= 0) return v;
   // the pair-wise kernel (its outputs go through 32-bit buffer records): the
   // block that the model in lc_fused_wav.hip expects to be fastest on this
   // grid; else one z-step per slide
   if (wav_plane_fits(b, prec) && 4L * b.ny[0] * b.ny[1] * prec <= kPlaneMax) return wav_default_variant(prec, form, b);
   return 5;
+}
+
+int chosen_variant(int prec, int form, int id, const Box3& b) {
+  const int v = tuned_variant(prec, form, id, b);
+  if (v >= 0) return v;
+  return env_variant(form == FORM_SUM ? "LIBCONV_SUM3D_VARIANT" : form == FORM_SEP ? "LIBCONV_SEP3D_VARIANT"
+                                                                                   : "LIBCONV_WAV3D_VARIANT",
+                     variant_count(form));
+}
+
+int select_variant(int prec, int form, int id, const Box3& b) {
+  const int v = chosen_variant(prec, form, id, b);
+  return v >= 0 ? v : default_variant(prec, form, b);
 }
 
 template <typename R>

@@ -317,13 +317,13 @@ int wav_default_variant(int prec, int form, const Box3& b) {
   return best;
 }
 
-// The variant of a batch stage whose largest item would take `single` by
-// itself: a stage that fills every CU is bound by bytes, so it takes the block
+// The default of a batch stage whose largest item by itself would take `single`
+// by default: a stage that fills every CU is bound by bytes, so it takes the block
 // with the widest tiles, in FP64 512 output steps, in FP32 (more blocks per
 // CU) 256.  128 orbitals of 24..96 pairs, DWT stage: FP64 1.55 / 1.34 / 1.25
 // ms for 128 / 256 / 512 steps, FP32 0.90 / 0.78 / 0.83.
 int wav_batch_variant(int prec, int single, const Box3* b, int count) {
-  if (single < 7) return single;  // a tuned or environment choice of the step-at-a-time form
+  if (single < 7) return single;  // the step-at-a-time form: planes beyond the buffer records
   long steps = 0;
   for (int i = 0; i < count; ++i) {
     if (!wavq_fits(b[i], prec)) return single;
