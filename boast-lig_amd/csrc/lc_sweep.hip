@@ -4,7 +4,7 @@
 // synthesis) along one dimension of an array seen as (L, line, R) with L
 // the product of the faster dims and R the product of the slower dims
 // (the libconv 1D dispatcher's ndat_left / ndat_right,
-// BigDFT/GenericConvolution2.rb:1701-1766).  Two kernels, one plan: a block
+// BigDFT/GenericConvolution2.rb:1701-1766).  Two tiled kernels: a block
 // stages a tile of lines -- every line's input steps for a chunk of outputs,
 // halo included -- in LDS with all of its loads in flight at once, and every
 // lane then computes Q consecutive outputs of one line, each LDS value feeding
@@ -19,14 +19,24 @@
 //                  the outputs go back through the LDS to be stored along the
 //                  lines.
 //
+// And two without a tile of fixed size, for lines that would leave most of one
+// empty (ring_pays, seg_pays):
+//
+//   sweep_ring     L > 1: one lane per column, which walks a chunk of the line
+//                  with a register ring of W input steps;
+//   sweep_seg      L == 1: 4 to 64 lanes share a segment of one line.
+//
+// All sum in the same order, so an output's bits do not depend on the form.
+//
 // What bounds them: latency.  A sweep moves two values per output and the
 // arrays of one orbital are 2..130 MB, so a launch lasts a few memory round
-// trips; what counts is how many loads are in flight (here a block's whole
-// tile, 12..20 loads per lane) and that every CU has its blocks in the first
-// wave.  The form before this kept one load per lane in flight per step (a
-// register ring along the line): 27 us for a 128^3 FP64 second-derivative
-// sweep with its energy along a strided dim, 19 us along the contiguous one
-// (bank conflicts on a third of its LDS cycles).
+// trips; what counts is how many loads are in flight (a block's whole tile: 4
+// loads per lane for the magic filter with Q = 2, 20 for the second derivative
+// with Q = 16) and that every CU has its blocks in the first wave.  The ring
+// keeps one load per lane in flight per step: 27 us for a 128^3 FP64
+// second-derivative sweep with its energy along a strided dim, 12 with tiles;
+// the segments' LDS has bank conflicts on a third of its cycles: 19 us along
+// the contiguous dim, 13 with tiles.
 //
 // Epilogue per output (ConvolutionFilter#post_process_and_store_values,
 // GenericConvolution2.rb:173-203): t *= a; dot += x_i t; t += a_x x_i;
@@ -84,6 +94,34 @@ struct SweepSrc {
   }
 };
 
+// one input value of a line (the forms without a tile)
+template <int K, int BC, typename R>
+__device__ __forceinline__ R load_step(const R* __restrict__ xb, long L, int j, int c, int n, int nx, int ox) {
+  if (BC == PER) return xb[in_elem<K>(pmod(j, n), c, nx) * L];
+  if (BC == GROW) {
+    const bool ok = (j >= 0) & (j < n);
+    const R v = xb[in_elem<K>(ok ? j : 0, c, nx) * L];
+    return ok ? v : R(0);
+  }
+  return xb[in_elem<K>(j - ox, c, nx) * L];
+}
+
+// the epilogue of output step i up to the a_y term; xc: x at step i
+template <class Op, int BC, typename R>
+__device__ __forceinline__ void sweep_post(const SweepArgs<R>& p, int i, R xc, bool want_dot, double& dot, R* o) {
+  if (p.flags & F_A) {
+#pragma unroll
+    for (int c = 0; c < Op::OUT; ++c) o[c] = o[c] * p.a;
+  }
+  if (Op::DOT) {
+    const bool has_x = BC != GROW || (i >= 0 && i < p.n);
+    if (has_x) {
+      if (want_dot) dot = fmar((double)xc, (double)o[0], dot);
+      if (p.flags & F_AX) o[0] = fmar(xc, p.a_x, o[0]);
+    }
+  }
+}
+
 // Q consecutive outputs from the LDS values v(c, s), s = 0 .. Q + W - 2 (the
 // input steps of the first output's window onwards): every accumulator takes
 // its terms in the order of Op::step.  xc[q]: the value at the output's own
@@ -112,21 +150,6 @@ struct SweepTask {
           Op::step(s, w, o[q]);
           if (Op::DOT && s == -Op::LO) xc[q] = w[0];
         }
-      }
-    }
-  }
-  // the epilogue up to the a_y term of output step i = i0 + q
-  template <int BC>
-  __device__ __forceinline__ void finish(const SweepArgs<R>& p, int q, int i, bool want_dot, double& dot) {
-    if (p.flags & F_A) {
-#pragma unroll
-      for (int c = 0; c < Op::OUT; ++c) o[q][c] = o[q][c] * p.a;
-    }
-    if (Op::DOT) {
-      const bool has_x = BC != GROW || (i >= 0 && i < p.n);
-      if (has_x) {
-        if (want_dot) dot = fmar((double)xc[q], (double)o[q][0], dot);
-        if (p.flags & F_AX) o[q][0] = fmar(xc[q], p.a_x, o[q][0]);
       }
     }
   }
@@ -199,7 +222,7 @@ __global__ __launch_bounds__(256) void sweep_strided(SweepArgs<R> p) {
     for (int q = 0; q < Q; ++q) {
       const int i = ib + q;
       if (i < i1) {
-        t.template finish<BC>(p, q, i, want_dot, dot);
+        sweep_post<Op, BC>(p, i, t.xc[q], want_dot, dot, t.o[q]);
 #pragma unroll
         for (int c = 0; c < Op::OUT; ++c) {
           R o = t.o[q][c];
@@ -266,7 +289,7 @@ __global__ __launch_bounds__(256) void sweep_contig(SweepArgs<R> p) {
     const bool want_dot = Op::DOT && (p.flags & F_DOT) && line < p.ncols && line >= (p.narr - 1) * p.nr;
 #pragma unroll
     for (int q = 0; q < Q; ++q)
-      if (ib + q < i1) t.template finish<BC>(p, q, ib + q, want_dot, dot);
+      if (ib + q < i1) sweep_post<Op, BC>(p, ib + q, t.xc[q], want_dot, dot, t.o[q]);
   }
   __syncthreads();
   // outputs back through the tile, in memory order along the line
@@ -291,6 +314,116 @@ __global__ __launch_bounds__(256) void sweep_contig(SweepArgs<R> p) {
         R o = tile[(ly + 4 * b) * G::ROW + e];
         if (p.flags & F_AY) o = fmar(p.a_y, *yp, o);
         *yp = o;
+      }
+    }
+  }
+  if (p.dot_part) {
+    const double s = block_sum<R>(dot, red);
+    if (threadIdx.x == 0) p.dot_part[blockIdx.x] = s;
+  }
+}
+
+// ------------------------------------------------- strided, a column per lane
+template <typename R, class Op, int BC>
+__global__ __launch_bounds__(256) void sweep_ring(SweepArgs<R> p) {
+  constexpr int K = KindOf<Op>::v;
+  constexpr int W = Op::W, IN = Op::IN, OUT = Op::OUT;
+  __shared__ double red[4];
+  const long col = (long)(blockIdx.x % (unsigned)p.cblocks) * 256 + threadIdx.x;
+  double dot = 0.0;
+  if (col < p.ncols) {
+    const long line = p.ncols <= 0x7fffffffL ? (int)col / (int)p.L : col / p.L, l = col - line * p.L;
+    const R* __restrict__ xb = p.x + line * p.line_in + l;
+    R* __restrict__ yb = p.y + line * p.line_out + l;
+    const bool want_dot = Op::DOT && (p.flags & F_DOT) && line >= (p.narr - 1) * p.nr;
+    const int i0 = p.i_first + (int)(blockIdx.x / (unsigned)p.cblocks) * p.chunk;
+    const int i1 = min(i0 + p.chunk, p.i_first + p.nout);
+    R win[W][IN];  // step j is in slot (j - (i0 + LO)) mod W
+    int jp = BC == PER ? pmod(i0 + Op::LO, p.n) : 0;
+    auto load = [&](R* w, int j) {
+#pragma unroll
+      for (int c = 0; c < IN; ++c)
+        w[c] = BC == PER ? xb[in_elem<K>(jp, c, p.nx) * p.L] : load_step<K, BC>(xb, p.L, j, c, p.n, p.nx, p.ox);
+      if (BC == PER) jp = jp + 1 == p.n ? 0 : jp + 1;
+    };
+#pragma unroll
+    for (int s = 0; s < W - 1; ++s) load(win[s], i0 + Op::LO + s);
+    for (int base = i0; base < i1; base += W) {
+#pragma unroll
+      for (int u = 0; u < W; ++u) {
+        const int i = base + u;
+        if (i < i1) {
+          load(win[(u + W - 1) % W], i + Op::UP);
+          R o[OUT];
+#pragma unroll
+          for (int c = 0; c < OUT; ++c) o[c] = R(0);
+#pragma unroll
+          for (int s = 0; s < W; ++s) Op::step(s, win[(u + s) % W], o);
+          sweep_post<Op, BC>(p, i, win[(u - Op::LO) % W][0], want_dot, dot, o);
+#pragma unroll
+          for (int c = 0; c < OUT; ++c) {
+            R* yp = yb + out_elem<K>(i - p.oy, c, p.ny) * p.L;
+            if (p.flags & F_AY) o[c] = fmar(p.a_y, *yp, o[c]);
+            *yp = o[c];
+          }
+        }
+      }
+    }
+  }
+  if (p.dot_part) {
+    const double s = block_sum<R>(dot, red);
+    if (threadIdx.x == 0) p.dot_part[blockIdx.x] = s;
+  }
+}
+
+// ------------------------------------------------- contiguous, a segment per group
+// 2^lg lanes of Q outputs share a line's segment: 256 >> lg lines per block,
+// the input steps of each in LDS, one run per component.
+constexpr int kSegQ = 4;
+template <typename R, class Op, int BC>
+__global__ __launch_bounds__(256) void sweep_seg(SweepArgs<R> p, int lg) {
+  constexpr int K = KindOf<Op>::v, Q = kSegQ;
+  constexpr int W = Op::W, IN = Op::IN, OUT = Op::OUT;
+  extern __shared__ __align__(16) unsigned char smem_raw[];
+  R* sm = reinterpret_cast<R*>(smem_raw);
+  __shared__ double red[4];
+  const int TPL = 1 << lg, LPB = 256 >> lg, NS = p.chunk + W - 1;  // chunk = TPL Q
+  const int tl = threadIdx.x & (TPL - 1), lnb = threadIdx.x >> lg;
+  const long line = (long)(blockIdx.x % (unsigned)p.cblocks) * LPB + lnb;
+  const bool active = line < p.ncols;
+  const int i0 = p.i_first + (int)(blockIdx.x / (unsigned)p.cblocks) * p.chunk;
+  const int iend = p.i_first + p.nout;
+  const R* __restrict__ xb = p.x + (active ? line * p.line_in : 0);
+  R* __restrict__ yb = p.y + (active ? line * p.line_out : 0);
+  if (active) {
+    // steps beyond iend - 1 + UP are never used and may lie outside x (shrink)
+    const int jmax = iend - 1 + Op::UP;
+    for (int e = tl; e < NS * IN; e += TPL) {  // memory order: pairs (DWT), bands (IDWT)
+      const int c = K == KDWT ? e & 1 : K == KIDWT ? e / NS : 0, s = K == KDWT ? e >> 1 : e - c * NS;
+      const int j = i0 + Op::LO + s;
+      sm[(c * LPB + lnb) * NS + s] = j <= jmax ? load_step<K, BC>(xb, 1, j, c, p.n, p.nx, p.ox) : R(0);
+    }
+  }
+  __syncthreads();
+  double dot = 0.0;
+  if (active) {
+    const bool want_dot = Op::DOT && (p.flags & F_DOT) && line >= (p.narr - 1) * p.nr;
+    const int ib = i0 + tl * Q;
+    SweepTask<R, Op, Q> t;
+    const R* base = sm + lnb * NS + tl * Q;
+    t.run([&](int c, int k) { return base[c * LPB * NS + k]; });
+#pragma unroll
+    for (int q = 0; q < Q; ++q) {
+      const int i = ib + q;
+      if (i < iend) {
+        sweep_post<Op, BC>(p, i, t.xc[q], want_dot, dot, t.o[q]);
+#pragma unroll
+        for (int c = 0; c < OUT; ++c) {
+          R* yp = yb + out_elem<K>(i - p.oy, c, p.ny);
+          R o = t.o[q][c];
+          if (p.flags & F_AY) o = fmar(p.a_y, *yp, o);
+          *yp = o;
+        }
       }
     }
   }
@@ -348,24 +481,93 @@ __global__ __launch_bounds__(kPartThreads) void sum_partials(const double* __res
 }
 
 // ---------------------------------------------------------------- launcher
-// Launch shape: the largest chunk (outputs per lane Q in 2, 4, 8, 16) whose
-// blocks still number four per CU -- halo rows cost reads, few blocks leave
-// CUs idle in a launch that lasts one round of blocks -- and chunks of equal
-// length.  The wavelets' tiles are twice as deep per output step: Q up to 8
-// (sym8) and 4 (windows of 16 pairs).
+// Which form.  The tiles hold 32 columns and at least 16 outputs of each and
+// are latency-lean; the forms without a tile need no column or output that is
+// not there.  They win where the tile would be mostly padding -- a few outputs
+// per line, or a few long lines -- once there are enough lines to fill the chip
+// by themselves, and for the wavelets, whose tile re-reads W - 1 pairs per
+// chunk, on ranges of longer lines too (up to 1.3 times as fast; over the rest
+// of those ranges the tiles are).  The bounds are where the two measured
+// times cross (periodic sweeps, device time, the tile's best chunk): second
+// derivative FP64, strided, 131072 columns: 6 outputs 7.0 us without a tile
+// against 11.0 with one, 16 outputs 11.5 against 13.2, 32 outputs 19 against
+// 15; a contiguous line of 2^20 points 11.4 against 57; symicomb8 FP64 along
+// the second of 100^3 pairs 27 against 37; sym8 FP64 on 32768 columns of 8
+// pairs 5.6 against 5.4, of 80 pairs 17 against 20.8.  All calls tried (1100
+// boxes and the grid of 1 .. 2^21 lines by 1 .. 2^20 outputs) are within 15% of
+// the faster form, 1% on average.
+static bool ring_pays(long ncols, long L, int nout, int in, int W, int rs) {
+  const double total = (double)ncols * nout;
+  if (in == 1)
+    return (ncols >= 49152 && nout <= (rs == 8 ? (W > 16 ? 16 : 12) : (W > 16 ? 24 : 16))) ||
+           (ncols >= 32768 && nout <= 4);
+  // a tile's rows straddle the lines' ends: more of them are split
+  const bool ragged = L % kSweepCols != 0 && nout >= 64 && nout <= 160;
+  if (W <= 8) {
+    if (ragged && ncols >= 16384 && total >= 1.2e6) return true;
+    if (rs == 8)
+      return (ncols >= 32768 && nout <= 12) || (ncols >= 24576 && nout <= 2) ||
+             (ncols >= 24576 && nout >= 40 && nout <= 160 && total >= 1.9e6);
+    return (ncols >= 49152 && nout <= 40) || (ncols >= 16384 && nout <= 4) ||
+           (ncols >= 2048 && nout >= 40 && total >= 1.2e6 && total <= 2.7e6);
+  }
+  if (rs == 8)
+    return (ncols >= 65536 && nout <= 160) || (ncols >= 49152 && nout <= 20) || (ncols >= 32768 && nout <= 4) ||
+           (ncols >= 64 && total >= 3e6 && total <= 8.5e6) || (ragged && ncols >= 16384 && total >= 2e6);
+  return (ncols >= 24576 && nout <= 6) || (ncols >= 49152 && nout <= 12) || (ncols >= 65536 && nout <= 28) ||
+         (ncols >= 131072 && nout <= 160) || (ncols >= 98304 && nout >= 64 && nout <= 160) ||
+         (ncols >= 24576 && nout >= 80 && nout <= 160 && total >= (ragged ? 3.6e6 : 5e6));
+}
+static bool seg_pays(long ncols, int nout, int in, int W, int rs) {
+  if ((ncols <= 4 && nout >= 60000) || (ncols <= 8 && nout >= 500000)) return true;
+  if (in == 1) return ncols >= 24576 && nout <= 12;
+  if (W <= 8) return (ncols >= 16384 && nout <= 2) || (ncols >= 262144 && nout <= 4);
+  return ncols >= 24576 && nout <= (rs == 8 ? 4 : 6);
+}
+
+// Launch shape.  Tiles: the largest chunk (outputs per lane Q in 2, 4, 8, 16)
+// whose blocks still number four per CU -- halo rows cost reads, few blocks
+// leave CUs idle in a launch that lasts one round of blocks --, not more than
+// twice the line (32 outputs of 65536 FP64 magic-filter columns: 15 us with
+// chunks for 128, 9 with chunks for 32), and chunks of equal length.  The
+// wavelets' tiles are twice as deep per output step: Q up to 8 (sym8) and 4
+// (windows of 16 pairs).  Ring: chunks of two windows and more, until eight
+// waves per CU.  Segments: the lanes that a line's outputs fill, 4 to 64.
+enum SweepForm { SWEEP_TILE, SWEEP_RING, SWEEP_SEG };
 struct SweepPlan {
-  int q, chunk;
+  SweepForm form;
+  int q, lg;  // outputs per lane of a tile; lanes per segment (log2)
+  int chunk;
   long cblocks, blocks;
 };
 template <typename R>
 static SweepPlan sweep_plan(const SweepArgs<R>& p, int in, int W) {
   constexpr int C = kSweepCols, G = 256 / C;
-  SweepPlan s;
-  s.cblocks = (p.ncols + C - 1) / C;
-  s.q = in == 1 ? 16 : W > 8 ? 4 : 8;
-  while (s.q > 2 && s.cblocks * ((p.nout + G * s.q - 1) / (G * s.q)) < 4L * num_cu()) s.q /= 2;
-  const int n = (p.nout + G * s.q - 1) / (G * s.q);
-  s.chunk = (p.nout + n - 1) / n;
+  SweepPlan s{};
+  int n;
+  if (p.L == 1 && seg_pays(p.ncols, p.nout, in, W, sizeof(R))) {
+    s.form = SWEEP_SEG;
+    s.lg = 2;
+    while (s.lg < 6 && (kSegQ << s.lg) < p.nout) ++s.lg;
+    s.chunk = kSegQ << s.lg;
+    s.cblocks = (p.ncols + (256 >> s.lg) - 1) / (256 >> s.lg);
+    n = (p.nout + s.chunk - 1) / s.chunk;
+  } else if (p.L > 1 && ring_pays(p.ncols, p.L, p.nout, in, W, sizeof(R))) {
+    s.form = SWEEP_RING;
+    const long waves = (p.ncols + 63) / 64;
+    n = (int)std::max(1L, std::min<long>((8L * num_cu() + waves - 1) / waves, p.nout / (2 * W)));
+    s.chunk = (p.nout + n - 1) / n;
+    s.cblocks = (p.ncols + 255) / 256;
+    n = (p.nout + s.chunk - 1) / s.chunk;
+  } else {
+    s.form = SWEEP_TILE;
+    s.cblocks = (p.ncols + C - 1) / C;
+    s.q = in == 1 ? 16 : W > 8 ? 4 : 8;
+    while (s.q > 2 && (s.cblocks * ((p.nout + G * s.q - 1) / (G * s.q)) < 4L * num_cu() || p.nout <= G * s.q / 2))
+      s.q /= 2;
+    n = (p.nout + G * s.q - 1) / (G * s.q);
+    s.chunk = (p.nout + n - 1) / n;
+  }
   s.blocks = s.cblocks * n;
   return s;
 }
@@ -381,6 +583,12 @@ static hipError_t run_sweep(const SweepArgs<R>& a0, hipStream_t st, double* dot_
   if (s.blocks > 0x7fffffffL) return hipErrorInvalidValue;
   p.chunk = s.chunk;
   p.cblocks = (int)s.cblocks;
+  if (s.form == SWEEP_RING) {
+    sweep_ring<R, Op, BC><<<(unsigned)s.blocks, 256, 0, st>>>(p);
+  } else if (s.form == SWEEP_SEG) {
+    const size_t lds = (size_t)(256 >> s.lg) * (s.chunk + Op::W - 1) * Op::IN * sizeof(R);
+    sweep_seg<R, Op, BC><<<(unsigned)s.blocks, 256, lds, st>>>(p, s.lg);
+  }
   auto launch = [&](auto q) {
     constexpr int Q = decltype(q)::value;
     if (p.L == 1)
