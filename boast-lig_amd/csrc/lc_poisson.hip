@@ -490,12 +490,12 @@ __device__ __forceinline__ double grad_epilogue2(const GradEpi<R>& e, const RhoI
 }
 
 // waves per SIMD asked of the compiler
-template <typename R, int NORD>
-constexpr int pz_waves() { return sizeof(R) == 8 && NORD == 16 ? 2 : 4; }
+template <typename R, int NORD, int MODE>
+constexpr int pz_waves() { return sizeof(R) == 8 && NORD == 16 ? (MODE == GE_SQUARE || MODE == GE_EPS ? 3 : 2) : 4; }
 
 template <typename R, int NORD, int MODE, int TY>
 __global__ __launch_bounds__((PzGeo<R, NORD, TY>::NT))
-__attribute__((amdgpu_waves_per_eu(pz_waves<R, NORD>()))) void poisson_zm_kernel(
+__attribute__((amdgpu_waves_per_eu(pz_waves<R, NORD, MODE>()))) void poisson_zm_kernel(
     PGeom g, int tiles_x, int tiles, int zchunk, const R* __restrict__ u, R* __restrict__ o0, R* __restrict__ o1,
     GradEpi<R> ep, R rh0, R rh1, R rh2) {
   using G = PzGeo<R, NORD, TY>;
@@ -801,26 +801,58 @@ hipError_t poisson_1d(int nord, int idim, const int* n, int bc, const R* u, R* d
   return hipGetLastError();
 }
 
-// z-march launch shape: tiles x z chunks.  The chunks put at most `resident`
-// blocks (what one CU holds of the kernel) on any CU, so the grid runs in one
-// even round; a chunk repeats only the 2m column loads of its window, so
-// chunks go down to 6 planes for that, and to 2 when the grid would leave CUs
+// z-march launch shape: tiles x z chunks.  Chunks of at least 6 planes by the
+// expected time of the busiest CU, in planes of a block alone on its CU: k
+// blocks on a CU, in rounds of at most `resident` (what it holds), take max(1,
+// add + mul k) of that per plane, or bw k where the arrays are beyond the
+// last-level cache; a chunk costs its plane count, `pre` planes for the loads of
+// its window and `blk` to start.  What the rule avoids is a CU
+// with one block more than the others: 190 tiles of 300^3 points in FP64, order
+// 8, nabla_u with square: 2 chunks (1.5 blocks per CU) 425 us, 4 (3.0) 357, 7
+// (5.2) 377.  Below 6 planes, down to 2, only when the grid would leave CUs
 // without a block (order 4 on 100 x 60 x 40: 11.6 us against 13.8 with 4).
+struct PzCost {
+  double blk, pre, add, mul, bw;
+};
+// fitted to 1 .. 40 chunks of every operator on 128^3 to 350^3 points
+constexpr double kPzCached = 128e6;  // bytes of four arrays: half the cache
+template <typename R, int NO, int MODE>
+static PzCost pz_cost(const PGeom& g, const GradEpi<R>& ep) {
+  if (sizeof(R) == 8) return PzCost{1.3, 0.2 * NO, 0, NO == 16 ? 0.44 : 0.4, 0};
+  // few arrays: several blocks overlap better
+  if (NO < 16 && (MODE == 0 || (MODE == GE_GRAD && !ep.du2))) return PzCost{0.3, 0.3 * NO, 0, 0.4, 0};
+  return PzCost{0.3, 0.3 * NO, 0.75, 0.31, 4.0 * sizeof(R) * g.np > kPzCached ? 0.5 : 0};
+}
+static int pz_zchunk(const PzCost& m, long tiles, int nz, int resident) {
+  int best = nz;
+  double bt = 1e300;
+  for (int c = 1; c <= std::max(1, nz / 6); ++c) {
+    const int zc = (nz + c - 1) / c;
+    const long k = (tiles * ((nz + zc - 1) / zc) + num_cu() - 1) / num_cu(), kr = std::min<long>(k, resident);
+    const long rounds = (k + resident - 1) / resident;
+    if (c > 1 && rounds > 3) break;
+    const double t = rounds * ((zc + m.pre) * std::max({1.0, m.add + m.mul * kr, m.bw * kr}) + m.blk * kr);
+    if (t < bt) bt = t, best = zc;
+  }
+  return best;
+}
 // False when the one-point kernels must do all (LIBCONV_POISSON_POINT set,
 // planes beyond the buffer-record limit).
 struct PzLaunch {
   int tiles_x, tiles, zchunk;
   unsigned blocks;
 };
-static bool pz_launch(const PGeom& g, int ty, int resident, PzLaunch& L) {
+static bool pz_launch(const PGeom& g, int ty, int resident, const PzCost& cost, PzLaunch& L) {
   if (getenv("LIBCONV_POISSON_POINT")) return false;
   if ((long)g.n0 * g.n1 * 8 > kPlaneMax) return false;
   L.tiles_x = (g.n0 + kZTX - 1) / kZTX;
   const long tiles = (long)L.tiles_x * ((g.n1 + ty - 1) / ty);
-  long chunks = std::min<long>((long)std::max(1, resident) * num_cu() / tiles, g.n2 / 6);
-  if (chunks * tiles < num_cu()) chunks = std::min<long>((num_cu() + tiles - 1) / tiles, g.n2 / 2);
-  chunks = std::max(1L, chunks);
-  L.zchunk = (int)((g.n2 + chunks - 1) / chunks);
+  if (tiles * (g.n2 / 6) >= num_cu()) {
+    L.zchunk = pz_zchunk(cost, tiles, g.n2, resident);
+  } else {
+    const long chunks = std::max(1L, std::min<long>((num_cu() + tiles - 1) / tiles, g.n2 / 2));
+    L.zchunk = (int)((g.n2 + chunks - 1) / chunks);
+  }
   const long nb = tiles * ((g.n2 + L.zchunk - 1) / L.zchunk);
   if (nb > 0x7fffffffL) return false;
   L.tiles = (int)tiles;
@@ -851,21 +883,6 @@ static int pz_resident() {
   return nb;
 }
 
-// Blocks per CU on arrays beyond the last-level cache, orders below 16 (order 16
-// has the registers or the work to be indifferent): longer chunks re-read
-// fewer window planes from memory.  256^3, all blocks that fit against this
-// many: FP64 order 4 div_u_i 112 -> 105 us, nabla_u 128 -> 122, with square 155
-// -> 149; FP32 order 8 nabla_u 59 -> 47, div_u_i 55 -> 46.  The operators that
-// gain nothing keep all (div_u_i with cc, three inputs in LDS: FP64 order 8 on
-// 200 x 150 x 180 59 us against 72; in FP32 those of four outputs or one).
-constexpr double kPzCached = 128e6;  // bytes of four arrays: half the cache
-template <typename R, int MODE>
-static int pz_stream_blocks(const GradEpi<R>& ep) {
-  if (MODE == 1) return 8;  // div_u_i with cc
-  if (sizeof(R) == 8) return MODE == GE_SQUARE ? 3 : 2;
-  return MODE == GE_SQUARE || MODE == GE_EPS || ep.du2 ? 8 : 3;
-}
-
 // one z-march launch; its blocks, or 0 when the one-point kernels must run;
 // dry: count only
 template <typename R, int NO, int MODE, int TY>
@@ -873,9 +890,8 @@ static long pz_run_rows(const PGeom& g, const R* u, R* o0, R* o1, const GradEpi<
                         hipStream_t st, bool dry) {
   constexpr int NT = PzGeo<R, NO, TY>::NT;
   PzLaunch L;
-  int resident = pz_resident<poisson_zm_kernel<R, NO, MODE, TY>, NT>();
-  if (NO < 16 && 4.0 * sizeof(R) * g.np > kPzCached) resident = std::min(resident, pz_stream_blocks<R, MODE>(ep));
-  if (!pz_launch(g, TY, resident, L)) return 0;
+  const int resident = pz_resident<poisson_zm_kernel<R, NO, MODE, TY>, NT>();
+  if (!pz_launch(g, TY, resident, pz_cost<R, NO, MODE>(g, ep), L)) return 0;
   if (!dry)
     poisson_zm_kernel<R, NO, MODE, TY><<<L.blocks, NT, 0, st>>>(g, L.tiles_x, L.tiles, L.zchunk, u, o0, o1, ep, r0,
                                                                 r1, r2);
