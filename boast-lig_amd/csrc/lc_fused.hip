@@ -194,7 +194,7 @@ static int env_variant(const char* name, int nvar) {
   return v >= 0 && v < nvar ? v : -1;
 }
 
-int default_variant(int prec, int form, const Box3& b) {
+int default_variant(int prec, int form, const Box3& b, int narr, bool acc) {
   if (form == FORM_SUM || form == FORM_SEP) {
     // defaults: the fastest variants on MI355X (MF in FP64: the 128-bit-LDS
     // kernel on 32 x 16 tiles, 4-10% ahead of the others from the 128^3
@@ -226,7 +226,8 @@ int default_variant(int prec, int form, const Box3& b) {
   // the pair-wise kernel (its outputs go through 32-bit buffer records): the
   // block that the model in lc_fused_wav.hip expects to be fastest on this
   // grid; else one z-step per slide
-  if (wav_plane_fits(b, prec) && 4L * b.ny[0] * b.ny[1] * prec <= kPlaneMax) return wav_default_variant(prec, form, b);
+  if (wav_plane_fits(b, prec) && 4L * b.ny[0] * b.ny[1] * prec <= kPlaneMax)
+    return wav_default_variant(prec, form, b, narr, acc);
   return 5;
 }
 

@@ -207,24 +207,63 @@ static int wav_zchunk(long tiles, int narr, int nout) {
 }
 
 // ---- tile and z chunk of the pair-wise kernels
-// Cycles of one block-step: the issue of its FMAs (x-tasks 32 QX, y-tasks
-// 128 / HB per wave of four cycles, over four SIMDs), its bytes at the CU's
-// share of the copy rate (9.3 bytes per cycle; rows and runs each cost most of
-// a 128-byte line more than they hold), and its serial chain (tile write, x,
-// y, z with a barrier between).  lat is a fit to blocks alone on their CU
-// (33 x 57 x 24 pairs, us per step in FP64 / FP32: QX 4 1.36 / 1.0, QX 2 1.21,
-// two lanes per y-task 1.06 / 0.73).
+// Work of one block-step: the issue of its FMAs in cycles (x-tasks 32 QX,
+// y-tasks 128 / HB per wave of four cycles, over four SIMDs), its bytes and its
+// runs of adjacent bytes.  A DWT row holds its pairs side by side and each band
+// of the output is a run of its own; an IDWT row lies in two bands and the
+// output's pairs side by side.
+struct WavWork {
+  double fma, rd, rd_runs, wr, wr_runs;
+};
+static WavWork wav_work(const WavqBlock& k, const WavqShape& g, int rs, bool inverse) {
+  WavWork w;
+  w.fma = 32.0 * k.QX * ((g.xtasks(k.QX) + 63) / 64) + 128.0 * ((2 * g.tx * g.ty + 63) / 64);
+  w.rd = 4.0 * g.nr * (g.tx + 7) * rs;
+  w.rd_runs = 2.0 * g.nr * (inverse ? 2 : 1);
+  w.wr = 8.0 * g.tx * g.ty * rs;
+  w.wr_runs = (inverse ? 4.0 : 8.0) * g.ty;
+  return w;
+}
+// Time of one step of a single call, in us, with n blocks on the CU: the serial
+// chain of a block (tile write, x, y, z with a barrier between), hardly longer
+// with a second one beside it, or what the blocks' FMAs and bytes take together.
+//   step(n) = max(lat (1 + 0.05 n), add + n (fma + mem bytes))
+// Fitted to 5 to 6000 launches (tile x chunk) of each of 70 calls: cubes of 32
+// to 160 pairs and flat and long boxes, all boundary conditions, with and
+// without a_y; the picked launch is 3 - 5% behind the best of them on average.
+// half: the chain of the two-lane block; halo: weight of the bytes read; run:
+// bytes that a run costs beside those it holds.
+struct WavFit {
+  double lat, half, halo, fma, mem, add, run;
+};
+constexpr WavFit kWavFit[2][2] = {  // [FP64, FP32][DWT, IDWT]
+    {{1.14, 0.83, 3.76, 0.096e-3, 0.671e-5, 0.451, 14}, {1.19, 0.776, 4.25, 0.355e-3, 0.235e-5, 0.481, 79}},
+    {{0.942, 0.70, 6.41, 0.288e-3, 0.07e-5, 0.367, 175}, {1.16, 0.693, 2.28, 0.121e-3, 0.735e-5, 0.418, 39}}};
+struct WavStep {
+  double lat, add, per;
+  double operator()(double n) const { return std::max(lat * (1.0 + 0.05 * n), add + n * per); }
+};
+// acc: with the a_y y term, whose loads of y end the step
+static WavStep wav_step(const WavqBlock& k, const WavqShape& g, int rs, bool inverse, bool acc) {
+  const WavFit& f = kWavFit[rs == 4][inverse];
+  const WavWork w = wav_work(k, g, rs, inverse);
+  const double bytes = f.halo * (w.rd + f.run * w.rd_runs) + (acc ? 2 : 1) * (w.wr + f.run * w.wr_runs);
+  WavStep s;
+  s.lat = f.lat * (k.HB == 2 ? f.half : k.S > 128 ? 1.35 : 1.0) * (acc ? 1.8 : 1.0);
+  s.add = acc ? 0.9 : f.add;
+  s.per = (f.fma * w.fma + f.mem * bytes) * (acc ? 1.1 : 1.0);
+  return s;
+}
+// Cycles and bytes of a step where blocks fill the chip for many rounds (batch
+// stages): half of the halo reads hit L2, rows and runs cost most of a line more
+// than they hold, 9.3 bytes per cycle are the CU's share of the copy rate.
 struct WavCost {
-  double fma, mem, lat;
+  double fma, mem;
 };
 static WavCost wav_cost(const WavqBlock& k, const WavqShape& g, int rs) {
   const double rd = 2.0 * g.nr * (2 * (g.tx + 7) * rs + 96), own = 8.0 * g.tx * g.ty * rs;
   const double wr = 8.0 * g.ty * (g.tx * rs + 48);
-  WavCost c;
-  c.fma = 32.0 * k.QX * ((g.xtasks(k.QX) + 63) / 64) + 128.0 * ((2 * g.tx * g.ty + 63) / 64);
-  c.mem = (0.5 * (rd + own) + wr) / 9.3;  // about half of the halo reads hit L2
-  c.lat = rs == 8 ? 1900 + 3.7 * (32 * k.QX + 128 / k.HB) : 900 + 4.8 * (32 * k.QX + 128 / k.HB);
-  return c;
+  return WavCost{wav_work(k, g, rs, false).fma, (0.5 * (rd + own) + wr) / 9.3};
 }
 struct WavPick {
   int tx = 0, ty = 0, zchunk = 0;
@@ -248,25 +287,19 @@ static void wav_tiles(const WavqBlock& k, int w0, int w1, int rs, F&& f) {
     if (ty <= 4) break;
   }
 }
-// Single calls: the tile and z chunk with the least (steps) x (time per step).
-// A chunk of c output steps takes c + 7 input steps; a step takes the serial
-// chain while a CU has one block and the blocks' FMAs (at half of their issue
-// rate, measured at 96^3 and 112^3 pairs) or bytes beyond: all blocks start
-// together, so most halo reads hit L2 and the bytes count half.
-static WavPick wav_pick(const WavqBlock& k, int w0, int w1, int nz, int narr, int rs) {
+// Single calls: the tile and z chunk with the least expected time.  A chunk of c
+// output steps takes c + 7 input steps; every CU is as late as the busiest.
+static WavPick wav_pick(const WavqBlock& k, int w0, int w1, int nz, int narr, int rs, bool inverse, bool acc) {
   WavPick best;
   const long ncu = num_cu();
   const int occ = std::max(1, 1024 / k.nt());  // blocks per CU: 128 VGPRs, four waves per SIMD
   wav_tiles(k, w0, w1, rs, [&](const WavqShape& g, long tiles) {
-    const WavCost c = wav_cost(k, g, rs);
-    const double full = std::max((rs == 8 ? 2.1 : 1.7) * c.fma, 0.52 * c.mem);
+    const WavStep step = wav_step(k, g, rs, inverse, acc);
     auto consider = [&](long chunks) {
       if (chunks < 1 || chunks > nz) return;
       const int zc = (int)((nz + chunks - 1) / chunks);
       const long blocks = tiles * narr * ((nz + zc - 1) / zc);
-      const long per = (blocks + ncu - 1) / ncu;
-      const double rounds = per <= occ ? 1.0 : (double)blocks / (ncu * occ);
-      const double t = (zc + 7) * rounds * std::max(c.lat, std::min<long>(per, occ) * full);
+      const double t = (zc + 7) * step((double)((blocks + ncu - 1) / ncu));
       if (t < best.t) best = WavPick{g.tx, g.ty, zc, t};
     };
     for (int q = 1; q <= 2 * occ; ++q) consider(q * ncu / (tiles * narr));
@@ -276,43 +309,42 @@ static WavPick wav_pick(const WavqBlock& k, int w0, int w1, int nz, int narr, in
   return best;
 }
 // The picks of recent shapes (the search takes some 10 us), per host thread.
-static WavPick wav_pick_cached(int v, const WavqBlock& k, int w0, int w1, int nz, int narr, int rs) {
+static WavPick wav_pick_cached(int v, const WavqBlock& k, int w0, int w1, int nz, int narr, int rs, bool inverse,
+                               bool acc) {
   struct Entry {
     int key[6];
     WavPick p;
   };
   constexpr int kEntries = 64;
   static thread_local Entry cache[kEntries];  // zero-initialised: no variant 0 here
-  const int key[6] = {v, w0, w1, nz, narr, rs};
+  const int key[6] = {4 * v + 2 * inverse + acc, w0, w1, nz, narr, rs};
   unsigned h = 0;
   for (int q : key) h = h * 31u + (unsigned)q;
   Entry& e = cache[h % kEntries];
   if (!std::equal(key, key + 6, e.key)) {
-    e.p = wav_pick(k, w0, w1, nz, narr, rs);
+    e.p = wav_pick(k, w0, w1, nz, narr, rs, inverse, acc);
     std::copy(key, key + 6, e.key);
   }
   return e.p;
 }
 
-// The variant a call takes by default: of the block for 128 output steps and
-// the two-lane block for 64 the one the model expects to be faster.  Larger
-// blocks were not faster at any single grid tried (16^3 to 112^3 pairs); FP64
-// with two outputs per x-task is within 6% of four.
-int wav_default_variant(int prec, int form, const Box3& b) {
+// The variant a call takes by default: of the block for 128 output steps (four
+// outputs per x-task) and the two-lane block for 64 the one expected to be
+// faster.  The best launches of larger blocks and of two outputs per x-task are
+// within 1.5% of the best of these on average, 5% up to 112^3 pairs (144^3 FP64
+// 115 us in 256 steps against 117).
+int wav_default_variant(int prec, int form, const Box3& b, int narr, bool acc) {
   const int lo = form == FORM_IDWT ? Idwt<Sym8Rec>::LO : Dwt<Sym8Dec>::LO;
   const FDim d0 = fdim(b.n[0], b.bc[0], b.nx[0], b.ny[0], lo, lo + 7), d1 = fdim(b.n[1], b.bc[1], b.nx[1], b.ny[1], lo, lo + 7),
              d2 = fdim(b.n[2], b.bc[2], b.nx[2], b.ny[2], lo, lo + 7);
-  static const int f64[] = {16, 11}, f32[] = {7, 11};
   int best = 5;
   double t = 1e300;
-  for (int v : prec == 4 ? f32 : f64) {
+  for (int v : {7, 11}) {
     WavqBlock k;
     if (!wavq_block(v, &k)) continue;
-    const WavPick p = wav_pick_cached(v, k, d0.nout, d1.nout, d2.nout, 1, prec);
-    // a synthesis tile takes two loads per pair, which the block of half the
-    // tile hides better (64^3 pairs, FP64: 31.8 against 33.2 us)
-    const double pt = p.t * (form == FORM_IDWT && k.HB == 1 ? 1.06 : 1.0);
-    if (pt < t) { t = pt; best = v; }
+    const WavPick p = wav_pick_cached(v, k, d0.nout, d1.nout, d2.nout, std::max(narr, 1), prec,
+                                      form == FORM_IDWT, acc);
+    if (p.t < t) { t = p.t; best = v; }
   }
   return best;
 }
@@ -343,7 +375,8 @@ static hipError_t launch_wavq(const Box3& b, int narr, const R* x, R* y, R a, R 
   if (narr == 0) return hipSuccess;
   constexpr WavqBlock kB{NG * TX * TY, QX, KB + 1};
   FusedArgs<R> p = wav_args<R, Op, TX, TY, QX, 1, 1>(b, narr, x, y, a, a_y);
-  const WavPick k = wav_pick_cached(V, kB, p.d0.nout, p.d1.nout, p.d2.nout, narr, sizeof(R));
+  const WavPick k = wav_pick_cached(V, kB, p.d0.nout, p.d1.nout, p.d2.nout, narr, sizeof(R), WavCoef<Op>::K == KIDWT,
+                                    (p.flags & F_AY) != 0);
   p.tile_x = k.tx;
   p.tile_y = k.ty;
   p.tiles_x = (p.d0.nout + k.tx - 1) / k.tx;
@@ -392,7 +425,9 @@ hipError_t sepw3d_v(int v, int kind, int id, const Box3& b, int narr, const R* x
 template <typename R>
 hipError_t sepw3d(int kind, int id, const Box3& b, int narr, const R* x, R* y, R a, R a_y,
                   hipStream_t st) {
-  const int v = select_variant(sizeof(R), kind == KIDWT ? FORM_IDWT : FORM_DWT, id, b);
+  const int form = kind == KIDWT ? FORM_IDWT : FORM_DWT;
+  int v = chosen_variant(sizeof(R), form, id, b);
+  if (v < 0) v = default_variant(sizeof(R), form, b, narr, a_y != R(0));
   return sepw3d_v<R>(v, kind, id, b, narr, x, y, a, a_y, st);
 }
 

@@ -185,13 +185,14 @@ enum Form : int { FORM_SEP = 0, FORM_SUM = 1, FORM_DWT = 2, FORM_IDWT = 3 };
 int variant_count(int form);          // single-call variants
 bool has_batch_form(int form, int v);  // the variant also has a batched kernel
 int wav_variant_count();
-int wav_default_variant(int prec, int form, const Box3& b);
+int wav_default_variant(int prec, int form, const Box3& b, int narr, bool acc);
 int wav_batch_variant(int prec, int single, const Box3* b, int count);
 // variant a call of this shape uses: the chosen one (tuner table, else
-// environment; -1: neither names one), else the default
+// environment; -1: neither names one), else the default (of narr arrays; acc:
+// with the a_y term)
 int select_variant(int prec, int form, int id, const Box3& b);
 int chosen_variant(int prec, int form, int id, const Box3& b);
-int default_variant(int prec, int form, const Box3& b);
+int default_variant(int prec, int form, const Box3& b, int narr = 1, bool acc = false);
 // tuner table lookup (lc_tune.cpp): -1 when the shape was not tuned
 int tuned_variant(int prec, int form, int id, const Box3& b);
 std::string fused_kernel_name(int prec, int form, int id, int v, bool batch);
