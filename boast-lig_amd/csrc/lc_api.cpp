@@ -1183,13 +1183,16 @@ int stage_default_variant(const lc_batch_item* it, int count, int prec) {
   }
   const int form = item_form(it[big]);
   int v = chosen_variant(prec, form, it[big].op, item_box(it[big]));
-  if (v < 0) {
-    v = default_variant(prec, form, item_box(it[big]));
-    if (form == FORM_DWT || form == FORM_IDWT) {
-      std::vector<Box3> boxes;
-      for (int i = 0; i < count; ++i) boxes.push_back(item_box(it[i]));
-      v = wav_batch_variant(prec, v, boxes.data(), count);
+  if (v < 0 && (form == FORM_DWT || form == FORM_IDWT)) {
+    std::vector<Box3> boxes;
+    bool acc = false;
+    for (int i = 0; i < count; ++i) {
+      boxes.push_back(item_box(it[i]));
+      acc = acc || it[i].a_y != 0.0;
     }
+    v = wav_batch_variant(prec, form, boxes.data(), count, acc);
+  } else if (v < 0) {
+    v = default_variant(prec, form, item_box(it[big]));
   }
   if (has_batch_form(form, v)) return v;
   bool fit = true;

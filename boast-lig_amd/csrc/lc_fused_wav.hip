@@ -20,6 +20,7 @@
 //         step i at c + 2 (i - oy)
 // Periodic dims wrap, free dims read zero outside the stored input, exactly
 // as the 1D sweeps.  Epilogue: y = a * t + a_y * y.
+#include <math.h>
 #include <stdio.h>
 #include <stdlib.h>
 
@@ -349,21 +350,32 @@ int wav_default_variant(int prec, int form, const Box3& b, int narr, bool acc) {
   return best;
 }
 
-// The default of a batch stage whose largest item by itself would take `single`
-// by default: a stage that fills every CU is bound by bytes, so it takes the block
-// with the widest tiles, in FP64 512 output steps, in FP32 (more blocks per
-// CU) 256.  128 orbitals of 24..96 pairs, DWT stage: FP64 1.55 / 1.34 / 1.25
-// ms for 128 / 256 / 512 steps, FP32 0.90 / 0.78 / 0.83.
-int wav_batch_variant(int prec, int single, const Box3* b, int count) {
-  if (single < 7) return single;  // the step-at-a-time form: planes beyond the buffer records
+// How many items of this one's size the items of a stage make together: the
+// stage is laid out as a call with that many arrays.
+static double wav_points(const Box3& b) { return (double)b.ny[0] * b.ny[1] * b.ny[2]; }
+static int wav_copies(double total, const Box3& b) {
+  return (int)std::min(1e6, std::max(1.0, std::ceil(total / wav_points(b))));
+}
+
+// The default of a batch stage: one that fills every CU is bound by bytes, so it
+// takes the block with the widest tiles, in FP64 512 output steps, in FP32 (more
+// blocks per CU) 256.  128 orbitals of 24..96 pairs, DWT stage: FP64 1.55 / 1.34
+// / 1.25 ms for 128 / 256 / 512 steps, FP32 0.90 / 0.78 / 0.83.  A smaller one
+// takes what a call with as many arrays of its largest item would.
+int wav_batch_variant(int prec, int form, const Box3* b, int count, bool acc) {
   long steps = 0;
+  double total = 0;
+  int big = 0;
   for (int i = 0; i < count; ++i) {
-    if (!wavq_fits(b[i], prec)) return single;
+    if (!wavq_fits(b[i], prec)) return 5;  // the step-at-a-time form: planes beyond the buffer records
     steps += (long)b[i].ny[0] * b[i].ny[1];
+    total += wav_points(b[i]);
+    if (wav_points(b[i]) > wav_points(b[big])) big = i;
   }
   const int v = prec == 4 ? 10 : 9;
   WavqBlock k;
-  return wavq_block(v, &k) && steps >= (long)k.S * num_cu() * std::max(1, 1024 / k.nt()) ? v : single;
+  if (wavq_block(v, &k) && steps >= (long)k.S * num_cu() * std::max(1, 1024 / k.nt())) return v;
+  return wav_default_variant(prec, form, b[big], wav_copies(total, b[big]), acc);
 }
 
 template <int V, typename R, class Op, int NG, int TX, int TY, int QX, int PD, int WPE, int KB>
@@ -432,10 +444,75 @@ hipError_t sepw3d(int kind, int id, const Box3& b, int narr, const R* x, R* y, R
 }
 
 // ---- batches of independent 3D sym8 wavelet transforms
+// Tiles and z chunks of a pair-wise stage that leaves CUs without a full load and
+// whose arrays the last-level cache holds.  Items of one shape: as one call with
+// that many arrays.  Others: the tiles with the least work, and marches of one
+// length, the one with the least expected time of the busiest CU.
+constexpr double kWavCached = 256e6;  // bytes read and written
+template <typename R, class Op>
+static void wav_batch_layout(const WavqBlock& k, const BatchItem<R>* it, int count, bool acc, FusedArgs<R>* tab) {
+  constexpr bool inverse = WavCoef<Op>::K == KIDWT;
+  bool same = true;
+  for (int o = 1; o < count; ++o)
+    same = same && tab[o].d0.nout == tab[0].d0.nout && tab[o].d1.nout == tab[0].d1.nout && tab[o].d2.nout == tab[0].d2.nout;
+  if (same) {
+    const WavPick w = wav_pick(k, tab[0].d0.nout, tab[0].d1.nout, tab[0].d2.nout, count, sizeof(R), inverse, acc);
+    for (int o = 0; o < count; ++o) {
+      tab[o].tile_x = w.tx;
+      tab[o].tile_y = w.ty;
+      tab[o].zchunk = w.zchunk;
+    }
+  } else {
+    double lat = 0, add = 0, per = 0, tiles_all = 0;
+    int nz = 1;
+    for (int o = 0; o < count; ++o) {
+      FusedArgs<R>& p = tab[o];
+      double best = 1e300;
+      WavStep bs{};
+      wav_tiles(k, p.d0.nout, p.d1.nout, sizeof(R), [&](const WavqShape& g, long tiles) {
+        const WavStep st = wav_step(k, g, sizeof(R), inverse, acc);
+        if (tiles * st.per < best) { best = tiles * st.per; bs = st; p.tile_x = g.tx; p.tile_y = g.ty; }
+      });
+      const double t = (double)((p.d0.nout + p.tile_x - 1) / p.tile_x) * ((p.d1.nout + p.tile_y - 1) / p.tile_y);
+      lat = bs.lat;
+      add = bs.add;
+      per += t * bs.per;
+      tiles_all += t;
+      nz = std::max(nz, p.d2.nout);
+    }
+    const WavStep mean{lat, add, per / tiles_all};
+    int march = nz;
+    double bt = 1e300;
+    for (int z = std::min(4, nz); z <= nz; ++z) {
+      long n = 0;
+      int most = 0;
+      for (int o = 0; o < count; ++o) {
+        const FusedArgs<R>& p = tab[o];
+        const int c = (p.d2.nout + z - 1) / z, zc = (p.d2.nout + c - 1) / c;
+        n += (long)((p.d0.nout + p.tile_x - 1) / p.tile_x) * ((p.d1.nout + p.tile_y - 1) / p.tile_y) *
+             ((p.d2.nout + zc - 1) / zc);
+        most = std::max(most, zc);
+      }
+      const double t = (most + 7) * mean((double)((n + num_cu() - 1) / num_cu()));
+      if (t < bt) { bt = t; march = z; }
+    }
+    for (int o = 0; o < count; ++o) {
+      const int c = (tab[o].d2.nout + march - 1) / march;
+      tab[o].zchunk = (tab[o].d2.nout + c - 1) / c;
+    }
+  }
+  for (int o = 0; o < count; ++o) {
+    FusedArgs<R>& p = tab[o];
+    p.tiles_x = (p.d0.nout + p.tile_x - 1) / p.tile_x;
+    p.tiles_y = (p.d1.nout + p.tile_y - 1) / p.tile_y;
+  }
+}
+
 template <typename R, class Op, int TX, int TY, int QX, int BZ, int AD, int WPE>
 static hipError_t wav_stage_build(const BatchItem<R>* it, int count, BatchStage* s) {
   std::vector<FusedArgs<R>> tab(count);
   long tiles_all = 0;
+  double total = 0;
   WavqBlock k{};
   const bool pairwise = wavq_block(s->variant, &k);
   for (int o = 0; o < count; ++o)
@@ -444,6 +521,7 @@ static hipError_t wav_stage_build(const BatchItem<R>* it, int count, BatchStage*
     FusedArgs<R>& p = tab[o];
     p = wav_args<R, Op, TX, TY, QX, BZ, AD>(it[o].b, 1, it[o].x, it[o].y, (R)it[o].a[0], (R)it[o].a_y);
     if (p.flags & F_AY) s->any_acc = true;
+    total += wav_points(it[o].b);
     if (pairwise) {
       // a full chip: the tile with the least bytes and (half hidden) FMAs
       double best = 1e300;
@@ -461,10 +539,14 @@ static hipError_t wav_stage_build(const BatchItem<R>* it, int count, BatchStage*
   const long want = (pairwise ? std::max(1, 1024 / k.nt()) : 2) * (long)num_cu();
   const long chunks = std::max(1L, (want + tiles_all - 1) / std::max(1L, tiles_all));
   std::vector<long> blocks(count), steps(count);
+  const bool fitted = pairwise && chunks > 1 && 16.0 * sizeof(R) * total <= kWavCached;
+  if (fitted) wav_batch_layout<R, Op>(k, it, count, s->any_acc, tab.data());
   for (int o = 0; o < count; ++o) {
     FusedArgs<R>& p = tab[o];
-    const long c = std::max(1L, std::min<long>(chunks, std::max(1, p.d2.nout / (2 * Op::W))));
-    p.zchunk = (int)((p.d2.nout + c - 1) / c);
+    if (!fitted) {
+      const long c = std::max(1L, std::min<long>(chunks, std::max(1, p.d2.nout / (2 * Op::W))));
+      p.zchunk = (int)((p.d2.nout + c - 1) / c);
+    }
     blocks[o] = (long)p.tiles_x * p.tiles_y * ((p.d2.nout + p.zchunk - 1) / p.zchunk);
     steps[o] = p.zchunk + Op::W - 1;
   }

@@ -186,7 +186,7 @@ int variant_count(int form);          // single-call variants
 bool has_batch_form(int form, int v);  // the variant also has a batched kernel
 int wav_variant_count();
 int wav_default_variant(int prec, int form, const Box3& b, int narr, bool acc);
-int wav_batch_variant(int prec, int single, const Box3* b, int count);
+int wav_batch_variant(int prec, int form, const Box3* b, int count, bool acc);
 // variant a call of this shape uses: the chosen one (tuner table, else
 // environment; -1: neither names one), else the default (of narr arrays; acc:
 // with the a_y term)
