@@ -127,20 +127,21 @@ def _ints(v):
     return a
 
 
-def _iv(v):
+def _iv(v, flat=False):
     """A dims argument as a C int array, for the calls on device tensors: the
     smallest of them last a few microseconds on the GPU, and a numpy array and
     its pointer cost one each.  Whatever array('i') does not take goes through
-    _ints, with its conversions and errors."""
+    _ints, with its conversions and errors.  flat: an argument that is only
+    passed on, whose values are taken in memory order whatever its shape."""
     if type(v) in (list, tuple) and v:
         try:
             return (_I * len(v)).from_buffer(array('i', v))
         except (TypeError, OverflowError):
             pass
     a = _ints(v)
-    if a.size != len(a):
+    if a.size != len(a) and not flat:
         raise TypeError('dims: one integer per dimension')
-    return (_I * len(a))(*a.ravel().tolist())
+    return (_I * a.size)(*a.ravel().tolist())
 
 
 def _addr(t):
@@ -386,7 +387,7 @@ def wavelet_1d(wav, inverse, idim, n, bc, nx, ny, narr, x, y, a=1.0, a_y=0.0, st
 
 
 def conv_md(fil, n, bc, nx, ny, narr, x, y, a=1.0, a_x=0.0, a_y=0.0, stream=None):
-    n_, b_, nx_, ny_ = _iv(n), _iv(bc), _iv(nx), _iv(ny)
+    n_, b_, nx_, ny_ = _iv(n), _iv(bc, flat=True), _iv(nx), _iv(ny)
     pr = _prec(x)
     _dev(x, 'x', pr, _count(nx_) * narr)
     _dev(y, 'y', pr, _count(ny_) * narr)
@@ -396,7 +397,7 @@ def conv_md(fil, n, bc, nx, ny, narr, x, y, a=1.0, a_x=0.0, a_y=0.0, stream=None
 
 
 def conv_1ds(fil, n, bc, nx, ny, narr, a, a_x, a_y, x, y, dot=None, stream=None):
-    n_, b_, nx_, ny_ = _iv(n), _iv(bc), _iv(nx), _iv(ny)
+    n_, b_, nx_, ny_ = _iv(n), _iv(bc, flat=True), _iv(nx), _iv(ny)
     pr = _prec(x)
     _dev(x, 'x', pr, _count(nx_) * narr)
     _dev(y, 'y', pr, _count(ny_) * narr)
@@ -412,7 +413,7 @@ def conv_1ds_noalloc(fil, n, bc, nx, ny, narr, a, a_x, a_y, x, y, dot=None, stre
     """conv_1ds through lc_conv_1ds_noalloc: the energy partials use the
     library's static device buffer, no allocation (calls on one GPU must not
     overlap)."""
-    n_, b_, nx_, ny_ = _iv(n), _iv(bc), _iv(nx), _iv(ny)
+    n_, b_, nx_, ny_ = _iv(n), _iv(bc, flat=True), _iv(nx), _iv(ny)
     av = np.ascontiguousarray(np.asarray(a, dtype=np.float64))
     pr = _prec(x)
     _dev(x, 'x', pr, _count(nx_) * narr)
@@ -425,7 +426,7 @@ def conv_1ds_noalloc(fil, n, bc, nx, ny, narr, a, a_x, a_y, x, y, dot=None, stre
 
 
 def wavelet_md(wav, inverse, n, bc, nx, ny, narr, x, y, a=1.0, a_y=0.0, stream=None):
-    n_, b_, nx_, ny_ = _iv(n), _iv(bc), _iv(nx), _iv(ny)
+    n_, b_, nx_, ny_ = _iv(n), _iv(bc, flat=True), _iv(nx), _iv(ny)
     pr = _prec(x)
     _dev(x, 'x', pr, _count(nx_, 2) * narr)
     _dev(y, 'y', pr, _count(ny_, 2) * narr)
@@ -438,7 +439,7 @@ def local_hamiltonian_work(n):
     """Elements of the work array lc_local_hamiltonian needs for n pairs per dim."""
     L = lib()
     L.lc_local_hamiltonian_work.restype = ctypes.c_long
-    w = L.lc_local_hamiltonian_work(_iv(n))
+    w = L.lc_local_hamiltonian_work(_iv(n, flat=True))
     check()
     return int(w)
 
