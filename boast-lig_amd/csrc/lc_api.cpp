@@ -146,6 +146,17 @@ bool is_device_ptr(const void* p) {
   return at.type == hipMemoryTypeDevice || at.type == hipMemoryTypeManaged;
 }
 
+// memory of the current device, which its kernels write without a mapping
+bool is_local_ptr(const void* p) {
+  hipPointerAttribute_t at;
+  int dev = -1;
+  if (hipPointerGetAttributes(&at, p) != hipSuccess) {
+    (void)hipGetLastError();
+    return false;
+  }
+  return hipGetDevice(&dev) == hipSuccess && at.type == hipMemoryTypeDevice && at.device == dev;
+}
+
 // Host-or-device array argument of a drop-in call.
 template <typename R>
 struct Arg {
@@ -513,14 +524,15 @@ int run_1ds(int fil, int d, const int* n, const int* bc, const int* nx, const in
     dot3 = reinterpret_cast<double*>(static_cast<char*>(sc) + sbytes);
     // three energies go straight to the caller's device array (a copy is a
     // launch of its own: 2 us and the gap before it); with fewer dims the
-    // kernel's three values do not fit there
-    if (d == 3 && dot_dev_user) dot3 = dot_dev_user;
+    // kernel's three values do not fit there, and memory of the host or of
+    // another GPU takes the copy
+    if (d == 3 && dot_dev_user && is_local_ptr(dot_dev_user)) dot3 = dot_dev_user;
   }
   hipError_t e = sum3d<R>(fil, b, narr, ax.dev, ay.dev, a3, (R)a_x, (R)a_y, want_dot ? dot3 : nullptr,
                           st, scratch, sbytes);
   if (e != hipSuccess) return hip_fail(e, who);
   if (want_dot && dot_dev_user && dot3 != dot_dev_user)
-    HIPCHK(hipMemcpyAsync(dot_dev_user, dot3, d * sizeof(double), hipMemcpyDeviceToDevice, st));
+    HIPCHK(hipMemcpyAsync(dot_dev_user, dot3, d * sizeof(double), hipMemcpyDefault, st));
   if (!device_api) {
     if (ay.host_in) HIPCHK(hipMemcpyAsync(y, ay.dev, (size_t)tout * narr * sizeof(R), hipMemcpyDeviceToHost, st));
     if (dot_host) HIPCHK(hipMemcpyAsync(dot_host, dot3, d * sizeof(double), hipMemcpyDeviceToHost, st));
