@@ -248,7 +248,10 @@ struct WavStep {
 static WavStep wav_step(const WavqBlock& k, const WavqShape& g, int rs, bool inverse, bool acc) {
   const WavFit& f = kWavFit[rs == 4][inverse];
   const WavWork w = wav_work(k, g, rs, inverse);
-  const double bytes = f.halo * (w.rd + f.run * w.rd_runs) + (acc ? 2 : 1) * (w.wr + f.run * w.wr_runs);
+  // FP64 synthesis with two outputs per x-task takes narrow tiles better: 96^3
+  // pairs 49.1 us with tiles of 8 x 16 steps, 50.9 with 16 x 8
+  const double run = k.QX == 2 && k.HB == 1 && rs == 8 && inverse ? 55 : f.run;
+  const double bytes = f.halo * (w.rd + run * w.rd_runs) + (acc ? 2 : 1) * (w.wr + run * w.wr_runs);
   WavStep s;
   s.lat = f.lat * (k.HB == 2 ? f.half : k.S > 128 ? 1.35 : 1.0) * (acc ? 1.8 : 1.0);
   s.add = acc ? 0.9 : f.add;
@@ -333,14 +336,20 @@ static WavPick wav_pick_cached(int v, const WavqBlock& k, int w0, int w1, int nz
 // outputs per x-task) and the two-lane block for 64 the one expected to be
 // faster.  The best launches of larger blocks and of two outputs per x-task are
 // within 1.5% of the best of these on average, 5% up to 112^3 pairs (144^3 FP64
-// 115 us in 256 steps against 117).
+// 115 us in 256 steps against 117).  Except FP64 synthesis of some 95^3 to 119^3
+// pairs, where two outputs per x-task take less: 2% on average of periodic, grown
+// and accumulated calls of 96^3 to 116^3 (96^3 48.4 us against 49.0, 100^3 55.6
+// against 58.1, 112^3 grown 75.2 against 81.3, with a_y 82.8 against 90.2); 88^3
+// and 128^3 and more take 1% to 9% longer.
 int wav_default_variant(int prec, int form, const Box3& b, int narr, bool acc) {
   const int lo = form == FORM_IDWT ? Idwt<Sym8Rec>::LO : Dwt<Sym8Dec>::LO;
   const FDim d0 = fdim(b.n[0], b.bc[0], b.nx[0], b.ny[0], lo, lo + 7), d1 = fdim(b.n[1], b.bc[1], b.nx[1], b.ny[1], lo, lo + 7),
              d2 = fdim(b.n[2], b.bc[2], b.nx[2], b.ny[2], lo, lo + 7);
   int best = 5;
   double t = 1e300;
-  for (int v : {7, 11}) {
+  const double points = (double)d0.nout * d1.nout * d2.nout * std::max(narr, 1);
+  const bool two = prec == 8 && form == FORM_IDWT && points >= 8.5e5 && points <= 1.7e6;
+  for (int v : {two ? 16 : 7, 11}) {
     WavqBlock k;
     if (!wavq_block(v, &k)) continue;
     const WavPick p = wav_pick_cached(v, k, d0.nout, d1.nout, d2.nout, std::max(narr, 1), prec,
