@@ -29,6 +29,9 @@ struct SweepArgs {
   int nout;       // number of output steps
   int chunk;      // outputs per block and line (set by launcher)
   int cblocks;    // blocks over the lines / columns (set by launcher)
+  int nchunk, run;  // tiles: chunks per line, tiles per XCD's run (set by launcher)
+  unsigned nchunk_inv, run_inv;  // min(2^32 / n, 2^32 - 1) of both
+  unsigned run_end;  // tiles in full rounds of 8 runs
   R a, a_x, a_y;
   int flags;      // F_A | F_AX | F_AY | F_DOT
   double* dot_part;  // per-block FP64 partials of <x, a f(x)> (or null)

@@ -160,6 +160,7 @@ struct SweepTask {
 // 32 columns: a row of the tile is 256 bytes in FP64 and a full line in FP32,
 // whose chunk would halve (and its halo reads double) with 64.
 constexpr int kSweepCols = 32;
+constexpr int kSweepRun = 8;
 template <typename R, class Op, int Q>
 struct SweepGeo {
   static constexpr int C = kSweepCols, G = 256 / C, CH = G * Q, NS = CH + Op::W - 1;
@@ -167,6 +168,39 @@ struct SweepGeo {
   // contiguous: a row holds IN runs of NS steps (or OUT runs of CH outputs)
   static constexpr int ROW = (Op::IN * NS > Op::OUT * CH ? Op::IN * NS : Op::OUT * CH) | 1;
 };
+
+// t / n and t % n, inv = min(2^32 / n, 2^32 - 1): the product is at most one short
+__device__ __forceinline__ unsigned div_inv(unsigned t, unsigned n, unsigned inv, unsigned& r) {
+  unsigned q = __umulhi(t, inv);
+  r = t - q * n;
+  if (r >= n) {
+    ++q;
+    r -= n;
+  }
+  return q;
+}
+
+// The tile of a block, chunks of a line fastest.  Consecutive blocks go to the 8
+// XCDs in turn; here each XCD takes runs of p.run neighbouring tiles, so what
+// those share -- the halo of a chunk, the memory lines that a tile's edge splits
+// -- is in one L2: the chunks of one column of tiles, of kSweepRun of them where
+// L is not a multiple of the tile's columns and its rows end within lines.
+// Against tiles dealt out one by one: strided 0.85 to 0.91 of the time with such
+// L, 0.96 to 1.02 with others (second derivative FP64 of 192^3 30.2 -> 25.3 us).
+// One run per XCD, an eighth of the array, is 0 to 3% behind in FP64.  The blocks
+// past the last full round of runs take the tiles in order.
+template <typename R>
+__device__ __forceinline__ long tile_of(const SweepArgs<R>& p, int& bk) {
+  const unsigned b = blockIdx.x;
+  unsigned t = b, w;
+  if (b < p.run_end) {
+    const unsigned g = div_inv(b >> 3, (unsigned)p.run, p.run_inv, w);
+    t = (g * 8 + (b & 7)) * (unsigned)p.run + w;
+  }
+  const unsigned bc = div_inv(t, (unsigned)p.nchunk, p.nchunk_inv, w);
+  bk = (int)w;
+  return bc;
+}
 
 // ---------------------------------------------------------------- strided
 template <typename R, class Op, int BC, int Q>
@@ -178,8 +212,9 @@ __global__ __launch_bounds__(256) void sweep_strided(SweepArgs<R> p) {
   const int tc = threadIdx.x % C, tg = threadIdx.x / C;
   // arrays of a call lie line_in * nr (line_out * nr) apart, so a line's place
   // follows from its number in the whole call
-  const int bc = (int)(blockIdx.x % (unsigned)p.cblocks), bk = (int)(blockIdx.x / (unsigned)p.cblocks);
-  const long col = (long)bc * C + tc;
+  int bk;
+  const long bc = tile_of(p, bk);
+  const long col = bc * C + tc;
   const bool active = col < p.ncols;
   const long line = !active ? 0 : p.ncols <= 0x7fffffffL ? (int)col / (int)p.L : col / p.L;
   const long l = active ? col - line * p.L : 0;
@@ -239,17 +274,18 @@ __global__ __launch_bounds__(256) void sweep_strided(SweepArgs<R> p) {
 }
 
 // ---------------------------------------------------------------- contiguous
-template <typename R, class Op, int BC, int Q>
+template <typename R, class Op, int BC, int Q, bool AY>
 __global__ __launch_bounds__(256) void sweep_contig(SweepArgs<R> p) {
   using G = SweepGeo<R, Op, Q>;
   constexpr int K = KindOf<Op>::v, C = G::C;
   __shared__ R tile[C * G::ROW];
   __shared__ double red[4];
-  const int bc = (int)(blockIdx.x % (unsigned)p.cblocks), bk = (int)(blockIdx.x / (unsigned)p.cblocks);
+  int bk;
+  const long bc = tile_of(p, bk);
   const int i0 = p.i_first + bk * p.chunk;
   const int i1 = min(i0 + p.chunk, p.i_first + p.nout);
   const SweepSrc<K, BC, R> src(p, i0 + Op::LO, i1 - 1 + Op::UP);
-  const long line0 = (long)bc * C;
+  const long line0 = bc * C;
   // filled 64 lanes along a line: 4 lines per pass
   constexpr int NX = (Op::IN * G::NS + 63) / 64, NY = C / 4;
   const int lx = threadIdx.x & 63, ly = threadIdx.x >> 6;
@@ -265,6 +301,33 @@ __global__ __launch_bounds__(256) void sweep_contig(SweepArgs<R> p) {
       const int c = K == KDWT ? e & 1 : e / G::NS, s = K == KDWT ? e >> 1 : e - c * G::NS;
       const long at = act && e < Op::IN * G::NS ? src.at(i0 + Op::LO + s, c) : -1;
       val[b * NX + a] = at >= 0 ? xb[at] : R(0);
+    }
+  }
+  // The outputs of the tile in memory order along its lines: a wave's lanes take
+  // 64 of one line, or all of several lines with short chunks.  The y values of
+  // the a_y term come with the loads of x; they are a kernel of their own, for
+  // their registers cost the others a wave per SIMD (second derivative FP64 of
+  // 160^3 without a_y: 23.1 us in one kernel, 20.9 in its own).  Magic filter FP64
+  // of 107 x 118 x 64 points with a_y: 11.4 us with 64 lanes per line, y read last
+  // and the chunks of a line on different XCDs, now 6.5.
+  constexpr int OC = Op::OUT * G::CH, LW = OC < 64 ? OC : 64, OX = OC / LW, LP = 256 / LW, OY = C / LP;
+  const int of = threadIdx.x % LW, ol = threadIdx.x / LW;
+  R* __restrict__ yb = p.y + (line0 + ol) * p.line_out;
+  // output a of a line: element in the line (or -1), f its place in the tile's row
+  auto out_at = [&](int a, int& f) {
+    f = of + LW * a;
+    const int c = K == KIDWT ? f & 1 : f / G::CH, i = i0 + (K == KIDWT ? f >> 1 : f - c * G::CH);
+    return i < i1 ? out_elem<K>(i - p.oy, c, p.ny) : -1;
+  };
+  R yv[AY ? OX * OY : 1];
+  if (AY) {
+#pragma unroll
+    for (int a = 0; a < OX; ++a) {
+      int f;
+      const long at = out_at(a, f);
+#pragma unroll
+      for (int b = 0; b < OY; ++b)
+        yv[a * OY + b] = at >= 0 && line0 + ol + LP * b < p.ncols ? yb[LP * b * p.line_out + at] : R(0);
     }
   }
 #pragma unroll
@@ -299,22 +362,17 @@ __global__ __launch_bounds__(256) void sweep_contig(SweepArgs<R> p) {
     for (int c = 0; c < Op::OUT; ++c)
       tile[tc * G::ROW + (K == KIDWT ? 2 * (tg * Q + q) + c : c * G::CH + tg * Q + q)] = t.o[q][c];
   __syncthreads();
-  constexpr int OX = (Op::OUT * G::CH + 63) / 64;
 #pragma unroll
-  for (int b = 0; b < NY; ++b) {
-    const long ln = line0 + ly + 4 * b;
-    if (ln >= p.ncols) break;
-    R* __restrict__ yb = p.y + ln * p.line_out;
+  for (int b = 0; b < OY; ++b) {
+    if (line0 + ol + LP * b >= p.ncols) break;
 #pragma unroll
     for (int a = 0; a < OX; ++a) {
-      const int e = lx + 64 * a;
-      const int c = K == KIDWT ? e & 1 : e / G::CH, i = i0 + (K == KIDWT ? e >> 1 : e - c * G::CH);
-      if (e < Op::OUT * G::CH && i < i1) {
-        R* yp = yb + out_elem<K>(i - p.oy, c, p.ny);
-        R o = tile[(ly + 4 * b) * G::ROW + e];
-        if (p.flags & F_AY) o = fmar(p.a_y, *yp, o);
-        *yp = o;
-      }
+      int f;
+      const long at = out_at(a, f);
+      if (at < 0) continue;
+      R o = tile[(ol + LP * b) * G::ROW + f];
+      if (AY) o = fmar(p.a_y, yv[a * OY + b], o);
+      yb[LP * b * p.line_out + at] = o;
     }
   }
   if (p.dot_part) {
@@ -486,40 +544,40 @@ __global__ __launch_bounds__(kPartThreads) void sum_partials(const double* __res
 // not there.  They win where the tile would be mostly padding -- a few outputs
 // per line, or a few long lines -- once there are enough lines to fill the chip
 // by themselves, and for the wavelets, whose tile re-reads W - 1 pairs per
-// chunk, on ranges of longer lines too (up to 1.3 times as fast; over the rest
+// chunk, on ranges of longer lines too (up to 1.4 times as fast; over the rest
 // of those ranges the tiles are).  The bounds are where the two measured
-// times cross (periodic sweeps, device time, the tile's best chunk): second
-// derivative FP64, strided, 131072 columns: 6 outputs 7.0 us without a tile
-// against 11.0 with one, 16 outputs 11.5 against 13.2, 32 outputs 19 against
-// 15; a contiguous line of 2^20 points 11.4 against 57; symicomb8 FP64 along
-// the second of 100^3 pairs 27 against 37; sym8 FP64 on 32768 columns of 8
-// pairs 5.6 against 5.4, of 80 pairs 17 against 20.8.  All calls tried (1100
-// boxes and the grid of 1 .. 2^21 lines by 1 .. 2^20 outputs) are within 15% of
-// the faster form, 1% on average.
+// times cross (periodic sweeps, device time): second derivative FP64, strided,
+// 131072 columns: 6 outputs 7.0 us without a tile against 11.0 with one, 32
+// outputs 19 against 15; a contiguous line of 2^20 points 11.4 against 57, of
+// 28000 points 3.8 against 5.7, 8 of 57000 points 6.2 against 7.3, 16 of them
+// 8.8 against 8.1; symicomb8 FP64 along the second of 100^3 pairs 28 against
+// 37; sym8 FP64 on 32768 columns of 8 pairs 5.6 against 5.4, of 80 pairs 17
+// against 20.8.  Over 15000 calls tried (boxes, and grids of 1 .. 2^19 lines
+// by 1 .. 2^20 outputs, L odd and even) the choice is 0.4% behind the faster
+// form on average, and more than 15% behind it in 70.
 static bool ring_pays(long ncols, long L, int nout, int in, int W, int rs) {
   const double total = (double)ncols * nout;
   if (in == 1)
-    return (ncols >= 49152 && nout <= (rs == 8 ? (W > 16 ? 16 : 12) : (W > 16 ? 24 : 16))) ||
+    return (ncols >= 49152 && nout <= (rs == 4 && ncols >= 196608 ? 16 : W > 16 ? 12 : 8)) ||
            (ncols >= 32768 && nout <= 4);
-  // a tile's rows straddle the lines' ends: more of them are split
-  const bool ragged = L % kSweepCols != 0 && nout >= 64 && nout <= 160;
+  if (ncols >= 16384 && nout <= 4) return true;
+  if (L < 8 && nout > 12) return false;  // lanes of a wave on several lines, far apart
   if (W <= 8) {
-    if (ragged && ncols >= 16384 && total >= 1.2e6) return true;
     if (rs == 8)
-      return (ncols >= 32768 && nout <= 12) || (ncols >= 24576 && nout <= 2) ||
-             (ncols >= 24576 && nout >= 40 && nout <= 160 && total >= 1.9e6);
-    return (ncols >= 49152 && nout <= 40) || (ncols >= 16384 && nout <= 4) ||
-           (ncols >= 2048 && nout >= 40 && total >= 1.2e6 && total <= 2.7e6);
+      return (ncols >= 32768 && nout <= 12) || (ncols >= 196608 && nout >= 32 && nout <= 64) ||
+             (ncols >= 512 && nout >= 40 && total >= (ncols >= 24576 ? 1.9e6 : 2.3e6) && total <= 8.5e6);
+    return (ncols >= 49152 && nout <= 40) || (ncols >= 2048 && nout >= 40 && total >= 1.2e6 && total <= 2.7e6);
   }
   if (rs == 8)
-    return (ncols >= 65536 && nout <= 160) || (ncols >= 49152 && nout <= 20) || (ncols >= 32768 && nout <= 4) ||
-           (ncols >= 64 && total >= 3e6 && total <= 8.5e6) || (ragged && ncols >= 16384 && total >= 2e6);
+    return (ncols >= 65536 && nout <= 160) || (ncols >= 49152 && nout <= 20) ||
+           (ncols >= 64 && total >= 2.6e6 && total <= 8.5e6);
   return (ncols >= 24576 && nout <= 6) || (ncols >= 49152 && nout <= 12) || (ncols >= 65536 && nout <= 28) ||
          (ncols >= 131072 && nout <= 160) || (ncols >= 98304 && nout >= 64 && nout <= 160) ||
-         (ncols >= 24576 && nout >= 80 && nout <= 160 && total >= (ragged ? 3.6e6 : 5e6));
+         (ncols >= 16384 && nout >= 80 && nout <= 512 && total >= 5e6);
 }
 static bool seg_pays(long ncols, int nout, int in, int W, int rs) {
-  if ((ncols <= 4 && nout >= 60000) || (ncols <= 8 && nout >= 500000)) return true;
+  if ((ncols <= 8 && nout >= 50000) || (ncols <= 12 && nout >= 80000)) return true;
+  if (ncols <= 4 && nout >= (in == 2 ? 34000 : ncols > 2 ? 25000 : rs == 8 ? 17000 : 22000)) return true;
   if (in == 1) return ncols >= 24576 && nout <= 12;
   if (W <= 8) return (ncols >= 16384 && nout <= 2) || (ncols >= 262144 && nout <= 4);
   return ncols >= 24576 && nout <= (rs == 8 ? 4 : 6);
@@ -572,6 +630,9 @@ static SweepPlan sweep_plan(const SweepArgs<R>& p, int in, int W) {
   return s;
 }
 
+// for div_inv
+static unsigned inv32(int n) { return (unsigned)std::min<unsigned long>((1ul << 32) / (unsigned)n, 0xfffffffful); }
+
 template <typename R, class Op, int BC>
 static hipError_t run_sweep(const SweepArgs<R>& a0, hipStream_t st, double* dot_out) {
   SweepArgs<R> p = a0;
@@ -589,10 +650,17 @@ static hipError_t run_sweep(const SweepArgs<R>& a0, hipStream_t st, double* dot_
     const size_t lds = (size_t)(256 >> s.lg) * (s.chunk + Op::W - 1) * Op::IN * sizeof(R);
     sweep_seg<R, Op, BC><<<(unsigned)s.blocks, 256, lds, st>>>(p, s.lg);
   }
+  p.nchunk = (int)(s.blocks / s.cblocks);
+  p.run = p.nchunk * (p.L > 1 && p.L % kSweepCols ? kSweepRun : 1);
+  p.nchunk_inv = inv32(p.nchunk);
+  p.run_inv = inv32(p.run);
+  p.run_end = (unsigned)(s.blocks - s.blocks % (8L * p.run));
   auto launch = [&](auto q) {
     constexpr int Q = decltype(q)::value;
-    if (p.L == 1)
-      sweep_contig<R, Op, BC, Q><<<(unsigned)s.blocks, 256, 0, st>>>(p);
+    if (p.L == 1 && (p.flags & F_AY))
+      sweep_contig<R, Op, BC, Q, true><<<(unsigned)s.blocks, 256, 0, st>>>(p);
+    else if (p.L == 1)
+      sweep_contig<R, Op, BC, Q, false><<<(unsigned)s.blocks, 256, 0, st>>>(p);
     else
       sweep_strided<R, Op, BC, Q><<<(unsigned)s.blocks, 256, 0, st>>>(p);
   };

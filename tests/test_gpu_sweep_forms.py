@@ -171,3 +171,31 @@ def test_wavelet_forms(gpu, shape, comb, prec):
             if bc == 1 and nout <= (15 if comb else 7):
                 continue
             run_wav(lc, gpu, wav, dt, fast, nout, slow, bc, inverse)
+
+
+@pytest.mark.parametrize('lines,nout', [(1, 16999), (2, 17000), (1, 22000), (4, 25000), (5, 34567), (8, 50000),
+                                        (12, 80001), (13, 80001)])
+@pytest.mark.parametrize('prec', [8, 4])
+def test_long_lines_among_others(gpu, lines, nout, prec):
+    test_few_long_lines(gpu, lines, nout, prec)
+
+
+@pytest.mark.parametrize('lines,nout', [(2, 33999), (4, 34001), (8, 49999), (8, 50000), (12, 80000), (16, 80001)])
+@pytest.mark.parametrize('prec', [8, 4])
+def test_wavelet_long_lines(gpu, lines, nout, prec):
+    """The lines of a few-line call against the same lines among many."""
+    import libconv as lc
+    torch = gpu
+    dt = torch.float64 if prec == 8 else torch.float32
+    g = torch.Generator(device='cuda').manual_seed(nout + lines)
+    for wav in (lc.WAV_SYM8, lc.WAV_SYMICOMB8):
+        for inverse in (False, True):
+            wide = (torch.rand((32, 2 * nout), device='cuda', generator=g, dtype=torch.float64) - 0.5).to(dt)
+            y0 = (torch.rand((32, 2 * nout), device='cuda', generator=g, dtype=torch.float64) - 0.5).to(dt)
+            for kw in (dict(), dict(a=0.75, a_y=-0.25)):
+                y, yw = y0[:lines].clone(), y0.clone()
+                n, nw = [nout, lines // 2], [nout, 16]
+                lc.wavelet_1d(wav, inverse, 0, n, 0, n, n, 1, wide[:lines].contiguous(), y, **kw)
+                lc.wavelet_1d(wav, inverse, 0, nw, 0, nw, nw, 1, wide, yw, **kw)
+                torch.cuda.synchronize()
+                assert torch.equal(y, yw[:lines])
