@@ -225,8 +225,6 @@ hipError_t sep3d(int id, const Box3& b, int narr, const R* x, R* y, R a, R a_y, 
     p.ny = b.ny[s];
     p.line_in = L * p.nx;
     p.line_out = L * p.ny;
-    p.nti = p.line_in * Rr;
-    p.nto = p.line_out * Rr;
     p.n = b.n[s];
     p.ox = b.bc[s] == SHRINK ? gm.lo : 0;
     p.oy = b.bc[s] == GROW ? -gm.up : 0;

@@ -263,8 +263,6 @@ int run_1d(int kind, int id, int d, int idim, const int* n, int bc, const int* n
   p.ny = ny[idim];
   p.line_in = L * mul * nx[idim];
   p.line_out = L * mul * ny[idim];
-  p.nti = p.line_in * Rr;
-  p.nto = p.line_out * Rr;
   p.ox = bc == -1 ? g.lo : 0;
   p.oy = bc == 1 ? -g.up : 0;
   p.i_first = bc == 1 ? -g.up : 0;
@@ -277,7 +275,7 @@ int run_1d(int kind, int id, int d, int idim, const int* n, int bc, const int* n
   if (want_dot) p.flags |= F_DOT;
 
   Arg<R> ax, ay;
-  const size_t nin = (size_t)p.nti * narr, nout = (size_t)p.nto * narr;
+  const size_t nin = (size_t)p.line_in * Rr * narr, nout = (size_t)p.line_out * Rr * narr;
   if (device_api) {
     ax.dev = const_cast<R*>(x);
     ay.dev = y;
@@ -437,8 +435,6 @@ int run_md(int kind, int id, int d, const int* n, const int* bc, const int* nx, 
     p.ny = ny[s];
     p.line_in = L * mul * cur[s];
     p.line_out = L * mul * ny[s];
-    p.nti = p.line_in * Rr;
-    p.nto = p.line_out * Rr;
     p.ox = bc[s] == -1 ? g.lo : 0;
     p.oy = bc[s] == 1 ? -g.up : 0;
     p.i_first = bc[s] == 1 ? -g.up : 0;

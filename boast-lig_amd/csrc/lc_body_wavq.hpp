@@ -23,14 +23,18 @@
 // Strides of A and B are odd numbers of pairs, and consecutive lanes take
 // consecutive rows (x) or columns (y): no bank conflicts.
 //
-// What bounds it (96^3 pairs and a 128-orbital batch, FP64): bytes.  Without
-// its FMAs the batch takes as long as with them (1.45 ms on fixed 16 x 16
-// tiles, HBM traffic 1.7 times the arrays); the FMAs and LDS reads alone take
-// 0.87 ms.  Hence tiles of any shape, chosen per grid (WavqShape): no lanes
-// on padding and the widest tile the block holds, since a halo read that
-// misses L2 costs as much as an input value.  The form it replaced worked a
-// plane per barrier on 8 x 8 tiles with 8-byte y reads (LDS busy 52% of its
-// cycles, a fifth of that bank conflicts): 1.65 ms for the same batch.
+// What bounds it (FP64).  A batch that fills the chip (128 orbitals): bytes.
+// Without its FMAs it takes as long as with them (1.45 ms on fixed 16 x 16 tiles;
+// the FMAs and LDS reads alone 0.87), and it moves 3.9 GB, halo lines that miss
+// L2 included, at 3.6 TB/s (a copy: 5.1).  Hence tiles of any shape, chosen per
+// grid (WavqShape): no lanes on padding and the widest tile the block holds,
+// since a halo read that misses L2 costs as much as an input value.  A single
+// call (96^3 pairs): the serial chain of a step with two barriers, 504 blocks
+// or two waves per SIMD to hide it -- 3.0 TB/s, VALU busy 35% and LDS 24 - 31%
+// of the time, none of them at its limit; hence the choice of tile and z chunk
+// by expected time.  The form with a plane per barrier on 8 x 8 tiles and 8-byte
+// y reads (LDS busy 52% of its cycles, a fifth of that bank conflicts) takes
+// 1.65 ms for the batch.
 //
 // ME: the epilogue reads y (F_AY).  Without (ME false) every wave issues the
 // same memory operations in every step, the outputs as buffer stores that drop

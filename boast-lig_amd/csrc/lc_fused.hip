@@ -37,8 +37,9 @@ size_t fused_sum3d_parts(const Box3& b, int narr, int lo, int up, int w) {
   FDim g0 = fdim(b.n[0], b.bc[0], b.nx[0], b.ny[0], lo, up);
   FDim g1 = fdim(b.n[1], b.bc[1], b.nx[1], b.ny[1], lo, up);
   FDim g2 = fdim(b.n[2], b.bc[2], b.nx[2], b.ny[2], lo, up);
-  // upper bound over the variants: tiles no smaller than 16 x 8, z chunks no
-  // shorter than 16 planes (two-plane kinetic form) or 4 w (the others)
+  // partials per array.  The one-plane variants need no more (tiles of 16 x 8
+  // and larger, chunks of 4 w planes); the two-plane kinetic form would take
+  // chunks down to 4 planes and is held to this number by its launch
   const long tiles = (long)((g0.nout + 15) / 16) * ((g1.nout + 7) / 8);
   const long maxc = std::max(std::max(1, g2.nout / (4 * w)), g2.nout / 16) + 2;
   (void)narr;

@@ -212,9 +212,9 @@ hipError_t launch_sum3d2(const Box3& b, int narr, const R* x, R* y, const double
     // A block's prefill (W - 1 column loads per lane) takes the time of about
     // ten planes, three for each block more; two FP64 blocks on a CU run a
     // plane in 1.6 times the time of one (fitted to 1 - 5 blocks per CU on
-    // 24^3 to 256^3).  Chunks of 16 planes and more, filling the CUs, took
-    // 26 us on 24^3, 22 on 100 x 90 x 110 and 32 on 143^3 in FP64; now 16
-    // (the host's launch rate), 18 and 29.
+    // 24^3 to 256^3).  FP64, against chunks of 16 planes and more that fill the
+    // CUs: 24^3 16 us (the host's launch rate; 26), 100 x 90 x 110 18 (22),
+    // 143^3 29 (32).
     const ZCost m = sizeof(R) == 8 ? ZCost{13, 3.1, 0, 0, 0.8} : ZCost{9, 3, 0, 0, 0.58};
     const long maxc = (long)fused_sum3d_parts(b, narr, F::LO, F::UP, F::N) / tiles;
     p.zchunk = cost_zchunk(m, tiles, p.d2.nout, narr, -ZC, maxc, QZ, num_cu());
@@ -440,9 +440,9 @@ int sep_plane_args(const Box3& b, int narr, const R* x, R* y, R a, R a_y, const 
     // planes run 486 blocks of 95 planes 6% faster than 648 of 71).  A chunk
     // repeats W - 1 planes; two FP64 blocks on a CU run a plane in 1.74 times
     // the time of one, two FP32 ones in 1.55 (fitted to 1 - 5 blocks per CU on
-    // 24^3 to 256^3).  Chunks of 2 W planes and more left CUs idle on small
-    // grids: 37 us on 48^3, 32 on 100 x 90 x 110, 30 on 128^3 in FP64, 47 on
-    // 200^3 in FP32; now 16 (the host's launch rate), 20, 23 and 37.
+    // 24^3 to 256^3).  Against chunks of 2 W planes and more, which leave CUs
+    // idle on small grids: FP64 48^3 16 us (the host's launch rate; 37), 100 x
+    // 90 x 110 20 (32), 128^3 23 (30), FP32 200^3 37 (47).
     const ZCost m = sizeof(R) == 8 ? ZCost{10, 0, F::N - 1, 0, 0.87} : ZCost{10, 0, F::N - 1, 0.15, 0.7};
     p.zchunk = cost_zchunk(m, tiles, p.d2.nout, narr, -ZC, p.d2.nout, 1, num_cu());
   } else {
@@ -633,14 +633,15 @@ hipError_t launch_sepq_batch(const FusedArgs<R>* tab, const BatchStage* s, hipSt
 
 // ---- magic filter with the potential step of the local Hamiltonian (one
 // array, a_y = 0): y = pot t, rho += t^2 of the filtered value t.
-// Bound: memory, five arrays (x, pot and rho read, y and rho written).  The
-// pipelined kernels' epilogue had loads and stores inside a branch and so
-// waits for everything in flight: 78 us on the 157^3 points of 64^3 pairs in
-// FP64 and 55 us in FP32 (69% of the wave cycles were waits).  This one: 53 us
-// (155 MB, 2.9 TB/s) and 36 us; deeper prefetch, tiles of 32 x 32 and more
-// blocks are no faster in FP64 (53 - 57 us).  In FP32 a block has four waves,
-// and two blocks per CU run a plane in little more time than one: 36 against
-// 45 us.
+// It moves five arrays (x, pot and rho read, y and rho written): on the 157^3
+// points of 64^3 pairs 50 - 53 us in FP64 (168 MB counted, 3.3 TB/s, 65% of what
+// a copy moves; VALU busy 24%, LDS 19%) and 36 in FP32, so what bounds it is the
+// serial chain of a plane (two barriers, one block per CU), not bytes.  With the loads and stores of
+// the epilogue inside a branch, as the pipelined kernels have them, a wave waits
+// for everything in flight: 78 and 55 us (69% of the wave cycles waits).  Deeper
+// prefetch, tiles of 32 x 32 and more blocks are no faster in FP64 (53 - 57 us).
+// In FP32 a block has four waves, and two blocks per CU run a plane in little
+// more time than one: 36 against 45 us.
 template <typename R>
 struct PotTile {
   static constexpr int TX = 32, TY = 16, QX = sizeof(R) == 8 ? 4 : 8, QY = sizeof(R) == 8 ? 2 : 4, PD = 2,

@@ -192,21 +192,6 @@ static hipError_t launch_sepw3d(const Box3& b, int narr, const R* x, R* y, R a, 
   return hipGetLastError();
 }
 
-// z chunk of a single call: ZC < 0: at most -ZC blocks on any CU, at least
-// one where the grid allows, chunks >= W steps; else ~2 blocks per CU,
-// chunks >= 2 W steps
-template <class Op, int ZC>
-static int wav_zchunk(long tiles, int narr, int nout) {
-  if (ZC < 0) {
-    const long per = tiles * std::max(narr, 1);
-    long chunks = (long)(-ZC) * num_cu() / per;
-    if (chunks * per < num_cu()) chunks = (num_cu() + per - 1) / per;
-    chunks = std::max(1L, std::min<long>(chunks, std::max(1, nout / Op::W)));
-    return (int)((nout + chunks - 1) / chunks);
-  }
-  return pick_zchunk(tiles, nout, std::max(narr, 1), std::max(1, Op::W / 2), num_cu());
-}
-
 // ---- tile and z chunk of the pair-wise kernels
 // Work of one block-step: the issue of its FMAs in cycles (x-tasks 32 QX,
 // y-tasks 128 / HB per wave of four cycles, over four SIMDs), its bytes and its

@@ -21,7 +21,6 @@ struct SweepArgs {
   long ncols;     // L * R * narr
   long line_in;   // distance between consecutive r in x (= L * IN * nx)
   long line_out;  // distance between consecutive r in y (= L * OUT * ny)
-  long nti, nto;  // distance between consecutive arrays
   int narr;
   int n, nx, ny;  // logical length and extents along the line (steps)
   int ox, oy;     // logical index of the first stored input / output step

@@ -430,7 +430,7 @@ __device__ __forceinline__ void pz_get(const R* base, long p, R* v, bool both) {
 
 // update_rhopol's other inputs at the points p and (both) p + 1, loaded before
 // the stencils (loads and a store per point after them are two chained round
-// trips: order 16 at 256^3 FP64 203 us, now 168)
+// trips: order 16 at 256^3 FP64 203 us against 168)
 template <typename R>
 struct RhoIn {
   R d[6], rho[2];

@@ -565,7 +565,7 @@ static bool ring_pays(long ncols, long L, int nout, int in, int W, int rs) {
   if (W <= 8) {
     if (rs == 8)
       return (ncols >= 32768 && nout <= 12) || (ncols >= 196608 && nout >= 32 && nout <= 64) ||
-             (ncols >= 512 && nout >= 40 && total >= (ncols >= 24576 ? 1.9e6 : 2.3e6) && total <= 8.5e6);
+             (ncols >= 100 && nout >= 40 && total >= (ncols >= 24576 ? 1.9e6 : 2.3e6) && total <= 8.5e6);
     return (ncols >= 49152 && nout <= 40) || (ncols >= 2048 && nout >= 40 && total >= 1.2e6 && total <= 2.7e6);
   }
   if (rs == 8)
