@@ -651,7 +651,9 @@ static hipError_t run_sweep(const SweepArgs<R>& a0, hipStream_t st, double* dot_
     sweep_seg<R, Op, BC><<<(unsigned)s.blocks, 256, lds, st>>>(p, s.lg);
   }
   p.nchunk = (int)(s.blocks / s.cblocks);
-  p.run = p.nchunk * (p.L > 1 && p.L % kSweepCols ? kSweepRun : 1);
+  // whole rounds of 8 runs, of about as many columns of tiles as said at tile_of
+  const long col = (long)p.nchunk * (p.L > 1 && p.L % kSweepCols ? kSweepRun : 1);
+  p.run = (int)std::max(1L, s.blocks / (8 * std::max(1L, s.blocks / (8 * col))));
   p.nchunk_inv = inv32(p.nchunk);
   p.run_inv = inv32(p.run);
   p.run_end = (unsigned)(s.blocks - s.blocks % (8L * p.run));
